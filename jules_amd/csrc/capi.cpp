@@ -670,8 +670,8 @@ int k_attn_causal(int ni, const jh_tensor* in, int no, jh_tensor* out, const cha
 // for the caller's (device, stream), grown on demand.  Calls on one stream
 // run in stream order and may share it; calls on another stream get their
 // own buffer, so registry calls on two streams of one device do not race.
-int registry_workspace(size_t need, void* stream, void** ws) {
-    return check_hip(jh::stream_workspace(need, static_cast<hipStream_t>(stream), ws),
+int registry_workspace(size_t need, void* stream, void** ws, jh::WorkspaceLock* lock) {
+    return check_hip(jh::stream_workspace(need, static_cast<hipStream_t>(stream), ws, lock),
                      "registry workspace");
 }
 
@@ -696,8 +696,9 @@ int k_w8a16_silu(int ni, const jh_tensor* in, int no, jh_tensor* out, const char
     }
     const size_t need = jules_hip_w8a16_workspace_size((int)M, (int)N, (int)K);
     void* ws = nullptr;
+    jh::WorkspaceLock lock;
     if (need) {
-        const int st = registry_workspace(need, s, &ws);
+        const int st = registry_workspace(need, s, &ws, &lock);
         if (st != JH_OK) return st;
     }
     return jules_hip_w8a16_gemm_bias_act(JH_ACT_SILU, addr(x), static_cast<const int8_t*>(addr(w)),
@@ -817,7 +818,8 @@ int k_cross_entropy(int ni, const jh_tensor* in, int no, jh_tensor* out, const c
     if (M > INT32_MAX || N > INT32_MAX) return fail(JH_ERR_SHAPE, "fusedCrossEntropyLoss: too large");
     const size_t need = jules_hip_cross_entropy_workspace_size((int)M);
     void* ws = nullptr;
-    const int st = registry_workspace(need, s, &ws);
+    jh::WorkspaceLock lock;
+    const int st = registry_workspace(need, s, &ws, &lock);
     if (st != JH_OK) return st;
     return jules_hip_cross_entropy(static_cast<const float*>(addr(x)),
                                    static_cast<const int32_t*>(addr(t)),
@@ -844,8 +846,9 @@ int k_mlp_forward(int ni, const jh_tensor* in, int no, jh_tensor* out, const cha
         return fail(JH_ERR_SHAPE, "fusedMLPForward: too large");
     const size_t need = jules_hip_mlp_forward_workspace_size((int)M, (int)K1, (int)N1, (int)N2);
     void* ws = nullptr;
+    jh::WorkspaceLock lock;
     if (need > 0) {
-        const int st = registry_workspace(need, s, &ws);
+        const int st = registry_workspace(need, s, &ws, &lock);
         if (st != JH_OK) return st;
     }
     return jules_hip_mlp_forward(static_cast<const float*>(addr(x)), static_cast<const float*>(addr(w1)),
@@ -879,8 +882,9 @@ int k_mlp(int ni, const jh_tensor* in, int no, jh_tensor* out, const char*, void
         return fail(JH_ERR_SHAPE, "interleavedMLPForwardBackward: too large");
     const size_t need = jules_hip_mlp_workspace_size((int)M, (int)K1, (int)N1, (int)N2);
     void* ws = nullptr;
+    jh::WorkspaceLock lock;
     if (need > 0) {
-        const int st = registry_workspace(need, s, &ws);
+        const int st = registry_workspace(need, s, &ws, &lock);
         if (st != JH_OK) return st;
     }
     float* f[7];

@@ -21,13 +21,17 @@ namespace jh {
 // One workspace per (device, stream), kept for the process: calls on one
 // stream run in order and may share it, calls on other streams get their
 // own.  A larger need replaces it once the stream is done with the old one.
-hipError_t stream_workspace(size_t need, hipStream_t s, void** ws) {
-    static std::mutex mu;
+// The lock is the caller's until it has enqueued every kernel that uses the
+// workspace, so that threads sharing a stream neither interleave their kernels
+// nor replace the buffer under each other; recursive, since a registry call
+// holds it around entry points of the library.
+hipError_t stream_workspace(size_t need, hipStream_t s, void** ws, WorkspaceLock* lock) {
+    static std::recursive_mutex mu;
     static std::map<std::pair<int, hipStream_t>, std::pair<void*, size_t>> cache;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(mu);
+    *lock = WorkspaceLock(mu);
     auto& slot = cache[{dev, s}];
     if (slot.second < need) {
         if (slot.first) {
@@ -96,7 +100,8 @@ hipError_t launch_flash_fwd_padded(int dtype, int causal, float scale, const voi
     const size_t es = dtype == JH_BF16 ? 2 : 4;
     const size_t one = a256((size_t)rows * Dp * es);
     void* ws = nullptr;
-    hipError_t e = stream_workspace(4 * one, s, &ws);
+    WorkspaceLock lock;
+    hipError_t e = stream_workspace(4 * one, s, &ws, &lock);
     if (e != hipSuccess) return e;
     char* w = static_cast<char*>(ws);
     void *Qp = w, *Kp = w + one, *Vp = w + 2 * one, *Op = w + 3 * one;
@@ -117,7 +122,8 @@ hipError_t launch_flash_bwd_padded(int dtype, int causal, float scale, const voi
     const size_t es = dtype == JH_BF16 ? 2 : 4;
     const size_t one = a256((size_t)rows * Dp * es);
     void* ws = nullptr;
-    hipError_t e = stream_workspace(8 * one, s, &ws);
+    WorkspaceLock lock;
+    hipError_t e = stream_workspace(8 * one, s, &ws, &lock);
     if (e != hipSuccess) return e;
     char* w = static_cast<char*>(ws);
     void* p[8];

@@ -4,31 +4,22 @@
 // reference's layout, FusedKernels.h:378: A[i*K+k], B[k*N+j]), fp32
 // accumulation in v_mfma_f32_32x32x16_bf16, epilogue in fp32.
 //
-// Block tile 256 x 256 x 64, 256 threads = 4 waves in a 2 x 2 grid, each wave
-// owning a 128 x 128 sub-tile = 4 x 4 MFMA tiles of 32 x 32 (256 fp32
-// accumulators per lane).  At 4096^3 this is 256 workgroups: one per CU.
-//
-// Operand staging.  The MFMA wants, per lane, 8 consecutive k of one row of
-// A and 8 consecutive k of one column of B.  A rows are k-contiguous in HBM;
-// B columns are not (B is [K,N] row-major).  Each thread therefore loads an
-// 8(k) x 8(n) block of B with eight 16-byte row loads and transposes it in
-// registers with 32 v_perm_b32, so that B is stored in LDS n-major with k
-// contiguous, exactly like A.  Both LDS tiles are 256 rows x 128 bytes, 16-byte
-// chunk c of row r stored at chunk position c ^ ((r ^ (r >> 3)) & 7): the
-// MFMA fragment reads (8 consecutive rows, one chunk) and the transposed B
-// stores (rows 8 apart, one chunk) then both hit distinct bank groups.
-//
-// Pipeline: two LDS stages (128 KiB).  Iteration kt issues the HBM loads of
-// slice kt+1 into registers, runs the 64 MFMAs of slice kt from LDS, then
-// writes slice kt+1 into the other stage; one barrier per slice.
+// Three kernels, chosen by launch_gemm_bf16:
+//   - gemm_bf16_tile_kernel (gemm_tile.hpp): any shape, output tiles from
+//     32 x 64 to 256 x 256, K split over workgroups where the tiles alone
+//     would leave CUs idle;
+//   - gemm_bf16_dma_kernel: whole 256 x 256 tiles, 4 waves of 128 x 128;
+//   - gemm_bf16_kernel: rows of A or B so long that a tile's byte offsets
+//     pass 2^31, 64-bit addresses throughout.
 //
 // Workgroup order is XCD aware: consecutive workgroup ids land on different
 // XCDs (round robin over 8), so ids are remapped so that each XCD's workgroups
-// cover a compact 4-row band of output tiles that shares A and B slices in
-// that XCD's L2.
+// cover a compact band of output tiles that shares A and B slices in that
+// XCD's L2.
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemm_tile.hpp"
 #include "launch.hpp"
 #include "tiles.hpp"
 
@@ -71,6 +62,17 @@ __device__ __forceinline__ float act_bf16(float x) {
     else return x;
 }
 
+// ---------------------------------------------------------------------------
+// Rows too long for 32-bit tile offsets.  Block tile 256 x 256 x 64, 4 waves of
+// 128 x 128 (4 x 4 MFMA tiles).  Each thread loads an 8(k) x 8(n) block of B
+// with eight 16-byte row loads and transposes it in registers with 32
+// v_perm_b32, so B is stored in LDS n-major with k contiguous, like A.  Both
+// LDS tiles are 256 rows x 128 bytes, 16-byte chunk c of row r at chunk
+// position c ^ ((r ^ (r >> 3)) & 7): the fragment reads (8 consecutive rows,
+// one chunk) and the transposed B stores (rows 8 apart, one chunk) then both
+// hit distinct bank groups.  Two LDS stages (128 KiB); iteration kt loads slice
+// kt+1 into registers, runs the 64 MFMAs of slice kt, then writes slice kt+1.
+// ---------------------------------------------------------------------------
 template <int ACT>
 __global__ __launch_bounds__(THREADS, 1) void gemm_bf16_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
@@ -491,23 +493,196 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_bf16_dma_kernel(
     }
 }
 
+// ---------------------------------------------------------------------------
+// Any shape: the tile loop of gemm_tile.hpp.
+//
+// A workgroup computes one output tile over K range z (kc elements, a multiple
+// of the slice).  With one range it finishes the tile; with several it writes
+// fp32 partial sums to part[z][M][N], which the reduce kernel adds in range
+// order before bias and activation.
+//
+// What bounds it (328 x 4096 x 4096): the copies of the operand tiles from L2
+// to LDS, (1/BM + 1/BN) of K per output.  64 x 128 tiles move 302 MB in 22.7
+// us; 256 x 256 tiles move a third of that but only fill 32 CUs, which took the
+// register-staged kernel 181 us.  The tile is as large as still fills the chip.
+// ---------------------------------------------------------------------------
+template <class T>
+__global__ __launch_bounds__(T::THREADS) void gemm_bf16_tile_kernel(
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, const float* __restrict__ bias,
+    uint16_t* __restrict__ C, float* __restrict__ part, int act, int M, int N, int K, int kc) {
+    __shared__ __attribute__((aligned(1024))) uint8_t sm[T::LDS];
+    const TileCoord t = tile_coord<8>((M + T::BM - 1) / T::BM, (N + T::BN - 1) / T::BN);
+    const int m0 = t.tm * T::BM, n0 = t.tn * T::BN, kb = t.z * kc;
+    typename T::Acc own[T::OWN];
+    T::run(reinterpret_cast<const uint8_t*>(A + (int64_t)m0 * K + kb), (int64_t)K * 2, min(T::BM, M - m0),
+           reinterpret_cast<const uint8_t*>(B + (int64_t)kb * N + n0), (int64_t)N * 2, (int64_t)(N - n0) * 2,
+           min(K - kb, kc), sm, own);
+    // a lane's 16 elements: one column, rows 4 at a time
+    auto each = [&](auto&& f) {
+#pragma unroll
+        for (int q = 0; q < T::OWN; ++q) {
+            const int col = n0 + T::own_col(q);
+            if (col >= N) continue;
+            const float bv = bias && !part ? bias[col] : 0.0f;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = m0 + T::own_row(q, e);
+                if (row < M) f((int64_t)row * N + col, own[q][e] + bv);
+            }
+        }
+    };
+    if (part) {
+        float* p = part + (int64_t)t.z * M * N;
+        each([&](int64_t o, float v) { p[o] = v; });
+        return;
+    }
+    JH_DISPATCH_ACT(act, ACT, each([&](int64_t o, float v) {
+                        C[o] = __builtin_bit_cast(uint16_t, (__bf16)act_bf16<ACT>(v));
+                    }));
+}
+
+template <int ACT>
+__device__ __forceinline__ u32x4_t act_pack8(const float (&v)[8]) {
+    u32x4_t o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(act_bf16<ACT>(v[2 * j]), act_bf16<ACT>(v[2 * j + 1]));
+    return o;
+}
+
+// C = act(sum over z of part[z], in z order, + bias): 8 columns per thread
+// (N % 8 == 0)
+__global__ __launch_bounds__(256) void gemm_bf16_reduce_kernel(const float* __restrict__ part, int S,
+                                                               const float* __restrict__ bias,
+                                                               uint16_t* __restrict__ C, int act,
+                                                               int64_t total, int N) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (i >= total) return;
+    const f32x4_t* p = reinterpret_cast<const f32x4_t*>(part + i);
+    f32x4_t lo = p[0], hi = p[1];
+#pragma unroll 4
+    for (int z = 1; z < S; ++z) {
+        p += total / 4;
+        lo += p[0];
+        hi += p[1];
+    }
+    float v[8];
+    const int col = (int)(i % N);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (j < 4 ? lo[j] : hi[j - 4]) + (bias ? bias[col + j] : 0.0f);
+    JH_DISPATCH_ACT(act, ACT, *reinterpret_cast<u32x4_t*>(C + i) = act_pack8<ACT>(v));
+}
+
+// The tile kernel's configurations: waves, slice bytes and ring depth as
+// measured best per tile, and the plan's cost model.  A launch of `wg`
+// workgroups over kc elements each takes about
+//   base + rounds * (kc * per_k + round) us,
+// rounds = ceil(wg / 256), times `shared` where two workgroups share a CU,
+// and K split in S adds split_base + 0.19 S + 1.2e-6 S M N us for the partial
+// sums and their reduction.  The constants are a least-squares fit to 250
+// shapes (M 24-4096, N and K 256-8192) timed at every tile and S: its choice
+// is 2 % off the best of them on average.  Larger tiles move fewer bytes per
+// output (per_k / (BM BN) falls from 1.2 to 0.34 ps), smaller ones fill the
+// chip sooner.
+struct TilePlan {
+    int bm, bn, bk;
+    float base, per_k, round, shared;
+};
+constexpr TilePlan kTilePlans[] = {
+    {32, 64, 64, 5.0f, 0.0024f, 1.2f, 0.79f},  {64, 64, 64, 5.9f, 0.0025f, 0.4f, 1.1f},
+    {64, 128, 64, 2.0f, 0.0039f, 4.2f, 1.0f},  {128, 128, 64, 0.7f, 0.0062f, 6.0f, 1.0f},
+    {128, 256, 32, 0.5f, 0.0126f, 7.2f, 1.0f}, {256, 256, 32, 1.7f, 0.0222f, 8.1f, 1.0f},
+};
+constexpr int kTilePlanCount = sizeof(kTilePlans) / sizeof(kTilePlans[0]);
+constexpr int64_t kMaxPartialBytes = int64_t(64) << 20;  // bound of the split's workspace
+
+struct TileChoice {
+    int plan, splits, kc;
+};
+
+TileChoice tile_choice(int M, int N, int K, bool may_split) {
+    TileChoice best{0, 1, 0};
+    float best_us = 0.0f;
+    for (int c = 0; c < kTilePlanCount; ++c) {
+        const TilePlan& p = kTilePlans[c];
+        const int64_t tiles = ((int64_t)(M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
+        const int slices = (K + p.bk - 1) / p.bk;
+        for (int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            if (S > 1 && (!may_split || slices < 2 * S || tiles * S > 512 ||
+                          (int64_t)S * M * N * 4 > kMaxPartialBytes))
+                break;
+            const int per = (slices + S - 1) / S;
+            const int z = slices ? (slices + per - 1) / per : 1;
+            const float rounds = (float)((tiles * z + 255) / 256);
+            float us = p.base + (rounds > 1.0f ? rounds * p.shared : 1.0f) *
+                                    ((float)per * p.bk * p.per_k + p.round);
+            if (z > 1) us += 1.75f + 0.19f * z + 1.2e-6f * z * M * N;
+            if (best_us == 0.0f || us < best_us) {
+                best_us = us;
+                best = {c, z, per * p.bk};
+            }
+        }
+    }
+    return best;
+}
+
+template <class T>
+void launch_tile(int act, const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C, float* part,
+                 int M, int N, int K, const TileChoice& c, hipStream_t s) {
+    const int64_t tiles = ((int64_t)(M + T::BM - 1) / T::BM) * ((N + T::BN - 1) / T::BN);
+    hipLaunchKernelGGL(gemm_bf16_tile_kernel<T>, dim3((unsigned)(tiles * c.splits)), dim3(T::THREADS), 0, s,
+                       A, B, bias, C, part, act, M, N, K, c.kc);
+}
+
 }  // namespace
 
 hipError_t launch_gemm_bf16(int act, const uint16_t* A, const uint16_t* B, const float* bias,
                             uint16_t* C, int M, int N, int K, hipStream_t s) {
-    const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    const bool full = bf16_gemm_tile(M, N, K).variant == GV_BF16_DMA;
-    hipError_t e = hipSuccess;
-    JH_DISPATCH_ACT(act, ACT, {
-        if (full)
-            hipLaunchKernelGGL(gemm_bf16_dma_kernel<ACT>, dim3(tiles), dim3(THREADS), 0, s, A, B,
-                               bias, C, M, N, K);
-        else
-            hipLaunchKernelGGL(gemm_bf16_kernel<ACT>, dim3(tiles), dim3(THREADS), 0, s, A, B, bias,
-                               C, M, N, K);
-        e = hipGetLastError();
-    });
-    return e;
+    // byte offsets within a tile (256 rows of A, 64 of B) below 2^31
+    if (K >= (1 << 22) || N >= (1 << 24)) {
+        const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+        JH_DISPATCH_ACT(act, ACT, hipLaunchKernelGGL(gemm_bf16_kernel<ACT>, dim3(tiles), dim3(THREADS), 0, s,
+                                                     A, B, bias, C, M, N, K));
+        return hipGetLastError();
+    }
+    // Partial sums live in the stream's workspace.  It may not be allocated
+    // while a graph is being captured, nor kept by the graph (a later call may
+    // replace it), and streams that share a handle may not share it.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    bool may_split = s != hipStreamPerThread;
+    if (may_split && hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError(), may_split = false;
+    may_split = may_split && cap == hipStreamCaptureStatusNone;
+    TileChoice c = tile_choice(M, N, K, may_split);
+    void* ws = nullptr;
+    WorkspaceLock lock;
+    if (c.splits > 1 && stream_workspace((size_t)c.splits * M * N * 4, s, &ws, &lock) != hipSuccess) {
+        (void)hipGetLastError();
+        c = tile_choice(M, N, K, false);
+    }
+    float* part = c.splits > 1 ? static_cast<float*>(ws) : nullptr;
+    switch (c.plan) {
+    case 0: launch_tile<TileCfg<Bf16Op, 32, 64, 1, 2, 1, 128, 6, 3>>(act, A, B, bias, C, part, M, N, K, c, s); break;
+    case 1: launch_tile<TileCfg<Bf16Op, 64, 64, 2, 2, 1, 128, 4, 3>>(act, A, B, bias, C, part, M, N, K, c, s); break;
+    case 2: launch_tile<TileCfg<Bf16Op, 64, 128, 2, 2, 2, 128, 6, 1>>(act, A, B, bias, C, part, M, N, K, c, s); break;
+    case 3: launch_tile<TileCfg<Bf16Op, 128, 128, 2, 2, 2, 128, 4, 1>>(act, A, B, bias, C, part, M, N, K, c, s); break;
+    case 4: launch_tile<TileCfg<Bf16Op, 128, 256, 2, 4, 1, 64, 6, 1>>(act, A, B, bias, C, part, M, N, K, c, s); break;
+    default:
+        // Whole 256 x 256 tiles: 4 waves of 128 x 128 read less LDS per MFMA
+        // than 8 of 128 x 64 (4096^3 113 against 122 us; 2304 x 3840 x 2560
+        // 60 against 65), but hold every register, none left for the edges.
+        if (!part && bf16_gemm_tile(M, N, K).variant == GV_BF16_DMA) {
+            const int tiles = (M / BM) * (N / BN);
+            JH_DISPATCH_ACT(act, ACT, hipLaunchKernelGGL(gemm_bf16_dma_kernel<ACT>, dim3(tiles), dim3(THREADS),
+                                                         0, s, A, B, bias, C, M, N, K));
+            return hipGetLastError();
+        }
+        launch_tile<TileCfg<Bf16Op, 256, 256, 2, 4, 1, 64, 4, 1>>(act, A, B, bias, C, part, M, N, K, c, s);
+    }
+    if (part) {
+        const int64_t total = (int64_t)M * N;
+        hipLaunchKernelGGL(gemm_bf16_reduce_kernel, dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0, s,
+                           part, c.splits, bias, C, act, total, N);
+    }
+    return hipGetLastError();
 }
 
 }  // namespace jh

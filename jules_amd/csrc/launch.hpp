@@ -6,6 +6,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <mutex>
+
 namespace jh {
 
 hipError_t launch_gemm_f32(int act, const float* A, const float* B, const float* bias,
@@ -126,8 +128,10 @@ hipError_t launch_flash_bwd_padded(int dtype, int causal, float scale, const voi
                                    void* dQ, void* dK, void* dV, int B, int H, int S, int D,
                                    void* bwd_ws, hipStream_t s);
 // device memory of `need` bytes for entry points without a workspace
-// argument: one buffer per (device, stream), kept for the process
-hipError_t stream_workspace(size_t need, hipStream_t s, void** ws);
+// argument: one buffer per (device, stream), kept for the process, and the
+// lock under which the caller enqueues what uses it
+using WorkspaceLock = std::unique_lock<std::recursive_mutex>;
+hipError_t stream_workspace(size_t need, hipStream_t s, void** ws, WorkspaceLock* lock);
 // the library's static device scratch (scratch.hip): its size, and the
 // device address of the current device's copy (looked up once per device;
 // allocates nothing)

@@ -498,7 +498,8 @@ hipError_t launch_int8(const int8_t* A, const int8_t* B, float* C, int M, int N,
     const bool vec = K > 0 && K % 16 == 0 && N % 16 == 0 && aligned16(A) && aligned16(B);
     if (vec && M <= 16) {
         void* ws = nullptr;
-        const hipError_t e = stream_workspace(int8_decode_workspace_size(M, N, K), s, &ws);
+        WorkspaceLock lock;
+        const hipError_t e = stream_workspace(int8_decode_workspace_size(M, N, K), s, &ws, &lock);
         if (e != hipSuccess) return e;
         return launch_int8_decode(A, B, C, M, N, K, scale_a, scale_b, row_scale, col_scale, bias, ws, s);
     }

@@ -440,10 +440,11 @@ hipError_t launch_sgemm(bool transA, bool transB, int M, int N, int K, float alp
         return hipGetLastError();
     }
     float* part = nullptr;
+    WorkspaceLock lock;
     const size_t pf = kplan_floats(M, N, K);
     if (pf) {
         void* ws = nullptr;
-        const hipError_t e = stream_workspace(pf * sizeof(float), s, &ws);
+        const hipError_t e = stream_workspace(pf * sizeof(float), s, &ws, &lock);
         if (e != hipSuccess) return e;
         part = static_cast<float*>(ws);
     }

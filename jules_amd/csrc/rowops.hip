@@ -1004,7 +1004,8 @@ template <typename W>
 hipError_t launch_split(int M, int N, bool vec, bool layer, const float* x, hipStream_t s, W&& write) {
     const int nseg = (N + SEG - 1) / SEG;
     void* ws = nullptr;
-    hipError_t e = stream_workspace(2 * (size_t)M * (size_t)nseg * sizeof(float), s, &ws);
+    WorkspaceLock lock;
+    hipError_t e = stream_workspace(2 * (size_t)M * (size_t)nseg * sizeof(float), s, &ws, &lock);
     if (e != hipSuccess) return e;
     float* part1 = static_cast<float*>(ws);
     float* part2 = part1 + (size_t)M * (size_t)nseg;

@@ -15,9 +15,9 @@
 //     Tile (4*rw) x 64 x K.
 //   F32_T32 / F32_T64: 32x32 (2x2 per thread) and 64x64 (4x4 per thread)
 //     output tiles, A and B staged through LDS in K slices of 32.
-// bf16 (MFMA): 256x256 output tiles of 4 waves; BF16_DMA copies 32-deep K
-// slices HBM -> LDS with LDS DMA (full tiles only), BF16_REG stages 64-deep
-// slices through registers and zero-fills ragged edges.
+// bf16 (MFMA): BF16_DMA, 256x256 output tiles of 4 waves over 32-deep K slices
+// by LDS DMA, can run whole tiles only; BF16_REG stands for every other shape.
+// Which kernel and tile a launch takes is the cost model of gemm_bf16.hip.
 #pragma once
 
 #include <stdint.h>
@@ -76,8 +76,8 @@ inline GemmTile f32_gemm_tile(int M, int N, int K) {
     return f32_variant_tile(tiles64 >= 512 ? GV_F32_T64 : GV_F32_T32, K);
 }
 
-// The variant a bf16 GEMM launch uses: LDS DMA when M and N are multiples of
-// the 256 tile and K of the 32-deep stage, register staging otherwise.
+// LDS DMA over whole tiles can run when M and N are multiples of the 256 tile
+// and K of the 32-deep stage.
 inline GemmTile bf16_gemm_tile(int M, int N, int K) {
     const bool full = M % kBf16Tile == 0 && N % kBf16Tile == 0 && K % kBf16DmaK == 0 && K > 0;
     return full ? GemmTile{GV_BF16_DMA, kBf16Tile, kBf16Tile, kBf16DmaK}

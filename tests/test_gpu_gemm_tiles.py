@@ -1,0 +1,88 @@
+"""The bf16 GEMM's tile kernel (gemm_tile.hpp) at the edges of its tiles, its K
+slices and its K split, and the long-row kernel past its offset limit.
+
+Tolerance: products of bf16 values are exact in fp32, a K-long fp32 sum is off
+by at most K * 2^-24 of the sum of |terms| and the bf16 result by 2^-9 of
+itself, so |y - ref| <= 2^-8 |ref| + 2^-20 sum |a b| holds with room for the
+hardware exp2 of the activations."""
+import pytest
+import torch
+
+from jules_amd import ops
+from tests.helpers import case
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(dev, M, N, K, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    A = (torch.randn((M, K), generator=g, device=dev) / K ** 0.5).bfloat16()
+    B = torch.randn((K, N), generator=g, device=dev).bfloat16()
+    bias = torch.rand((N,), generator=g, device=dev) - 0.5
+    return A, B, bias
+
+
+def _check(y, A, B, bias, act):
+    a, b = A.double(), B.double()
+    z = a @ b
+    z = z if bias is None else z + bias.double()
+    ref = torch.nn.functional.silu(z) if act == "silu" else z
+    bound = ref.abs() * 2.0 ** -8 + (a.abs() @ b.abs() + 1.0) * 2.0 ** -20
+    assert ((y.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (8, 8, 8), (8, 72, 16), (32, 64, 64), (40, 264, 136),   # 32 x 64 tiles
+    (24, 504, 4352),                                        # the same, K split in 8
+    (72, 1096, 4360),                                       # 64 x 64, split in 6, ragged last range
+    (1016, 384, 4544),                                      # 64 x 128, two k groups, split in 4
+    (600, 2056, 1032), (1272, 2304, 520),                   # 64 x 128 and 128 x 128
+    (1000, 5000, 328),                                      # 128 x 256
+    (1288, 6152, 776), (1376, 3120, 4888),                  # 256 x 256, whole and split in 3
+])
+@pytest.mark.parametrize("act", ["none", "silu"])
+def test_bf16_tiles(dev, M, N, K, act):
+    case(f"gemm bf16 tiles {M}x{N}x{K} {act}")
+    A, B, bias = _operands(dev, M, N, K, M + N + K)
+    bias = bias if act == "silu" else None
+    y = ops.gemm_bias_act(A, B, bias, act)
+    _check(y, A, B, bias, act)
+    assert torch.equal(y, ops.gemm_bias_act(A, B, bias, act))
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 8, 1 << 22), (8, 1 << 24, 8)])
+def test_bf16_long_rows(dev, M, N, K):
+    case(f"gemm bf16 long rows {M}x{N}x{K}")
+    A, B, _ = _operands(dev, M, N, K, 1)
+    _check(ops.gemm_bias_act(A, B, None, "none"), A, B, None, "none")
+
+
+@pytest.mark.parametrize("K", [8, 40, 72, 4360])
+def test_bf16_k_tail_keeps_rows_apart(dev, K):
+    """An infinity in one row of A may not reach the row before it through
+    the part of a K slice past the row's end."""
+    case(f"gemm bf16 K tail {K}")
+    A, B, _ = _operands(dev, 40, 136, K, 5)
+    A[1::2] = float("inf")
+    y = ops.gemm_bias_act(A, B, None, "none")
+    _check(y[::2], A[::2].contiguous(), B, None, "none")
+    assert not torch.isfinite(y[1::2]).any()
+
+
+def test_bf16_split_under_capture(dev):
+    """A shape whose K is split outside a graph: the captured call replays
+    with the program's own calls in between."""
+    case("gemm bf16 split under capture")
+    A, B, bias = _operands(dev, 24, 504, 4352, 9)
+    y = torch.empty((24, 504), dtype=torch.bfloat16, device=dev)
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        ops.gemm_bias_act(A, B, bias, "silu", out=y)
+    for i in range(3):
+        A.copy_((torch.randn(A.shape, device=dev) / 66).bfloat16())
+        g.replay()
+        eager = ops.gemm_bias_act(A, B, bias, "silu")
+        torch.cuda.synchronize()
+        _check(y, A, B, bias, "silu")
+        _check(eager, A, B, bias, "silu")
