@@ -572,58 +572,19 @@ __global__ __launch_bounds__(256) void gemm_bf16_reduce_kernel(const float* __re
     JH_DISPATCH_ACT(act, ACT, *reinterpret_cast<u32x4_t*>(C + i) = act_pack8<ACT>(v));
 }
 
-// The tile kernel's configurations: waves, slice bytes and ring depth as
-// measured best per tile, and the plan's cost model.  A launch of `wg`
-// workgroups over kc elements each takes about
-//   base + rounds * (kc * per_k + round) us,
-// rounds = ceil(wg / 256), times `shared` where two workgroups share a CU,
-// and K split in S adds split_base + 0.19 S + 1.2e-6 S M N us for the partial
-// sums and their reduction.  The constants are a least-squares fit to 250
-// shapes (M 24-4096, N and K 256-8192) timed at every tile and S: its choice
-// is 2 % off the best of them on average.  Larger tiles move fewer bytes per
-// output (per_k / (BM BN) falls from 1.2 to 0.34 ps), smaller ones fill the
-// chip sooner.
-struct TilePlan {
-    int bm, bn, bk;
-    float base, per_k, round, shared;
-};
-constexpr TilePlan kTilePlans[] = {
-    {32, 64, 64, 5.0f, 0.0024f, 1.2f, 0.79f},  {64, 64, 64, 5.9f, 0.0025f, 0.4f, 1.1f},
-    {64, 128, 64, 2.0f, 0.0039f, 4.2f, 1.0f},  {128, 128, 64, 0.7f, 0.0062f, 6.0f, 1.0f},
-    {128, 256, 32, 0.5f, 0.0126f, 7.2f, 1.0f}, {256, 256, 32, 1.7f, 0.0222f, 8.1f, 1.0f},
-};
-constexpr int kTilePlanCount = sizeof(kTilePlans) / sizeof(kTilePlans[0]);
-constexpr int64_t kMaxPartialBytes = int64_t(64) << 20;  // bound of the split's workspace
-
-struct TileChoice {
-    int plan, splits, kc;
-};
-
-TileChoice tile_choice(int M, int N, int K, bool may_split) {
-    TileChoice best{0, 1, 0};
-    float best_us = 0.0f;
-    for (int c = 0; c < kTilePlanCount; ++c) {
-        const TilePlan& p = kTilePlans[c];
-        const int64_t tiles = ((int64_t)(M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn);
-        const int slices = (K + p.bk - 1) / p.bk;
-        for (int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
-            if (S > 1 && (!may_split || slices < 2 * S || tiles * S > 512 ||
-                          (int64_t)S * M * N * 4 > kMaxPartialBytes))
-                break;
-            const int per = (slices + S - 1) / S;
-            const int z = slices ? (slices + per - 1) / per : 1;
-            const float rounds = (float)((tiles * z + 255) / 256);
-            float us = p.base + (rounds > 1.0f ? rounds * p.shared : 1.0f) *
-                                    ((float)per * p.bk * p.per_k + p.round);
-            if (z > 1) us += 1.75f + 0.19f * z + 1.2e-6f * z * M * N;
-            if (best_us == 0.0f || us < best_us) {
-                best_us = us;
-                best = {c, z, per * p.bk};
-            }
-        }
-    }
-    return best;
-}
+// The tile kernel's tiles, with the waves, slice bytes and ring depth measured
+// best for each.  The model is a least-squares fit to 250 shapes (M 24-4096, N
+// and K 256-8192) timed at every tile and split: its choice is 2 % off the
+// best of them on average.  Larger tiles move fewer bytes per output (per_k /
+// (bm bn) falls from 1.2 to 0.34 ps), smaller ones fill the chip sooner.
+constexpr TileModel kBf16Model = {
+    {{32, 64, 64, 5.0f, 0.0024f, 1.2f, 0.79f},
+     {64, 64, 64, 5.9f, 0.0025f, 0.4f, 1.1f},
+     {64, 128, 64, 2.0f, 0.0039f, 4.2f, 1.0f},
+     {128, 128, 64, 0.7f, 0.0062f, 6.0f, 1.0f},
+     {128, 256, 32, 0.5f, 0.0126f, 7.2f, 1.0f},
+     {256, 256, 32, 1.7f, 0.0222f, 8.1f, 1.0f}},
+    0.0f, 1.75f, 0.19f, 1.2e-6f};
 
 template <class T>
 void launch_tile(int act, const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C, float* part,
@@ -644,21 +605,10 @@ hipError_t launch_gemm_bf16(int act, const uint16_t* A, const uint16_t* B, const
                                                      A, B, bias, C, M, N, K));
         return hipGetLastError();
     }
-    // Partial sums live in the stream's workspace.  It may not be allocated
-    // while a graph is being captured, nor kept by the graph (a later call may
-    // replace it), and streams that share a handle may not share it.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    bool may_split = s != hipStreamPerThread;
-    if (may_split && hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError(), may_split = false;
-    may_split = may_split && cap == hipStreamCaptureStatusNone;
-    TileChoice c = tile_choice(M, N, K, may_split);
-    void* ws = nullptr;
     WorkspaceLock lock;
-    if (c.splits > 1 && stream_workspace((size_t)c.splits * M * N * 4, s, &ws, &lock) != hipSuccess) {
-        (void)hipGetLastError();
-        c = tile_choice(M, N, K, false);
-    }
-    float* part = c.splits > 1 ? static_cast<float*>(ws) : nullptr;
+    void* ws;
+    const TileChoice c = tile_plan(kBf16Model, M, N, K, s, &ws, &lock);
+    float* part = static_cast<float*>(ws);
     switch (c.plan) {
     case 0: launch_tile<TileCfg<Bf16Op, 32, 64, 1, 2, 1, 128, 6, 3>>(act, A, B, bias, C, part, M, N, K, c, s); break;
     case 1: launch_tile<TileCfg<Bf16Op, 64, 64, 2, 2, 1, 128, 4, 3>>(act, A, B, bias, C, part, M, N, K, c, s); break;

@@ -36,6 +36,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "launch.hpp"
 
 namespace jh {
 
@@ -371,6 +372,73 @@ __device__ __forceinline__ TileCoord tile_coord(int tiles_m, int tiles_n) {
     const int band = t / (GM * tiles_n), first = band * GM;
     const int gs = min(GM, tiles_m - first), in = t - band * GM * tiles_n;
     return {first + in % gs, in / gs, z};
+}
+
+// Which tile and how many K ranges a launch takes: the least of a cost model
+// over the tiles.  `wg` workgroups over kc elements each take about
+//   base + rounds * (kc * per_k * (1 + fill * min(1, wg / 256)) + round) us,
+// rounds = ceil(wg / 256), times `shared` where two workgroups share a CU, and
+// S K ranges add split_base + split_z S + split_mn S M N us for the partial
+// sums and their reduction.  Each operand type has its own constants, fitted
+// to measured times (gemm_bf16.hip, matmul_int8.hip).
+struct TilePlan {
+    int bm, bn, bk;
+    float base, per_k, round, shared;
+};
+struct TileModel {
+    TilePlan plan[6];
+    float fill, split_base, split_z, split_mn;
+};
+struct TileChoice {
+    int plan, splits, kc;
+};
+constexpr int64_t kMaxPartialBytes = int64_t(64) << 20;  // bound of the split's workspace
+
+inline TileChoice tile_choice(const TileModel& m, int M, int N, int K, bool may_split) {
+    TileChoice best{0, 1, 0};
+    float best_us = 0.0f;
+    for (int c = 0; c < 6; ++c) {
+        const TilePlan& p = m.plan[c];
+        const int64_t tiles = (((int64_t)M + p.bm - 1) / p.bm) * (((int64_t)N + p.bn - 1) / p.bn);
+        const int slices = (K + p.bk - 1) / p.bk;
+        for (int S : {1, 2, 3, 4, 6, 8}) {
+            if (S > 1 && (!may_split || slices < 2 * S || tiles * S > 512 ||
+                          (int64_t)S * M * N * 4 > kMaxPartialBytes))
+                break;
+            const int per = (slices + S - 1) / S;
+            const int z = slices ? (slices + per - 1) / per : 1;
+            const int64_t wg = tiles * z;
+            const float rounds = (float)((wg + 255) / 256);
+            const float per_k = p.per_k * (1.0f + m.fill * (wg < 256 ? (float)wg / 256.0f : 1.0f));
+            float us = p.base + (rounds > 1.0f ? rounds * p.shared : 1.0f) *
+                                    ((float)per * (float)p.bk * per_k + p.round);
+            if (z > 1) us += m.split_base + m.split_z * z + m.split_mn * z * M * N;
+            if (best_us == 0.0f || us < best_us) {
+                best_us = us;
+                best = {c, z, per * p.bk};
+            }
+        }
+    }
+    return best;
+}
+
+// tile_choice with the partial sums' memory: the stream's workspace, under its
+// lock until the caller has enqueued the reduction.  It may not be allocated
+// while a graph is being captured, nor kept by the graph (a later call may
+// replace it), and hipStreamPerThread is one handle for many streams: there,
+// and without memory for it, K is not split.
+inline TileChoice tile_plan(const TileModel& m, int M, int N, int K, hipStream_t s, void** part,
+                            WorkspaceLock* lock) {
+    *part = nullptr;
+    TileChoice c = tile_choice(m, M, N, K, s != hipStreamPerThread);
+    if (c.splits == 1) return c;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+        stream_workspace((size_t)c.splits * M * N * 4, s, part, lock) == hipSuccess)
+        return c;
+    (void)hipGetLastError();
+    *part = nullptr;
+    return tile_choice(m, M, N, K, false);
 }
 
 }  // namespace jh

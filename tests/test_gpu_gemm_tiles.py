@@ -86,3 +86,43 @@ def test_bf16_split_under_capture(dev):
         torch.cuda.synchronize()
         _check(y, A, B, bias, "silu")
         _check(eager, A, B, bias, "silu")
+
+
+def _int8_ref(A, B, rs, cs, bias):
+    """The scalar path's arithmetic on the exact integer sums (each below
+    2^31, so the float64 product holds it exactly)."""
+    z = (A.double() @ B.double()).float() * (rs * cs)
+    return z if bias is None else z + bias
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (17, 16, 16), (40, 272, 144),                       # 32 x 64 tiles
+    (39, 2960, 8128), (72, 1104, 4368),                 # 64 x 64, K split, ragged last range
+    (645, 688, 6768), (540, 4112, 1040),                # 64 x 128, split in 3 and whole
+    (222, 5264, 7328), (1000, 2064, 912),               # 128 x 128
+    (796, 5616, 6864),                                  # 128 x 256
+    (1304, 6160, 784), (768, 1280, 320),                # 256 x 256; whole tiles
+    (1, 1, 1), (3, 65, 17), (64, 64, 64 - 1), (65, 130, 129), (33, 1000, 255),  # rows of any length
+])
+def test_int8_tiles(dev, M, N, K):
+    case(f"int8 tiles {M}x{N}x{K}")
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    A = torch.randint(-128, 128, (M, K), generator=g, device=dev, dtype=torch.int8)
+    B = torch.randint(-128, 128, (K, N), generator=g, device=dev, dtype=torch.int8)
+    sa = torch.rand((M,), generator=g, device=dev) + 0.01
+    sb = torch.rand((N,), generator=g, device=dev) + 0.01
+    bias = torch.rand((N,), generator=g, device=dev) - 0.5
+    assert torch.equal(ops.matmul_w8a8(A, B, sa, sb, bias), _int8_ref(A, B, sa[:, None], sb, bias))
+    f32 = torch.tensor(0.013, device=dev), torch.tensor(0.021, device=dev)
+    assert torch.equal(ops.matmul_int8(A, B, 0.013, 0.021), _int8_ref(A, B, *f32, None))
+
+
+def test_int8_misaligned_operands(dev):
+    """Operands that start between 16-byte addresses, and end with their
+    allocation's last byte."""
+    case("int8 misaligned")
+    M, N, K = 50, 96, 80
+    buf = torch.randint(-128, 128, (M * K + K * N + 3,), device=dev, dtype=torch.int8)
+    A, B = buf[3:3 + M * K].view(M, K), buf[3 + M * K:].view(K, N)
+    one = torch.ones((), device=dev)
+    assert torch.equal(ops.matmul_int8(A, B, 1.0, 1.0), _int8_ref(A, B, one, one, None))
