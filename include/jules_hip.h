@@ -103,15 +103,16 @@ int jules_hip_gemm_bias_act(int dtype, int act, const void* A, const void* B,
                             void* stream);
 
 /* ---- GEMM tile table -------------------------------------------------------
- * out[4] = {kernel variant, tile_m, tile_n, tile_k} that
- * jules_hip_gemm_bias_act launches for this dtype and shape (needs no GPU).
- * Variants: 0/1 fp32 row kernel with 1/2 rows per wave (tile 4 or 8 rows x
- * 64 columns, all of K in LDS, K <= 2048), 2/3 fp32 32x32 / 64x64 tiles with
- * 32-deep K slices, 4 bf16 256x256 tiles with 32-deep LDS-DMA stages, 5 the
- * other bf16 shapes (the largest tile is given; a launch takes tiles from
- * 32x64 up and splits K by a cost model of the shape).  Replaces the role of
- * TilePlanner::getTileConfig (reference TilePlanner.h:74-136), which sizes
- * tiles for the CPU caches; jules::kernel::TilePlanner returns these.
+ * out[4] = {entry, tile_m, tile_n, tile_k} of the table that plans
+ * jules_hip_gemm_bias_act for this dtype and shape (needs no GPU).
+ * Entries: 0/1 fp32 by rows, 1/2 rows per wave (4 or 8 rows x 64 columns, all
+ * of K, K <= 2048), 2/3 fp32 32x32 / 64x64 tiles with 32-deep K slices, 4 bf16
+ * 256x256 tiles with 32-deep LDS-DMA stages, 5 the other bf16 shapes.  An
+ * entry is a class of shapes: the launch picks its workgroup tile within it
+ * (fp32 32x32 to 128x128, bf16 32x64 to 256x256 with K split), which never
+ * changes fp32 results.  Replaces the role of TilePlanner::getTileConfig
+ * (reference TilePlanner.h:74-136), which sizes tiles for the CPU caches;
+ * jules::kernel::TilePlanner returns these.
  */
 int jules_hip_gemm_tile(int dtype, int M, int N, int K, int* out);
 

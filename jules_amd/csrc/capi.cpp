@@ -62,9 +62,9 @@ int set_last_error(int status, const std::string& message) {
     return status;
 }
 
-// jules_hip_gemm_bias_act for fp32 with a chosen kernel of the tile table
-// (variant < 0: the table's default for the shape).  Every variant gives the
-// same bits, so the choice changes speed only.
+// jules_hip_gemm_bias_act for fp32 with a chosen entry of the tile table
+// (variant < 0: the table's default for the shape), which must be able to
+// take the shape; the launch picks its own tile, every one with the same bits.
 int gemm_f32_with_variant(int variant, int act, const float* A, const float* B, const float* bias,
                           float* C, int M, int N, int K, hipStream_t s) {
     if (!valid_act(act)) return fail(JH_ERR_ACT, "gemm: activation code %d", act);
@@ -78,8 +78,7 @@ int gemm_f32_with_variant(int variant, int act, const float* A, const float* B, 
     if (!C || (K > 0 && (!A || !B))) return fail(JH_ERR_NULL, "gemm: null A, B or C");
     if (!aligned(A, 4) || !aligned(B, 4) || !aligned(C, 4) || !aligned(bias, 4))
         return fail(JH_ERR_ALIGN, "gemm f32: operands must be 4-byte aligned");
-    return check_hip(launch_gemm_f32_variant(variant, act, A, B, bias, C, M, N, K, s),
-                     "gemm f32 launch");
+    return check_hip(launch_gemm_f32(act, A, B, bias, C, M, N, K, s), "gemm f32 launch");
 }
 }  // namespace jh
 

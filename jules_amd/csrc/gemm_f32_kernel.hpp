@@ -1,0 +1,117 @@
+// gemm_f32_kernel.hpp - the kernel of the fp32 MFMA GEMM tiles and its launch
+// for one pair of operand orientations (gemm_f32_tile.hip and
+// gemm_f32_tile_t.hip compile it for op(A) op(B) without and with transposes).
+#pragma once
+
+#include "gemm_f32_tile.hpp"
+#include "gemm_tile.hpp"
+
+namespace jh {
+
+template <int MF_, int MT_, int NT_, int BK_, int PF_>
+struct F32Cfg {
+    static constexpr int MF = MF_, MT = MT_, NT = NT_, BK = BK_, PF = PF_;
+    static constexpr int BM = 2 * MT * MF, BN = 2 * NT * MF;
+};
+
+// BLAS sgemm epilogue: alpha * acc + beta * C, with C not read when beta = 0
+// (so NaNs in an uninitialised C never propagate)
+__device__ __forceinline__ float alpha_beta(float acc, float alpha, float beta, const float* c) {
+    const float v = alpha * acc;
+    return beta == 0.0f ? v : v + beta * *c;
+}
+
+// The epilogue g.epi over each(f), which calls f(m, n, sum, bias of column n).
+// ACTS: with the activations (the transposed products only take "none").
+template <bool ACTS, typename Each>
+__device__ __forceinline__ void finish(const F32Gemm& g, Each&& each) {
+    if (g.epi == F32_EPI_MASK) {
+        each([&](int m, int n, float v, float) {
+            g.C[(int64_t)m * g.ldc + n] = g.mask[(int64_t)m * g.ldm + n] > 0.0f ? v : 0.0f;
+        });
+    } else if (g.epi == F32_EPI_ALPHA_BETA) {
+        each([&](int m, int n, float v, float) {
+            float* c = g.C + (int64_t)m * g.ldc + n;
+            *c = alpha_beta(v, g.alpha, g.beta, c);
+        });
+    } else if constexpr (ACTS) {
+        JH_DISPATCH_ACT(g.act, ACT, each([&](int m, int n, float v, float b) {
+                            if (g.bias) v = v + b;
+                            g.C[(int64_t)m * g.ldc + n] = activate<ACT>(v);
+                        }));
+    } else {
+        each([&](int m, int n, float v, float) { g.C[(int64_t)m * g.ldc + n] = v; });
+    }
+}
+
+template <class CF, bool TA, bool TB, int V>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Gemm g, int kc, float* __restrict__ part) {
+    using T = F32Tile<CF::MF, CF::MT, CF::NT, CF::BK, CF::PF, TA, TB, V>;
+    constexpr bool ACTS = !TA && !TB;
+    __shared__ __attribute__((aligned(16))) float sm[2 * T::STAGE];
+    const TileCoord t = tile_coord<8>((g.M + T::BM - 1) / T::BM, (g.N + T::BN - 1) / T::BN);
+    const int m0 = t.tm * T::BM, n0 = t.tn * T::BN, kb = t.z * kc;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int mw = m0 + (wave >> 1) * CF::MT * CF::MF, nw = n0 + (wave & 1) * CF::NT * CF::MF + lane % CF::MF;
+    // the bias is in registers before the sums are (loaded after them, it costs
+    // a small product a memory latency)
+    float bias[CF::NT];
+#pragma unroll
+    for (int j = 0; j < CF::NT; ++j)
+        bias[j] = ACTS && g.bias ? g.bias[min(nw + j * CF::MF, g.N - 1)] : 0.0f;
+
+    typename T::Mf::Acc acc[CF::MT][CF::NT];
+    T::run(g.A, g.lda, g.B, g.ldb, m0, g.M, n0, g.N, kb, min(g.K, kb + kc), sm, acc);
+
+    auto each = [&](auto&& f) {
+#pragma unroll
+        for (int j = 0; j < CF::NT; ++j) {
+            const int n = nw + j * CF::MF;
+            if (n >= g.N) continue;
+#pragma unroll
+            for (int i = 0; i < CF::MT; ++i)
+#pragma unroll
+                for (int e = 0; e < T::Mf::NR; ++e) {
+                    const int m = mw + i * CF::MF + T::Mf::row(lane, e);
+                    if (m < g.M) f(m, n, acc[i][j][e], bias[j]);
+                }
+        }
+    };
+    if (part) {
+        float* p = part + (int64_t)t.z * g.M * g.N;
+        each([&](int m, int n, float v, float) { p[(int64_t)m * g.N + n] = v; });
+    } else {
+        finish<ACTS>(g, each);
+    }
+}
+
+using F32Cfg0 = F32Cfg<16, 1, 1, 64, 1>;
+using F32Cfg1 = F32Cfg<16, 2, 2, 32, 2>;
+using F32Cfg2 = F32Cfg<16, 2, 4, 16, 1>;
+using F32Cfg3 = F32Cfg<32, 2, 2, 16, 1>;
+
+template <bool TA, bool TB>
+void launch_f32_tile(int plan, bool v4, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
+    auto go = [&](auto cfg, auto v) {
+        using CF = decltype(cfg);
+        const int64_t wg =
+            (((int64_t)g.M + CF::BM - 1) / CF::BM) * (((int64_t)g.N + CF::BN - 1) / CF::BN) * splits;
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<CF, TA, TB, decltype(v)::value>), dim3((unsigned)wg), dim3(256), 0,
+                           s, g, kc, part);
+    };
+    auto pick = [&](auto v) {
+        switch (plan) {
+        case 0: go(F32Cfg0{}, v); break;
+        case 1: go(F32Cfg1{}, v); break;
+        case 2: go(F32Cfg2{}, v); break;
+        default: go(F32Cfg3{}, v); break;
+        }
+    };
+    if (v4) pick(std::integral_constant<int, 4>{});
+    else pick(std::integral_constant<int, 1>{});
+}
+
+// gemm_f32_tile_t.hip: at least one of ta, tb
+void launch_f32_tile_trans(int plan, bool v4, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s);
+
+}  // namespace jh

@@ -1,0 +1,75 @@
+// gemm_f32_tile.hip - the launch of the fp32 MFMA GEMM (gemm_f32_tile.hpp): the
+// fused GEMM of gemm_f32.hip, the MLP products and sgemm of mlp.hip.
+#include "gemm_f32_kernel.hpp"
+
+namespace jh {
+namespace {
+
+// C = epilogue(sum over z of part[z], in z order)
+__global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(F32Gemm g, int S, const float* __restrict__ part) {
+    const int64_t total = (int64_t)g.M * g.N, stride = (int64_t)gridDim.x * 256;
+    finish<true>(g, [&](auto&& f) {
+        for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += stride) {
+            float v = part[e];
+#pragma unroll 4
+            for (int z = 1; z < S; ++z) v += part[(int64_t)z * total + e];
+            const int m = (int)(e / g.N), n = (int)(e - (int64_t)m * g.N);
+            f(m, n, v, g.bias ? g.bias[n] : 0.0f);
+        }
+    });
+}
+
+// The tiles, and what they cost: n = ceil(workgroups / 256) tiles on a CU take
+// n (k * per_k + round) us, one alone k * alone + round (its own latencies
+// uncovered).  Measured at 4096^3, 2000 x 3072 x 1024, 1024^3 and 64 x 512 x
+// 2048: per output the larger tiles are up to 1.4 times as fast (5.5 ns per k
+// and 1024 outputs at 32 x 32, 4.0 at 128 x 128), the smaller ones fill the
+// chip and split the fma chain's latency over more waves.
+struct F32Plan {
+    int bm, bn;
+    float per_k, alone, round;
+};
+constexpr F32Plan kF32Plans[4] = {{32, 32, 0.0055f, 0.0064f, 1.0f},
+                                  {64, 64, 0.0175f, 0.024f, 1.1f},
+                                  {64, 128, 0.034f, 0.042f, 1.4f},
+                                  {128, 128, 0.065f, 0.075f, 3.0f}};
+
+int f32_plan(int M, int N, int kc, int splits) {
+    int best = 0;
+    float best_us = 0.0f;
+    for (int c = 0; c < 4; ++c) {
+        const F32Plan& p = kF32Plans[c];
+        const int64_t wg = (((int64_t)M + p.bm - 1) / p.bm) * (((int64_t)N + p.bn - 1) / p.bn) * splits;
+        const float n = (float)((wg + 255) / 256);
+        const float us = n > 1.0f ? n * (kc * p.per_k + p.round) : kc * p.alone + p.round;
+        if (c == 0 || us < best_us) {
+            best_us = us;
+            best = c;
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
+    if (g.M == 0 || g.N == 0) return hipSuccess;
+    if (splits <= 1) {
+        splits = 1;
+        kc = g.K;
+        part = nullptr;
+    }
+    // 16-byte pieces along the contiguous dimension of both operands
+    const bool v4 = (g.ta ? g.M : g.K) % 4 == 0 && (g.tb ? g.K : g.N) % 4 == 0;
+    const int plan = f32_plan(g.M, g.N, kc, splits);
+    if (g.ta || g.tb) launch_f32_tile_trans(plan, v4, g, splits, kc, part, s);
+    else launch_f32_tile<false, false>(plan, v4, g, splits, kc, part, s);
+    if (part) {
+        int64_t b = ((int64_t)g.M * g.N + 255) / 256;
+        if (b > 2048) b = 2048;
+        hipLaunchKernelGGL(gemm_f32_reduce_kernel, dim3((unsigned)b), dim3(256), 0, s, g, splits, part);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace jh

@@ -1,0 +1,12 @@
+// gemm_f32_tile_t.hip - the fp32 MFMA GEMM tiles with a transposed operand.
+#include "gemm_f32_kernel.hpp"
+
+namespace jh {
+
+void launch_f32_tile_trans(int plan, bool v4, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
+    if (!g.tb) launch_f32_tile<true, false>(plan, v4, g, splits, kc, part, s);
+    else if (!g.ta) launch_f32_tile<false, true>(plan, v4, g, splits, kc, part, s);
+    else launch_f32_tile<true, true>(plan, v4, g, splits, kc, part, s);
+}
+
+}  // namespace jh

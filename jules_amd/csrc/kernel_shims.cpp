@@ -220,11 +220,11 @@ TileConfig TilePlanner::autoTune(int M, int N, int K, const TileConfig& defaultC
     for (int v = jh::GV_F32_ROWS1; ok && v <= jh::GV_F32_T64; ++v) {
         if (!jh::f32_variant_valid(v, K)) continue;
         constexpr int iters = 10;
-        ok = jh::launch_gemm_f32_variant(v, JH_ACT_NONE, A, B, nullptr, C, M, N, K, nullptr) ==
+        ok = jh::launch_gemm_f32(JH_ACT_NONE, A, B, nullptr, C, M, N, K, nullptr) ==
                  hipSuccess &&
              hipEventRecord(e0, nullptr) == hipSuccess;
         for (int i = 0; ok && i < iters; ++i)
-            ok = jh::launch_gemm_f32_variant(v, JH_ACT_NONE, A, B, nullptr, C, M, N, K, nullptr) ==
+            ok = jh::launch_gemm_f32(JH_ACT_NONE, A, B, nullptr, C, M, N, K, nullptr) ==
                  hipSuccess;
         float ms = 0.0f;
         ok = ok && hipEventRecord(e1, nullptr) == hipSuccess &&

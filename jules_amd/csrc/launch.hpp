@@ -12,11 +12,31 @@ namespace jh {
 
 hipError_t launch_gemm_f32(int act, const float* A, const float* B, const float* bias,
                            float* C, int M, int N, int K, hipStream_t s);
-// one fp32 GEMM kernel of the tile table (tiles.hpp: GV_F32_*); the caller
-// has checked f32_variant_valid()
-hipError_t launch_gemm_f32_variant(int variant, int act, const float* A, const float* B,
-                                   const float* bias, float* C, int M, int N, int K,
-                                   hipStream_t s);
+// fp32 GEMM on the MFMA tiles (gemm_f32_tile.hip): C = epilogue(op(A) op(B)),
+// row-major, op(X) = X^T when ta / tb.  Each output is one fma chain over k =
+// 0 .. K-1 in order unless K is split: `splits` ranges of kc (a multiple of
+// 64), whose sums go to part[splits][M][N] and are added in order.
+enum F32Epi {
+    F32_EPI_ACT = 0,     // act(sum [+ bias[n]])
+    F32_EPI_MASK,        // mask[m][n] > 0 ? sum : 0
+    F32_EPI_ALPHA_BETA,  // alpha * sum + beta * C
+};
+struct F32Gemm {
+    bool ta, tb;
+    const float* A;
+    int64_t lda;
+    const float* B;
+    int64_t ldb;
+    float* C;
+    int64_t ldc;
+    int M, N, K;
+    int epi, act;
+    const float* bias;
+    const float* mask;
+    int64_t ldm;
+    float alpha, beta;
+};
+hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s);
 // the fp32 GEMM entry point's validation and launch with a chosen table
 // variant (-1: the table's default), for jules::kernel::tiledMatmulWithActivation
 int gemm_f32_with_variant(int variant, int act, const float* A, const float* B, const float* bias,

@@ -1,20 +1,16 @@
 // tiles.hpp - the gfx950 GEMM tile table of libjules_hip (internal).
 //
-// One table decides which kernel, and so which workgroup tile, every GEMM
-// launch uses.  The launchers (gemm_f32.hip, gemm_bf16.hip) read it, and so
-// does jules::kernel::TilePlanner (kernel_shims.cpp), whose getTileConfig
-// therefore returns the tile that actually runs (the reference's planner,
-// TilePlanner.h:74-136, sizes tiles for the CPU caches instead).
+// The table jules_hip_gemm_tile and jules::kernel::TilePlanner
+// (kernel_shims.cpp) plan with (the reference's planner, TilePlanner.h:74-136,
+// sizes tiles for the CPU caches instead).  It classifies shapes; within a
+// class the launchers (gemm_f32_tile.hip, gemm_bf16.hip) pick the workgroup
+// tile by their own measured costs.
 //
-// fp32 (the bit-exact fma-chain GEMM): every variant computes each output as
-// the same sequential fma chain over k, so the choice changes speed, never
-// bits.  The variants:
-//   F32_ROWS1 / F32_ROWS2: a wave owns 1 or 2 rows x 64 columns, 4 waves per
-//     workgroup; the workgroup's rows of A (all of K) sit in LDS, so K is
-//     limited to kF32RowsMaxK, and B streams through an LDS ring by LDS DMA.
-//     Tile (4*rw) x 64 x K.
-//   F32_T32 / F32_T64: 32x32 (2x2 per thread) and 64x64 (4x4 per thread)
-//     output tiles, A and B staged through LDS in K slices of 32.
+// fp32 (the bit-exact fma-chain GEMM): every output is the same sequential fma
+// chain over k whatever the entry, so the choice never changes bits.
+//   F32_ROWS1 / F32_ROWS2: outputs so few that 4 or 8 rows x 64 columns over
+//     all of K is a workgroup's share (K <= kF32RowsMaxK).
+//   F32_T32 / F32_T64: 32x32 and 64x64 output tiles in K slices of 32.
 // bf16 (MFMA): BF16_DMA, 256x256 output tiles of 4 waves over 32-deep K slices
 // by LDS DMA, can run whole tiles only; BF16_REG stands for every other shape.
 // Which kernel and tile a launch takes is the cost model of gemm_bf16.hip.
@@ -41,9 +37,9 @@ struct GemmTile {
     int tile_k;
 };
 
-constexpr int kF32RowsWaves = 4;     // waves per row-kernel workgroup
-constexpr int kF32RowsMaxK = 2048;   // 2 rows x 4 waves x K floats of A in 64 KiB of LDS
-constexpr int kF32SliceK = 32;       // K slice of the LDS-tiled fp32 kernels
+constexpr int kF32RowsWaves = 4;     // waves of a rows entry
+constexpr int kF32RowsMaxK = 2048;   // longest K of a rows entry
+constexpr int kF32SliceK = 32;       // K slice of the 32x32 and 64x64 entries
 constexpr int kBf16Tile = 256;       // bf16 output tile (both variants)
 constexpr int kBf16DmaK = 32;        // k per LDS-DMA stage
 constexpr int kBf16RegK = 64;        // k per register-staged slice
@@ -62,11 +58,9 @@ inline GemmTile f32_variant_tile(int v, int K) {
     }
 }
 
-// The variant an fp32 GEMM launch uses.  Up to 1M outputs (and K within the
-// row kernel's LDS): the row kernel, 2 rows per wave, or 1 when 2 would
-// leave fewer than 1024 waves (512^3: 21.7 us at 2 rows, 27.1 us at 1;
-// 64x256x784: 20.4 us at 1 row, 23.6 us at 2).  Larger: 64x64 tiles once
-// there are at least 512 of them (two per CU), else 32x32.
+// The entry of an fp32 shape.  Up to 1M outputs (and K <= kF32RowsMaxK): rows,
+// 2 per wave, or 1 when 2 would leave fewer than 1024 waves.  Larger: 64x64
+// tiles once there are at least 512 of them (two per CU), else 32x32.
 inline GemmTile f32_gemm_tile(int M, int N, int K) {
     if ((int64_t)M * N <= (int64_t(1) << 20) && K <= kF32RowsMaxK) {
         const bool one = (((int64_t)N + 63) / 64) * (((int64_t)M + 1) / 2) < 1024;

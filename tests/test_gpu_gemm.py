@@ -138,3 +138,31 @@ def test_activation_kernel_bit_exact(dev):
         y = to_np(ops.activation(dx, act))
         np.testing.assert_array_equal(y, po.act_array(act, x))
     np.testing.assert_array_equal(to_np(ops.activation(dx, "gelu")), po.fused_gelu(x))
+
+
+def _special(seed, shape):
+    """Values whose products and sums meet every corner of an fma: signed
+    zeros, ones, subnormals, numbers whose products are subnormal or overflow."""
+    v = I.uniform(seed, 0, shape, -1, 1)
+    pool = np.array([0.0, -0.0, 1.0, -1.0, 1e-40, -3e-39, 1e-25, -1e-22, 1e25, -3e19], np.float32)
+    pick = (I.uniform(seed, 1, shape, 0, 16)).astype(np.int64)
+    return np.where(pick < len(pool), pool[np.minimum(pick, len(pool) - 1)], v).astype(np.float32)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (33, 48, 65), (32, 32, 64), (1, 16, 3),             # 32 x 32 tiles, K tails, 4-byte and 16-byte loads
+    (1025, 1040, 33), (1024, 1008, 36),                 # 64 x 64
+    (1000, 2064, 70), (1024, 2048, 20),                 # 64 x 128
+    (2049, 4112, 17), (2048, 4096, 48),                 # 128 x 128
+])
+def test_f32_tiles_bit_exact(dev, M, N, K):
+    """Every tile at its edges is the oracle's fma chain bit for bit, on
+    ordinary values and on those where a different chain or a k past the end
+    would show (a -0 sum, a subnormal, an overflow)."""
+    case(f"gemm f32 tiles {M}x{N}x{K}")
+    A, B, _ = I.gemm_inputs(M, N, K, "f32", seed=M + N + K)
+    np.testing.assert_array_equal(_gemm_f32(dev, A, B, None, "none"), po.tiled_matmul_act(A, B, "none"))
+    A, B = _special(M, (M, K)), _special(N + 7, (K, N))
+    y, r = _gemm_f32(dev, A, B, None, "none"), po.tiled_matmul_act(A, B, "none")
+    same = (y.view(np.int32) == r.view(np.int32)) | (np.isnan(y) & np.isnan(r))
+    assert same.all(), f"{(~same).sum()} of {same.size} differ"
