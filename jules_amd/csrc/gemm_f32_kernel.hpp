@@ -89,29 +89,36 @@ using F32Cfg0 = F32Cfg<16, 1, 1, 64, 1>;
 using F32Cfg1 = F32Cfg<16, 2, 2, 32, 2>;
 using F32Cfg2 = F32Cfg<16, 2, 4, 16, 1>;
 using F32Cfg3 = F32Cfg<32, 2, 2, 16, 1>;
+using F32Cfg4 = F32Cfg<16, 1, 1, 128, 1>;
 
 template <bool TA, bool TB>
-void launch_f32_tile(int plan, bool v4, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
-    auto go = [&](auto cfg, auto v) {
+void launch_f32_tile(int plan, int v, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
+    auto go = [&](auto cfg, auto vec) {
         using CF = decltype(cfg);
         const int64_t wg =
             (((int64_t)g.M + CF::BM - 1) / CF::BM) * (((int64_t)g.N + CF::BN - 1) / CF::BN) * splits;
-        hipLaunchKernelGGL((gemm_f32_tile_kernel<CF, TA, TB, decltype(v)::value>), dim3((unsigned)wg), dim3(256), 0,
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<CF, TA, TB, decltype(vec)::value>), dim3((unsigned)wg), dim3(256), 0,
                            s, g, kc, part);
     };
-    auto pick = [&](auto v) {
+    auto pick = [&](auto vec) {
         switch (plan) {
-        case 0: go(F32Cfg0{}, v); break;
-        case 1: go(F32Cfg1{}, v); break;
-        case 2: go(F32Cfg2{}, v); break;
-        default: go(F32Cfg3{}, v); break;
+        case 0: go(F32Cfg0{}, vec); break;
+        case 1: go(F32Cfg1{}, vec); break;
+        case 2: go(F32Cfg2{}, vec); break;
+        case 3:
+            // a transposed B's fragments spill at 128 x 128 (64 x 128 is within 4 %)
+            if constexpr (TB) go(F32Cfg2{}, vec);
+            else go(F32Cfg3{}, vec);
+            break;
+        default: go(F32Cfg4{}, vec); break;
         }
     };
-    if (v4) pick(std::integral_constant<int, 4>{});
-    else pick(std::integral_constant<int, 1>{});
+    if (v == 4) pick(std::integral_constant<int, 4>{});
+    else if (v == 1) pick(std::integral_constant<int, 1>{});
+    else go(F32Cfg0{}, std::integral_constant<int, 0>{});
 }
 
 // gemm_f32_tile_t.hip: at least one of ta, tb
-void launch_f32_tile_trans(int plan, bool v4, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s);
+void launch_f32_tile_trans(int plan, int v, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s);
 
 }  // namespace jh

@@ -1,5 +1,7 @@
 // gemm_f32_tile.hip - the launch of the fp32 MFMA GEMM (gemm_f32_tile.hpp): the
 // fused GEMM of gemm_f32.hip, the MLP products and sgemm of mlp.hip.
+#include <algorithm>
+
 #include "gemm_f32_kernel.hpp"
 
 namespace jh {
@@ -29,7 +31,7 @@ struct F32Plan {
     int bm, bn;
     float per_k, alone, round;
 };
-constexpr F32Plan kF32Plans[4] = {{32, 32, 0.0055f, 0.0064f, 1.0f},
+constexpr F32Plan kF32Plans[4] = {{32, 32, 0.0053f, 0.0062f, 1.0f},
                                   {64, 64, 0.0175f, 0.024f, 1.1f},
                                   {64, 128, 0.034f, 0.042f, 1.4f},
                                   {128, 128, 0.065f, 0.075f, 3.0f}};
@@ -47,6 +49,9 @@ int f32_plan(int M, int N, int kc, int splits) {
             best = c;
         }
     }
+    // 32 x 32 tiles alone on their CUs: half as many barriers for a long chain
+    // (64 x 512 x 2048 17.7 -> 15.9 us); with neighbours the larger LDS costs more
+    if (best == 0 && kc >= 256 && ((int64_t)M + 31) / 32 * (((int64_t)N + 31) / 32) * splits <= 256) best = 4;
     return best;
 }
 
@@ -59,11 +64,16 @@ hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hi
         kc = g.K;
         part = nullptr;
     }
-    // 16-byte pieces along the contiguous dimension of both operands
-    const bool v4 = (g.ta ? g.M : g.K) % 4 == 0 && (g.tb ? g.K : g.N) % 4 == 0;
+    // whole 16-byte pieces of the operands whose k is the outer dimension; 32-bit
+    // offsets within a tile (128 rows, or the rows there are, or a slice's 64)
+    const auto spans = [](bool rows_are_k, int rows, int64_t ld) {
+        return (int64_t)std::min(rows, rows_are_k ? 64 : 128) * ld * 4 >= (int64_t(1) << 32);
+    };
+    const bool big = spans(g.ta, g.ta ? g.K : g.M, g.lda) || spans(!g.tb, g.tb ? g.N : g.K, g.ldb);
+    const int v = big ? 0 : (!g.ta || g.M % 4 == 0) && (g.tb || g.N % 4 == 0) ? 4 : 1;
     const int plan = f32_plan(g.M, g.N, kc, splits);
-    if (g.ta || g.tb) launch_f32_tile_trans(plan, v4, g, splits, kc, part, s);
-    else launch_f32_tile<false, false>(plan, v4, g, splits, kc, part, s);
+    if (g.ta || g.tb) launch_f32_tile_trans(plan, v, g, splits, kc, part, s);
+    else launch_f32_tile<false, false>(plan, v, g, splits, kc, part, s);
     if (part) {
         int64_t b = ((int64_t)g.M * g.N + 255) / 256;
         if (b > 2048) b = 2048;

@@ -27,6 +27,8 @@
 // in different banks.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -59,11 +61,14 @@ struct f32x4_any_t {  // 16 bytes at any 4-byte address
 } __attribute__((packed, aligned(4)));
 
 // One operand's slice, X rows (columns) of the tile by BK k.  CONTIG: k is the
-// contiguous dimension in memory.  V: floats per load; 4 needs the extent of
-// the contiguous dimension to be a multiple of 4, so that a piece is wholly
-// inside or outside.
-template <int MF, int X, int BK, bool CONTIG, int V, bool IS_B>
+// contiguous dimension in memory, loaded 4 floats at a time wherever the rows
+// start (only the last slice, one float at a time, can reach past a row).  Else
+// V = 4 needs the number of rows to be a multiple of 4, so that a piece is
+// wholly inside or outside, and V = 1 does not; V = 0 is 1 with 64-bit offsets.
+template <int MF, int X, int BK, bool CONTIG, int V_, bool IS_B>
 struct F32Slice {
+    static constexpr bool BIG = V_ == 0;
+    static constexpr int V = CONTIG ? 4 : BIG ? 1 : V_;
     static constexpr int KP = F32Mfma<MF>::KP;
     static constexpr int PITCH = CONTIG ? BK + 4 : X + MF;
     static constexpr int FLOATS = CONTIG ? X * PITCH : BK * PITCH;
@@ -79,17 +84,25 @@ struct F32Slice {
         const int i = threadIdx.x + 256 * p;
         return CONTIG ? i % (BK / V) * V : i / (X / V);
     }
-    // Where a thread's loads of a whole slice start, kept and advanced by the
-    // slice (recomputed, they were as many VALU cycles as a 32 x 32 tile's
-    // MFMAs).  Rows past xn repeat the last: their outputs are not stored.
+    // Where a thread's loads of a whole slice start: a base for the workgroup,
+    // advanced by the slice on the scalar unit, and a 32-bit byte offset per
+    // load (64-bit pointers took as many VALU cycles per slice as a 32 x 32
+    // tile's MFMAs).  BIG: the tile spans 2^32 bytes or more, 64-bit offsets.
+    // Rows past xn repeat the last: their outputs are not stored.
+    using Off = std::conditional_t<BIG, int64_t, uint32_t>;
     struct Src {
-        const float* q[NP];
+        const char* base;
+        Off o[NP];
         __device__ __forceinline__ Src(const float* P, int64_t ld, int x0, int xn, int k0) {
+            base = reinterpret_cast<const char*>(CONTIG ? P + x0 * ld + k0 : P + k0 * ld + x0);
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                const int64_t x = min(x0 + x_of(p), xn - (CONTIG ? 1 : V)), k = k0 + k_of(p);
-                q[p] = CONTIG ? P + x * ld + k : P + k * ld + x;
+                const Off x = (Off)min(x_of(p), xn - x0 - (CONTIG ? 1 : V)), k = (Off)k_of(p);
+                o[p] = (CONTIG ? x * (Off)ld + k : k * (Off)ld + x) * 4;
             }
+        }
+        __device__ __forceinline__ const float* at(int p) const {
+            return reinterpret_cast<const float*>(base + o[p]);
         }
     };
     static __device__ __forceinline__ f32x4_t get4(const float* q) {
@@ -101,35 +114,40 @@ struct F32Slice {
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
                 if constexpr (V == 4) {
-                    const f32x4_t v = get4(s.q[p]);
+                    const f32x4_t v = get4(s.at(p));
 #pragma unroll
                     for (int e = 0; e < 4; ++e) r[4 * p + e] = v[e];
                 } else {
-                    r[p] = *s.q[p];
+                    r[p] = *s.at(p);
                 }
-                s.q[p] += CONTIG ? BK : (int64_t)BK * ld;
             }
+            s.base += 4 * (CONTIG ? (int64_t)BK : BK * ld);
             return;
         }
-        // the last slice: pieces past kn are read from the last k instead, and
+        // the last slice: k past kn are read from the last k instead, and
         // replaced
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const int k = k0 + k_of(p), past = k - (kn - (CONTIG ? V : 1));
-            const float* q = s.q[p] - (past > 0 ? (CONTIG ? past : past * ld) : 0);
-            if constexpr (V == 4) {
-                const f32x4_t v = get4(q);
+            const int k = k0 + k_of(p);
+            if constexpr (CONTIG) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) r[4 * p + e] = v[e];
+                for (int e = 0; e < 4; ++e) {
+                    const float v = *(s.at(p) + (min(k + e, kn - 1) - k));
+                    r[4 * p + e] = k + e < kn ? v : (IS_B ? -0.0f : 0.0f);
+                }
             } else {
-                r[p] = *q;
+                const float* q = s.at(p) + (min(k, kn - 1) - k) * ld;
+                if constexpr (V == 4) {
+                    const f32x4_t v = get4(q);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) r[4 * p + e] = v[e];
+                } else {
+                    r[p] = *q;
+                }
+#pragma unroll
+                for (int e = 0; e < V; ++e) r[V * p + e] = k < kn ? r[V * p + e] : (IS_B ? -0.0f : 0.0f);
             }
         }
-#pragma unroll
-        for (int p = 0; p < NP; ++p)
-#pragma unroll
-            for (int e = 0; e < V; ++e)
-                r[V * p + e] = k0 + k_of(p) < kn ? r[V * p + e] : (IS_B ? -0.0f : 0.0f);
     }
     __device__ __forceinline__ void store(float* s) const {
 #pragma unroll
@@ -187,20 +205,31 @@ struct F32Tile {
 #pragma unroll
             for (int j = 0; j < NT; ++j) acc[i][j] = typename Mf::Acc{};
         if (kb >= ke) return;
-        // slice t + PF is loaded while slice t is multiplied; slice t + 1 goes
-        // to the other LDS buffer after it
+        // While slice t is multiplied, slice t + 1 goes from its registers to
+        // the other LDS buffer (free since the last barrier).  One accumulator:
+        // first of all, then slice t + 1 + PF is loaded into them, and the
+        // operands of four k-steps are read during the MFMAs of the four before.
+        // With more the compiler's own order is the better one (4096^3 at 128 x
+        // 128 1046 against 1374 us): slice t + PF loaded first, slice t + 1
+        // stored last.
+        constexpr bool AHEAD = MT * NT == 1;
         SA ra[PF];
         SB rb[PF];
         typename SA::Src pa(A, lda, m0, M, kb);
         typename SB::Src pb(B, ldb, n0, N, kb);
+        auto load = [&](int u, int k0) {
+            if (k0 >= ke) return;
+            ra[u].load(pa, lda, k0, ke);
+            rb[u].load(pb, ldb, k0, ke);
+        };
+        auto store = [&](int u, int b) {
+            ra[u].store(sm + b * STAGE);
+            rb[u].store(sm + b * STAGE + SA::FLOATS);
+        };
 #pragma unroll
-        for (int u = 0; u < PF; ++u)
-            if (kb + u * BK < ke) {
-                ra[u].load(pa, lda, kb + u * BK, ke);
-                rb[u].load(pb, ldb, kb + u * BK, ke);
-            }
-        ra[0].store(sm);
-        rb[0].store(sm + SA::FLOATS);
+        for (int u = 0; u < PF; ++u) load(u, kb + u * BK);
+        store(0, 0);
+        if constexpr (AHEAD) load(0, kb + PF * BK);
         lds_barrier();
         int buf = 0;
         for (int kt = kb; kt < ke; kt += PF * BK) {
@@ -208,16 +237,9 @@ struct F32Tile {
             for (int u = 0; u < PF; ++u) {
                 const int k0 = kt + u * BK;
                 if (k0 >= ke) break;
-                if (k0 + PF * BK < ke) {
-                    ra[u].load(pa, lda, k0 + PF * BK, ke);
-                    rb[u].load(pb, ldb, k0 + PF * BK, ke);
-                }
                 const float* sa = sm + buf * STAGE;
                 const float* sb = sa + SA::FLOATS;
-                // One accumulator: the operands of four k-steps are read during
-                // the MFMAs of the four before them.  With more the compiler's
-                // own order is the better one (4096^3 1079 against 1374 us).
-                constexpr bool AHEAD = MT * NT == 1;
+                buf ^= 1;
                 constexpr int NG = BK / KP / 4;
                 f32x4_t a[2][MT], b[2][NT];
                 auto read = [&](int g) {
@@ -227,11 +249,18 @@ struct F32Tile {
                     for (int j = 0; j < NT; ++j) b[g & 1][j] = SB::frag(sb, xb + j * MF, ph, g);
                 };
                 if constexpr (AHEAD) read(0);
+                else load(u, k0 + PF * BK);
 #pragma unroll
                 for (int g = 0; g < NG; ++g) {
                     if constexpr (!AHEAD) read(g);
                     else if (g + 1 < NG) read(g + 1);
-                    if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (AHEAD) {
+                        if (g == 0) {
+                            if (k0 + BK < ke) store((u + 1) % PF, buf);
+                            load((u + 1) % PF, k0 + (PF + 1) * BK);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
 #pragma unroll
                     for (int s = 0; s < 4; ++s)
 #pragma unroll
@@ -241,12 +270,8 @@ struct F32Tile {
                                 acc[i][j] = Mf::run(a[g & 1][i][s], b[g & 1][j][s], acc[i][j]);
                     if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
                 }
-                buf ^= 1;
-                if (k0 + BK < ke) {
-                    ra[(u + 1) % PF].store(sm + buf * STAGE);
-                    rb[(u + 1) % PF].store(sm + buf * STAGE + SA::FLOATS);
-                    lds_barrier();
-                }
+                if (!AHEAD && k0 + BK < ke) store((u + 1) % PF, buf);
+                lds_barrier();
             }
         }
     }
