@@ -40,12 +40,15 @@ __device__ __forceinline__ void finish(const F32Gemm& g, Each&& each) {
                             g.C[(int64_t)m * g.ldc + n] = activate<ACT>(v);
                         }));
     } else {
-        each([&](int m, int n, float v, float) { g.C[(int64_t)m * g.ldc + n] = v; });
+        each([&](int m, int n, float v, float) {
+            float* c = g.colsum && m == g.M - 1 ? g.colsum + n : g.C + (int64_t)m * g.ldc + n;
+            *c = v;
+        });
     }
 }
 
 template <class CF, bool TA, bool TB, int V>
-__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Gemm g, int kc, float* __restrict__ part) {
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Gemm g, int kc, int chunk, float* __restrict__ part) {
     using T = F32Tile<CF::MF, CF::MT, CF::NT, CF::BK, CF::PF, TA, TB, V>;
     constexpr bool ACTS = !TA && !TB;
     __shared__ __attribute__((aligned(16))) float sm[2 * T::STAGE];
@@ -61,7 +64,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Gemm g, int kc
         bias[j] = ACTS && g.bias ? g.bias[min(nw + j * CF::MF, g.N - 1)] : 0.0f;
 
     typename T::Mf::Acc acc[CF::MT][CF::NT];
-    T::run(g.A, g.lda, g.B, g.ldb, m0, g.M, n0, g.N, kb, min(g.K, kb + kc), sm, acc);
+    T::run(g.A, g.lda, g.B, g.ldb, m0, g.M - (g.colsum ? 1 : 0), n0, g.N, kb, min(g.K, kb + kc), part ? 0 : chunk,
+           g.colsum != nullptr, sm, acc);
 
     auto each = [&](auto&& f) {
 #pragma unroll
@@ -92,13 +96,13 @@ using F32Cfg3 = F32Cfg<32, 2, 2, 16, 1>;
 using F32Cfg4 = F32Cfg<16, 1, 1, 128, 1>;
 
 template <bool TA, bool TB>
-void launch_f32_tile(int plan, int v, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
+void launch_f32_tile(int plan, int v, const F32Gemm& g, int splits, int kc, int chunk, float* part, hipStream_t s) {
     auto go = [&](auto cfg, auto vec) {
         using CF = decltype(cfg);
         const int64_t wg =
             (((int64_t)g.M + CF::BM - 1) / CF::BM) * (((int64_t)g.N + CF::BN - 1) / CF::BN) * splits;
         hipLaunchKernelGGL((gemm_f32_tile_kernel<CF, TA, TB, decltype(vec)::value>), dim3((unsigned)wg), dim3(256), 0,
-                           s, g, kc, part);
+                           s, g, kc, chunk, part);
     };
     auto pick = [&](auto vec) {
         switch (plan) {
@@ -119,6 +123,6 @@ void launch_f32_tile(int plan, int v, const F32Gemm& g, int splits, int kc, floa
 }
 
 // gemm_f32_tile_t.hip: at least one of ta, tb
-void launch_f32_tile_trans(int plan, int v, const F32Gemm& g, int splits, int kc, float* part, hipStream_t s);
+void launch_f32_tile_trans(int plan, int v, const F32Gemm& g, int splits, int kc, int chunk, float* part, hipStream_t s);
 
 }  // namespace jh

@@ -36,7 +36,7 @@ constexpr F32Plan kF32Plans[4] = {{32, 32, 0.0053f, 0.0062f, 1.0f},
                                   {64, 128, 0.034f, 0.042f, 1.4f},
                                   {128, 128, 0.065f, 0.075f, 3.0f}};
 
-int f32_plan(int M, int N, int kc, int splits) {
+int f32_plan(int M, int N, int kc, int splits, float* us_out) {
     int best = 0;
     float best_us = 0.0f;
     for (int c = 0; c < 4; ++c) {
@@ -49,6 +49,7 @@ int f32_plan(int M, int N, int kc, int splits) {
             best = c;
         }
     }
+    *us_out = best_us;
     // 32 x 32 tiles alone on their CUs: half as many barriers for a long chain
     // (64 x 512 x 2048 17.7 -> 15.9 us); with neighbours the larger LDS costs more
     if (best == 0 && kc >= 256 && ((int64_t)M + 31) / 32 * (((int64_t)N + 31) / 32) * splits <= 256) best = 4;
@@ -59,10 +60,28 @@ int f32_plan(int M, int N, int kc, int splits) {
 
 hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
     if (g.M == 0 || g.N == 0) return hipSuccess;
+    int chunk = 0, plan;
+    float us, fold_us = 0.0f;
+    if (splits > 1) {
+        // The same sums in the same order in one launch, 32 x 32 tiles that fold
+        // a range at a time, unless spreading the ranges over workgroups pays
+        // for its reduction (64 x 256 x 784 in 10 ranges 17.4 -> 6 us).
+        plan = f32_plan(g.M, g.N, kc, splits, &us);
+        us += 4.5f + 0.1f * splits + 1.2e-6f * splits * g.M * g.N;
+        const int64_t wg = ((int64_t)g.M + 31) / 32 * (((int64_t)g.N + 31) / 32);
+        const float n = (float)((wg + 255) / 256);
+        fold_us = n > 1.0f ? n * (g.K * kF32Plans[0].per_k + kF32Plans[0].round)
+                           : g.K * kF32Plans[0].alone + kF32Plans[0].round;
+        if (!part || fold_us < us) {
+            chunk = kc;
+            splits = 1;
+            plan = wg <= 256 && g.K >= 256 ? 4 : 0;
+        }
+    }
     if (splits <= 1) {
-        splits = 1;
         kc = g.K;
         part = nullptr;
+        if (!chunk) plan = f32_plan(g.M, g.N, kc, 1, &us);
     }
     // whole 16-byte pieces of the operands whose k is the outer dimension; 32-bit
     // offsets within a tile (128 rows, or the rows there are, or a slice's 64)
@@ -70,10 +89,9 @@ hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hi
         return (int64_t)std::min(rows, rows_are_k ? 64 : 128) * ld * 4 >= (int64_t(1) << 32);
     };
     const bool big = spans(g.ta, g.ta ? g.K : g.M, g.lda) || spans(!g.tb, g.tb ? g.N : g.K, g.ldb);
-    const int v = big ? 0 : (!g.ta || g.M % 4 == 0) && (g.tb || g.N % 4 == 0) ? 4 : 1;
-    const int plan = f32_plan(g.M, g.N, kc, splits);
-    if (g.ta || g.tb) launch_f32_tile_trans(plan, v, g, splits, kc, part, s);
-    else launch_f32_tile<false, false>(plan, v, g, splits, kc, part, s);
+    const int v = big ? 0 : (!g.ta || (g.M - (g.colsum ? 1 : 0)) % 4 == 0) && (g.tb || g.N % 4 == 0) ? 4 : 1;
+    if (g.ta || g.tb) launch_f32_tile_trans(plan, v, g, splits, kc, chunk, part, s);
+    else launch_f32_tile<false, false>(plan, v, g, splits, kc, chunk, part, s);
     if (part) {
         int64_t b = ((int64_t)g.M * g.N + 255) / 256;
         if (b > 2048) b = 2048;

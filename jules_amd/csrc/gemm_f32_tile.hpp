@@ -94,10 +94,11 @@ struct F32Slice {
         const char* base;
         Off o[NP];
         __device__ __forceinline__ Src(const float* P, int64_t ld, int x0, int xn, int k0) {
-            base = reinterpret_cast<const char*>(CONTIG ? P + x0 * ld + k0 : P + k0 * ld + x0);
+            const int last = xn - (CONTIG ? 1 : V), xb = min(x0, last);
+            base = reinterpret_cast<const char*>(CONTIG ? P + xb * ld + k0 : P + k0 * ld + xb);
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                const Off x = (Off)min(x_of(p), xn - x0 - (CONTIG ? 1 : V)), k = (Off)k_of(p);
+                const Off x = (Off)(min(x0 + x_of(p), last) - xb), k = (Off)k_of(p);
                 o[p] = (CONTIG ? x * (Off)ld + k : k * (Off)ld + x) * 4;
             }
         }
@@ -149,6 +150,13 @@ struct F32Slice {
             }
         }
     }
+    // row x of the slice = 1
+    __device__ __forceinline__ void fill_row(int x) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int e = 0; e < V; ++e) r[V * p + e] = x_of(p) + (CONTIG ? 0 : e) == x ? 1.0f : r[V * p + e];
+    }
     __device__ __forceinline__ void store(float* s) const {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
@@ -194,10 +202,14 @@ struct F32Tile {
     using SB = F32Slice<MF, BN, BK, TB, V, true>;
     static constexpr int STAGE = SA::FLOATS + SB::FLOATS;
 
-    // acc = the tile at (m0, n0) over k in [kb, ke)
+    // acc = the tile at (m0, n0) over k in [kb, ke).  chunk > 0 (a multiple of
+    // 16; one accumulator a wave only): the sum is taken over chunks of that
+    // many k, each its own chain, added in order, as a K split into ranges of
+    // chunk would add its partial sums.  ones: row M of op(A) reads as 1, so
+    // output row M is the column sum of op(B) (TA only).
     static __device__ __forceinline__ void run(const float* A, int64_t lda, const float* B, int64_t ldb, int m0,
-                                               int M, int n0, int N, int kb, int ke, float* sm,
-                                               typename Mf::Acc (&acc)[MT][NT]) {
+                                               int M, int n0, int N, int kb, int ke, int chunk, bool ones,
+                                               float* sm, typename Mf::Acc (&acc)[MT][NT]) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         const int xa = (wave >> 1) * MT * MF + lane % MF, xb = (wave & 1) * NT * MF + lane % MF, ph = lane / MF;
 #pragma unroll
@@ -221,6 +233,8 @@ struct F32Tile {
             if (k0 >= ke) return;
             ra[u].load(pa, lda, k0, ke);
             rb[u].load(pb, ldb, k0, ke);
+            if constexpr (TA)
+                if (ones) ra[u].fill_row(M - m0);
         };
         auto store = [&](int u, int b) {
             ra[u].store(sm + b * STAGE);
@@ -231,7 +245,15 @@ struct F32Tile {
         store(0, 0);
         if constexpr (AHEAD) load(0, kb + PF * BK);
         lds_barrier();
-        int buf = 0;
+        int buf = 0, left = chunk;
+        bool first = true;
+        typename Mf::Acc tot[MT][NT];
+        auto fold = [&]() {
+            tot[0][0] = first ? acc[0][0] : tot[0][0] + acc[0][0];
+            acc[0][0] = typename Mf::Acc{};
+            first = false;
+            left = chunk;
+        };
         for (int kt = kb; kt < ke; kt += PF * BK) {
 #pragma unroll
             for (int u = 0; u < PF; ++u) {
@@ -268,12 +290,20 @@ struct F32Tile {
 #pragma unroll
                             for (int j = 0; j < NT; ++j)
                                 acc[i][j] = Mf::run(a[g & 1][i][s], b[g & 1][j][s], acc[i][j]);
-                    if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (AHEAD) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (chunk && k0 + 4 * KP * g < ke && (left -= 4 * KP) == 0) fold();
+                    }
                 }
                 if (!AHEAD && k0 + BK < ke) store((u + 1) % PF, buf);
                 lds_barrier();
             }
         }
+        if constexpr (AHEAD)
+            if (chunk) {
+                if (left != chunk) fold();
+                acc[0][0] = tot[0][0];
+            }
     }
 };
 

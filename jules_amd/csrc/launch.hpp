@@ -15,7 +15,8 @@ hipError_t launch_gemm_f32(int act, const float* A, const float* B, const float*
 // fp32 GEMM on the MFMA tiles (gemm_f32_tile.hip): C = epilogue(op(A) op(B)),
 // row-major, op(X) = X^T when ta / tb.  Each output is one fma chain over k =
 // 0 .. K-1 in order unless K is split: `splits` ranges of kc (a multiple of
-// 64), whose sums go to part[splits][M][N] and are added in order.
+// 16), summed apart and added in order, through part[splits][M][N] if that is
+// given and faster.
 enum F32Epi {
     F32_EPI_ACT = 0,     // act(sum [+ bias[n]])
     F32_EPI_MASK,        // mask[m][n] > 0 ? sum : 0
@@ -35,6 +36,10 @@ struct F32Gemm {
     const float* mask;
     int64_t ldm;
     float alpha, beta;
+    // not null (ta, F32_EPI_ACT without bias or activation, K not split): M is
+    // one more than op(A) has rows, and colsum[n] gets the sum of column n of
+    // op(B), added in row order
+    float* colsum;
 };
 hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s);
 // the fp32 GEMM entry point's validation and launch with a chosen table

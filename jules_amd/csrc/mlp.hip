@@ -21,14 +21,7 @@
 // which computes the same formula.  db1/db2 are column sums in a fixed order
 // (row chunks, then the chunks in order), so every result is deterministic.
 //
-// GEMM: C[M,N] = op(A)[M,K] op(B)[K,N] with v_mfma_f32_32x32x2_f32.  A 128x128
-// output tile per 256-thread workgroup (4 waves, 64x64 each = 2x2 MFMA
-// blocks), K in slices of 16 staged through LDS ([k][m] and [k][n], padded
-// rows), the next slice's global loads in registers while the current one is
-// multiplied, one barrier per slice.  op(A) = A^T and op(B) = B^T only change
-// which dimension the global loads run along; the LDS layout is the same.
-// Out-of-range elements are loaded as 0 (any summation order is allowed
-// here: the reference's products are BLAS calls).
+// The products run on the fp32 MFMA tiles of gemm_f32_tile.hip.
 #include <algorithm>
 #include <type_traits>
 
@@ -37,180 +30,6 @@
 
 namespace jh {
 namespace {
-
-typedef float f32x16_mfma_t __attribute__((ext_vector_type(16)));
-
-constexpr int BM = 128, BN = 128, BK = 16;
-constexpr int GT = 256;              // threads per GEMM workgroup
-constexpr int LDA_S = BM + 1;        // LDS row pitch (floats)
-constexpr int LDB_S = BN + 1;
-constexpr int PA = BM * BK / GT;     // A elements per thread per slice (8)
-constexpr int PB = BK * BN / GT;
-
-// BLAS sgemm epilogue: alpha * acc + beta * C, with C not read when
-// beta = 0 (so NaNs in an uninitialised C never propagate), and acc itself
-// when alpha = 1 and beta = 0
-__device__ __forceinline__ float alpha_beta(float acc, float alpha, float beta, const float* c) {
-    const float v = alpha * acc;
-    return beta == 0.0f ? v : v + beta * *c;
-}
-
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(GT, 2) void gemm_f32_mfma_kernel(
-    const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb,
-    float* __restrict__ C, int ldc, int M, int N, int K, const float* __restrict__ bias,
-    const float* __restrict__ mask, int ldm, int kc, float* __restrict__ part, float alpha,
-    float beta) {
-    __shared__ float As[2][BK * LDA_S];
-    __shared__ float Bs[2][BK * LDB_S];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;  // 64x64 quadrant of the tile
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    // this workgroup's K range (split-K: blockIdx.z of gridDim.z)
-    const int kb = blockIdx.z * kc, ke = min(K, kb + kc);
-
-    float ra[PA], rb[PB];
-    // element e of a slice: along the dimension contiguous in memory
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int p = 0; p < PA; ++p) {
-            const int e = tid + p * GT;
-            const int m = TA ? (e & (BM - 1)) : (e >> 4);
-            const int k = TA ? (e >> 7) : (e & (BK - 1));
-            const int gm = m0 + m, gk = k0 + k;
-            const bool ok = gm < M && gk < ke;
-            const int64_t off = TA ? (int64_t)gk * lda + gm : (int64_t)gm * lda + gk;
-            const float v = A[ok ? off : 0];  // branch-free: element 0, then dropped
-            ra[p] = ok ? v : 0.0f;
-        }
-#pragma unroll
-        for (int p = 0; p < PB; ++p) {
-            const int e = tid + p * GT;
-            const int n = TB ? (e >> 4) : (e & (BN - 1));
-            const int k = TB ? (e & (BK - 1)) : (e >> 7);
-            const int gn = n0 + n, gk = k0 + k;
-            const bool ok = gn < N && gk < ke;
-            const int64_t off = TB ? (int64_t)gn * ldb + gk : (int64_t)gk * ldb + gn;
-            const float v = B[ok ? off : 0];
-            rb[p] = ok ? v : 0.0f;
-        }
-    };
-    auto sstore = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < PA; ++p) {
-            const int e = tid + p * GT;
-            const int m = TA ? (e & (BM - 1)) : (e >> 4);
-            const int k = TA ? (e >> 7) : (e & (BK - 1));
-            As[buf][k * LDA_S + m] = ra[p];
-        }
-#pragma unroll
-        for (int p = 0; p < PB; ++p) {
-            const int e = tid + p * GT;
-            const int n = TB ? (e >> 4) : (e & (BN - 1));
-            const int k = TB ? (e & (BK - 1)) : (e >> 7);
-            Bs[buf][k * LDB_S + n] = rb[p];
-        }
-    };
-
-    f32x16_mfma_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    const int nk = (ke - kb + BK - 1) / BK;
-    gload(kb);
-    sstore(0);
-    __syncthreads();
-    const int lr = lane & 31, lk = lane >> 5;  // MFMA operand: row/col lr, k lk
-    for (int kt = 0; kt < nk; ++kt) {
-        const int buf = kt & 1;
-        if (kt + 1 < nk) gload(kb + (kt + 1) * BK);
-        const float* as = As[buf];
-        const float* bs = Bs[buf];
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 2) {
-            float a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = as[(kk + lk) * LDA_S + wm * 64 + i * 32 + lr];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) b[j] = bs[(kk + lk) * LDB_S + wn * 64 + j * 32 + lr];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (kt + 1 < nk) sstore(buf ^ 1);
-        __syncthreads();
-    }
-
-    // 32x32 accumulator layout: register r of lane l holds row
-    // 8*(r/4) + 4*(l/32) + r%4, column l%32
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + wn * 64 + j * 32 + lr;
-            if (n >= N) continue;
-            if (part) {  // split-K: raw partial sums, epilogue in the reduction
-                float* pz = part + (int64_t)blockIdx.z * M * N;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
-                    if (m < M) pz[(int64_t)m * N + n] = acc[i][j][r];
-                }
-                continue;
-            }
-            float bn = 0.0f;
-            if constexpr (EPI == 1 || EPI == 2) bn = bias[n];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
-                if (m >= M) continue;
-                float v = acc[i][j][r];
-                if constexpr (EPI == 1) {
-                    v = v + bn;
-                } else if constexpr (EPI == 2) {
-                    v = v + bn;
-                    v = v > 0.0f ? v : 0.0f;
-                } else if constexpr (EPI == 3) {
-                    v = mask[(int64_t)m * ldm + n] > 0.0f ? v : 0.0f;
-                } else if constexpr (EPI == 4) {
-                    v = alpha_beta(v, alpha, beta, C + (int64_t)m * ldc + n);
-                }
-                C[(int64_t)m * ldc + n] = v;
-            }
-        }
-}
-
-// Split-K reduction: C = epilogue(sum over z of part[z], in z order).
-template <int EPI>
-__global__ void splitk_reduce_kernel(const float* __restrict__ part, int S, int M, int N,
-                                     float* __restrict__ C, int ldc, const float* __restrict__ bias,
-                                     const float* __restrict__ mask, int ldm, float alpha,
-                                     float beta) {
-    const int64_t total = (int64_t)M * N, stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += stride) {
-        const int m = (int)(e / N), n = (int)(e - (int64_t)m * N);
-        float v = part[e];
-        for (int z = 1; z < S; ++z) v += part[(int64_t)z * total + e];
-        if constexpr (EPI == 1) {
-            v = v + bias[n];
-        } else if constexpr (EPI == 2) {
-            v = v + bias[n];
-            v = v > 0.0f ? v : 0.0f;
-        } else if constexpr (EPI == 3) {
-            v = mask[(int64_t)m * ldm + n] > 0.0f ? v : 0.0f;
-        } else if constexpr (EPI == 4) {
-            v = alpha_beta(v, alpha, beta, C + (int64_t)m * ldc + n);
-        }
-        C[(int64_t)m * ldc + n] = v;
-    }
-}
 
 // C = beta * C (alpha * op(A) op(B) vanishes: K = 0 or alpha = 0); beta = 0
 // writes zeros without reading C, as BLAS does
@@ -259,14 +78,15 @@ __global__ void fill_kernel(float* __restrict__ p, int64_t n, float v) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
 }
 
-enum { EPI_NONE = 0, EPI_BIAS = 1, EPI_BIAS_RELU = 2, EPI_MASK = 3, EPI_ALPHA_BETA = 4 };
-
-// Split-K plan: a GEMM with fewer than 128 output tiles gets its K range
-// split (at least 4 slices per split) so that about 256 workgroups run; the
-// partial sums go to the workspace and a reduction applies the epilogue.
+// K ranges of a product, each summed by itself: one with fewer than 128 output
+// tiles of 128 x 128 sums K in as many ranges (of at least 64) as would make
+// about 256 of them.  They say in which order the products are summed; whether
+// a range gets workgroups of its own is launch_f32_gemm's choice, and the
+// workspace holds their partial sums in case it does.
+constexpr int BM = 128, BN = 128, BK = 16;
 struct KPlan {
-    int S;   // splits
-    int kc;  // K elements per split, a multiple of BK
+    int S;   // ranges
+    int kc;  // K elements per range, a multiple of BK
 };
 
 KPlan kplan(int M, int N, int K) {
@@ -285,21 +105,13 @@ size_t kplan_floats(int M, int N, int K) {
     return p.S > 1 ? (size_t)p.S * M * N : 0;
 }
 
-template <bool TA, bool TB, int EPI>
-hipError_t gemm(const float* A, int lda, const float* B, int ldb, float* C, int ldc, int M, int N,
-                int K, const float* bias, const float* mask, int ldm, float* part, hipStream_t s,
-                float alpha = 1.0f, float beta = 0.0f) {
-    const KPlan p = kplan(M, N, K);
-    const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM, p.S);
-    hipLaunchKernelGGL((gemm_f32_mfma_kernel<TA, TB, EPI>), grid, dim3(GT), 0, s, A, lda, B, ldb, C,
-                       ldc, M, N, K, bias, mask, ldm, p.kc, p.S > 1 ? part : nullptr, alpha, beta);
-    if (p.S > 1) {
-        int64_t b = ((int64_t)M * N + 255) / 256;
-        if (b > 2048) b = 2048;
-        hipLaunchKernelGGL(splitk_reduce_kernel<EPI>, dim3((unsigned)b), dim3(256), 0, s, part, p.S,
-                           M, N, C, ldc, bias, mask, ldm, alpha, beta);
-    }
-    return hipGetLastError();
+hipError_t gemm(F32Gemm g, float* part, hipStream_t s) {
+    const KPlan p = kplan(g.M, g.N, g.K);
+    return launch_f32_gemm(g, p.S, p.kc, part, s);
+}
+// X W + bias, with or without ReLU
+F32Gemm layer(const float* X, const float* W, const float* bias, int act, float* Y, int M, int N, int K) {
+    return {false, false, X, K, W, N, Y, N, M, N, K, F32_EPI_ACT, act, bias, nullptr, 0, 1.0f, 0.0f, nullptr};
 }
 
 constexpr int COLSUM_ROWS = 256;  // rows per partial column sum
@@ -313,12 +125,22 @@ int colsum_chunks(int M, int* rows) {
     return S;
 }
 
-hipError_t colsum(const float* X, int M, int N, float* part, float* out, hipStream_t s) {
+// dW = A^T G and db = colsum(G), A [M,Ka], G [M,N].  Up to COLSUM_ROWS rows the
+// column sum is an extra row of ones in A^T, summed as the product is (a chain
+// over the rows, or over each range of them); more rows are summed in chunks by
+// kernels of their own.
+hipError_t weight_grad(const float* A, int Ka, const float* G, int M, int N, float* dW, float* db,
+                       float* colsum_part, float* part, hipStream_t s) {
+    const bool fold = M <= COLSUM_ROWS;
+    F32Gemm g = {true, false, A, Ka, G, N, dW, N, Ka + fold, N, M, F32_EPI_ACT, JH_ACT_NONE, nullptr, nullptr, 0,
+                 1.0f, 0.0f, fold ? db : nullptr};
+    const KPlan p = kplan(Ka, N, M);
+    const hipError_t e = launch_f32_gemm(g, p.S, p.kc, fold ? nullptr : part, s);
+    if (fold || e != hipSuccess) return e;
     int R;
     const int S = colsum_chunks(M, &R);
-    hipLaunchKernelGGL(colsum_partial_kernel, dim3((N + 255) / 256, S), dim3(256), 0, s, X, M, N, N,
-                       R, part);
-    hipLaunchKernelGGL(colsum_final_kernel, dim3((N + 255) / 256), dim3(256), 0, s, part, S, N, out);
+    hipLaunchKernelGGL(colsum_partial_kernel, dim3((N + 255) / 256, S), dim3(256), 0, s, G, M, N, N, R, colsum_part);
+    hipLaunchKernelGGL(colsum_final_kernel, dim3((N + 255) / 256), dim3(256), 0, s, colsum_part, S, N, db);
     return hipGetLastError();
 }
 
@@ -368,10 +190,9 @@ hipError_t launch_mlp_forward(const float* X, const float* W1, const float* b1, 
     float* act = static_cast<float*>(ws);
     float* kpart = reinterpret_cast<float*>(static_cast<char*>(ws) +
                                             align256((size_t)M * N1 * sizeof(float)));
-    hipError_t e;
-    if ((e = gemm<false, false, EPI_BIAS_RELU>(X, K1, W1, N1, act, N1, M, N1, K1, b1, nullptr, 0, kpart, s)))
-        return e;
-    return gemm<false, false, EPI_BIAS>(act, N1, W2, N2, output, N2, M, N2, N1, b2, nullptr, 0, kpart, s);
+    const hipError_t e = gemm(layer(X, W1, b1, JH_ACT_RELU, act, M, N1, K1), kpart, s);
+    if (e != hipSuccess) return e;
+    return gemm(layer(act, W2, b2, JH_ACT_NONE, output, M, N2, N1), kpart, s);
 }
 
 hipError_t launch_mlp_forward_backward(const float* X, const float* W1, const float* b1,
@@ -404,26 +225,22 @@ hipError_t launch_mlp_forward_backward(const float* X, const float* W1, const fl
 
     hipError_t e;
     // forward
-    if ((e = gemm<false, false, EPI_BIAS_RELU>(X, K1, W1, N1, act, N1, M, N1, K1, b1, nullptr, 0, kpart, s)))
-        return e;
-    if ((e = gemm<false, false, EPI_BIAS>(act, N1, W2, N2, output, N2, M, N2, N1, b2, nullptr, 0, kpart, s)))
-        return e;
+    if ((e = gemm(layer(X, W1, b1, JH_ACT_RELU, act, M, N1, K1), kpart, s))) return e;
+    if ((e = gemm(layer(act, W2, b2, JH_ACT_NONE, output, M, N2, N1), kpart, s))) return e;
     // loss and dO
     if ((e = launch_cross_entropy(output, targets, dO, loss, row_loss, M, N2, s))) return e;
     // layer 2 gradients
-    if ((e = gemm<true, false, EPI_NONE>(act, N1, dO, N2, dW2, N2, N1, N2, M, nullptr, nullptr, 0, kpart, s)))
-        return e;
-    if ((e = colsum(dO, M, N2, part, db2, s))) return e;
+    if ((e = weight_grad(act, N1, dO, M, N2, dW2, db2, part, kpart, s))) return e;
     // dH = (dO W2^T) * (a > 0)
-    if ((e = gemm<false, true, EPI_MASK>(dO, N2, W2, N2, dH, N1, M, N1, N2, nullptr, act, N1, kpart, s)))
-        return e;
+    const F32Gemm dh = {false, true, dO, N2, W2, N2, dH, N1, M, N1, N2, F32_EPI_MASK, JH_ACT_NONE, nullptr, act, N1,
+                        1.0f, 0.0f, nullptr};
+    if ((e = gemm(dh, kpart, s))) return e;
     // layer 1 gradients
-    if ((e = gemm<true, false, EPI_NONE>(X, K1, dH, N1, dW1, N1, K1, N1, M, nullptr, nullptr, 0, kpart, s)))
-        return e;
-    if ((e = colsum(dH, M, N1, part, db1, s))) return e;
-    if (dX && (e = gemm<false, true, EPI_NONE>(dH, N1, W1, N1, dX, K1, M, K1, N1, nullptr, nullptr, 0, kpart, s)))
-        return e;
-    return hipSuccess;
+    if ((e = weight_grad(X, K1, dH, M, N1, dW1, db1, part, kpart, s))) return e;
+    if (!dX) return hipSuccess;
+    const F32Gemm dx = {false, true, dH, N1, W1, N1, dX, K1, M, K1, N1, F32_EPI_ACT, JH_ACT_NONE, nullptr, nullptr, 0,
+                        1.0f, 0.0f, nullptr};
+    return gemm(dx, kpart, s);
 }
 
 // blasMatmul / cblas_sgemm (reference FusedKernels.h:633-644): the MFMA GEMM
@@ -448,14 +265,9 @@ hipError_t launch_sgemm(bool transA, bool transB, int M, int N, int K, float alp
         if (e != hipSuccess) return e;
         part = static_cast<float*>(ws);
     }
-    auto run = [&](auto ta, auto tb) {
-        return gemm<decltype(ta)::value, decltype(tb)::value, EPI_ALPHA_BETA>(
-            A, lda, B, ldb, C, ldc, M, N, K, nullptr, nullptr, 0, part, s, alpha, beta);
-    };
-    using F = std::false_type;
-    using T = std::true_type;
-    if (transA) return transB ? run(T{}, T{}) : run(T{}, F{});
-    return transB ? run(F{}, T{}) : run(F{}, F{});
+    return gemm({transA, transB, A, lda, B, ldb, C, ldc, M, N, K, F32_EPI_ALPHA_BETA, JH_ACT_NONE, nullptr, nullptr, 0,
+                 alpha, beta, nullptr},
+                part, s);
 }
 
 }  // namespace jh
