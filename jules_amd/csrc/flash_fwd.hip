@@ -257,11 +257,14 @@ __device__ __forceinline__ float pair_sum(float v) {
     return a + b;
 }
 
-template <int D, bool CAUSAL>
+// PAD: rows of dr < D elements, a multiple of 8 (dr is not used otherwise).
+// Columns dr .. D - 1 of Q, K and V are zeros made on the way in: Q's in
+// registers, K's and V's by range-checked copies whose offset lies outside.
+template <int D, bool CAUSAL, bool PAD>
 __device__ __forceinline__ void flash_bf16_body(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, uint16_t* __restrict__ O, float* __restrict__ lse, int BH, int S,
-    float c_log2) {
+    float c_log2, int dr) {
     using C = Bf16Cfg<D>;
     constexpr int BKV = C::BKV;
     constexpr float kLazy = 8.0f;
@@ -277,7 +280,8 @@ __device__ __forceinline__ void flash_bf16_body(
     const int nq = (S + BQ2 - 1) / BQ2;
     int bh, q0;
     block_coords(BH, nq, BQ2, &bh, &q0);
-    const int64_t hoff = (int64_t)bh * S * D;
+    const int ld = PAD ? dr : D;  // elements per row in memory
+    const int64_t hoff = (int64_t)bh * S * ld;
     const uint16_t* Qh = Q + hoff;
     const uint16_t* Kh = K + hoff;
     const uint16_t* Vh = V + hoff;
@@ -295,7 +299,7 @@ __device__ __forceinline__ void flash_bf16_body(
         const int qr = min(qrow, S - 1);  // rows past S compute on a valid row, never stored
 #pragma unroll
         for (int ks = 0; ks < C::KS; ++ks)
-            qv[ks] = global_b128_untracked(Qh + (int64_t)qr * D + ks * 16 + 8 * g);
+            qv[ks] = global_b128_untracked(Qh + (int64_t)qr * ld + (PAD && ks * 16 + 8 * g >= ld ? 0 : ks * 16 + 8 * g));
     }
 
     const int kv_end = CAUSAL ? min(S, q0 + BQ2) : S;
@@ -314,7 +318,14 @@ __device__ __forceinline__ void flash_bf16_body(
             const int up = lane % C::UNITS;                // physical 16-byte unit
             const int64_t key = min(t * BKV + r, S - 1);   // rows past S read a valid row
             uint8_t* dst = sm + (t % C::NSTAGE) * C::STAGE + seg * 1024;
-            if (p < C::SEGW)
+            if constexpr (PAD) {
+                const bool k = p < C::SEGW;
+                const int u = up ^ (k ? kswz<D>(r) : vswz<D>(r) >> 1);
+                const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+                    const_cast<uint16_t*>(k ? Kh : Vh), 0, (uint32_t)S * (uint32_t)ld * 2u, 0x00020000);
+                const uint32_t off = 8 * u < ld ? ((uint32_t)key * (uint32_t)ld + 8u * u) * 2u : 0x80000000u;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void*)(k ? dst : dst + C::TILE), 16, off, 0, 0, 0);
+            } else if (p < C::SEGW)
                 __builtin_amdgcn_global_load_lds(Kh + key * D + 8 * (up ^ kswz<D>(r)),
                                                  (lds_void*)dst, 16, 0, 0);
             else
@@ -481,6 +492,7 @@ __device__ __forceinline__ void flash_bf16_body(
 #pragma unroll
     for (int ks = 0; ks < C::KS; ++ks) {
         reg_fence(qv[ks]);  // after the wait above
+        if (PAD && ks * 16 + 8 * g >= ld) qv[ks] = u32x4_t{0u, 0u, 0u, 0u};
         qf[ks] = __builtin_bit_cast(bf16x8_t, qv[ks]);
     }
 
@@ -590,7 +602,8 @@ __device__ __forceinline__ void flash_bf16_body(
     for (int s = 0; s < U / 2; ++s) {
         const int r = s * RPI + lane / U, u = lane % U;
         const u32x4_t v = *reinterpret_cast<const u32x4_t*>(stg + r * (D * 2) + ((u ^ (r & (U - 1))) << 4));
-        if (qw0 + r < S) *reinterpret_cast<u32x4_t*>(O + hoff + (int64_t)(qw0 + r) * D + 8 * u) = v;
+        if (qw0 + r < S && (!PAD || 8 * u < ld))
+            *reinterpret_cast<u32x4_t*>(O + hoff + (int64_t)(qw0 + r) * ld + 8 * u) = v;
     }
 }
 
@@ -601,7 +614,14 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_bf16(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, uint16_t* __restrict__ O, float* __restrict__ lse, int BH, int S,
     float c_log2) {
-    flash_bf16_body<D, CAUSAL>(Q, K, V, O, lse, BH, S, c_log2);
+    flash_bf16_body<D, CAUSAL, false>(Q, K, V, O, lse, BH, S, c_log2, D);
+}
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(512, 1) void flash_fwd_bf16_pad(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
+    const uint16_t* __restrict__ V, uint16_t* __restrict__ O, float* __restrict__ lse, int BH, int S,
+    float c_log2, int dr) {
+    flash_bf16_body<D, CAUSAL, true>(Q, K, V, O, lse, BH, S, c_log2, dr);
 }
 
 // ---------------------------------------------------------------------------
@@ -837,6 +857,24 @@ hipError_t go(KFN kfn, const void* Q, const void* K, const void* V, void* O, flo
 }
 
 }  // namespace
+
+bool flash_fwd_takes_rows(int dtype, int S, int D) {
+    return dtype == JH_BF16 && D % 8 == 0 && D < 128 && (int64_t)S * D * 2 < (int64_t(1) << 31);
+}
+
+hipError_t launch_flash_fwd_rows(int causal, float scale, const void* Q, const void* K, const void* V, void* O,
+                                 float* lse, int B, int H, int S, int D, hipStream_t s) {
+    const int BH = B * H, nq = (S + BQ2 - 1) / BQ2;
+    if ((int64_t)BH * nq > 2147483647) return hipErrorInvalidValue;
+    const auto run = [&](auto kfn) {
+        hipLaunchKernelGGL(kfn, dim3(BH * nq), dim3(NW2 * 64), 0, s, static_cast<const uint16_t*>(Q),
+                           static_cast<const uint16_t*>(K), static_cast<const uint16_t*>(V),
+                           static_cast<uint16_t*>(O), lse, BH, S, scale * kLog2e, D);
+        return hipGetLastError();
+    };
+    if (D <= 64) return causal ? run(&flash_fwd_bf16_pad<64, true>) : run(&flash_fwd_bf16_pad<64, false>);
+    return causal ? run(&flash_fwd_bf16_pad<128, true>) : run(&flash_fwd_bf16_pad<128, false>);
+}
 
 hipError_t launch_flash_fwd(int dtype, int causal, float scale, const void* Q, const void* K,
                             const void* V, void* O, float* lse, int B, int H, int S, int D,

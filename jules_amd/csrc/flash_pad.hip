@@ -4,7 +4,8 @@
 //
 // The reference's flashAttention (include/jules/Kernel/FlashAttention.h:
 // 130-309) accepts any head_dim.  The MFMA kernels here are built for 64 and
-// 128; other sizes are zero-padded to the next of the two.  Zero columns
+// 128; other sizes are zero-padded to the next of the two, by the bf16 forward
+// itself where rows are whole 16-byte pieces, else through the workspace.  Zero columns
 // change neither the scores Q K^T, nor the log-sum-exp, nor the real columns
 // of O (padded V columns only produce padded O columns), nor, in the
 // backward, the real columns of dQ, dK and dV (rowsum(dO * O) is unchanged;
@@ -49,43 +50,45 @@ hipError_t stream_workspace(size_t need, hipStream_t s, void** ws, WorkspaceLock
 
 namespace {
 
-// dst[r][c] = c < D ? src[r][c] : 0 over [rows][Dp]
-template <typename T>
-__global__ void pad_rows_kernel(T* __restrict__ dst, const T* __restrict__ src, int64_t rows, int D,
-                                int Dp) {
+// Up to 8 tensors, one per blockIdx.y, moved in pieces of T: 16 bytes where a
+// row of D elements is whole pieces, else one element.
+struct RowsArgs {
+    void* dst[8];
+    const void* src[8];
+};
+// dst[r][c] = c < n ? src[r][c] : 0 over [rows][1 << sh] (PAD), or
+// dst[r][c] = src[r][c] for c < n, src rows 1 << sh wide
+template <typename T, bool PAD>
+__global__ void move_rows_kernel(RowsArgs a, int64_t rows, int n, int sh) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * Dp) return;
-    const int64_t r = i / Dp;
-    const int c = (int)(i % Dp);
-    dst[i] = c < D ? src[r * D + c] : T(0);
-}
-// dst[r][c] = src[r][c] for c < D, over [rows][D]
-template <typename T>
-__global__ void unpad_rows_kernel(T* __restrict__ dst, const T* __restrict__ src, int64_t rows, int D,
-                                  int Dp) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * D) return;
-    const int64_t r = i / D;
-    const int c = (int)(i % D);
-    dst[i] = src[r * Dp + c];
+    const int64_t r = i >> sh;
+    const int c = (int)(i & ((1 << sh) - 1));
+    if (r >= rows || (!PAD && c >= n)) return;
+    T* d = static_cast<T*>(a.dst[blockIdx.y]);
+    const T* s = static_cast<const T*>(a.src[blockIdx.y]);
+    if (PAD) d[i] = c < n ? s[r * n + c] : T{};
+    else d[r * n + c] = s[i];
 }
 
 inline size_t a256(size_t n) { return (n + 255) & ~size_t(255); }
 
-// element size: fp32 moved as uint32_t, bf16 as uint16_t
-template <typename T>
-hipError_t pad(void* dst, const void* src, int64_t rows, int D, int Dp, hipStream_t s) {
-    const int64_t n = rows * Dp;
-    hipLaunchKernelGGL(pad_rows_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                       static_cast<T*>(dst), static_cast<const T*>(src), rows, D, Dp);
-    return hipGetLastError();
-}
-template <typename T>
-hipError_t unpad(void* dst, const void* src, int64_t rows, int D, int Dp, hipStream_t s) {
-    const int64_t n = rows * D;
-    hipLaunchKernelGGL(unpad_rows_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                       static_cast<T*>(dst), static_cast<const T*>(src), rows, D, Dp);
-    return hipGetLastError();
+// `count` tensors of `rows` rows, D elements of es bytes wide, into (PAD) or
+// out of rows of Dp elements; one launch (a launch per tensor of 2-byte pieces
+// took 4.2 us each at 2 x 16 x 333 x 80)
+template <bool PAD>
+hipError_t move_rows(const RowsArgs& a, int count, int64_t rows, int D, int Dp, size_t es, hipStream_t s) {
+    auto go = [&](auto piece) {
+        using T = decltype(piece);
+        const int per = (int)(sizeof(T) / es), n = D / per;
+        int sh = 0;
+        while ((1 << sh) < Dp / per) ++sh;
+        const int64_t total = rows << sh;
+        hipLaunchKernelGGL((move_rows_kernel<T, PAD>), dim3((unsigned)((total + 255) / 256), (unsigned)count),
+                           dim3(256), 0, s, a, rows, n, sh);
+        return hipGetLastError();
+    };
+    if (D * es % 16 == 0) return go(u32x4_t{});
+    return es == 2 ? go(uint16_t{}) : go(uint32_t{});
 }
 
 }  // namespace
@@ -95,6 +98,12 @@ int flash_padded_dim(int D) { return D <= 64 ? 64 : 128; }
 hipError_t launch_flash_fwd_padded(int dtype, int causal, float scale, const void* Q, const void* K,
                                    const void* V, void* O, float* lse, int B, int H, int S, int D,
                                    hipStream_t s) {
+    // the workspace holds copies of K and V, so there O may lie over them
+    const char *o = static_cast<const char*>(O), *k = static_cast<const char*>(K), *v = static_cast<const char*>(V);
+    const int64_t bytes = (int64_t)B * H * S * D * 2;
+    const bool apart = (o + bytes <= k || k + bytes <= o) && (o + bytes <= v || v + bytes <= o);
+    if (apart && flash_fwd_takes_rows(dtype, S, D))
+        return launch_flash_fwd_rows(causal, scale, Q, K, V, O, lse, B, H, S, D, s);
     const int Dp = flash_padded_dim(D);
     const int64_t rows = (int64_t)B * H * S;
     const size_t es = dtype == JH_BF16 ? 2 : 4;
@@ -104,13 +113,10 @@ hipError_t launch_flash_fwd_padded(int dtype, int causal, float scale, const voi
     hipError_t e = stream_workspace(4 * one, s, &ws, &lock);
     if (e != hipSuccess) return e;
     char* w = static_cast<char*>(ws);
-    void *Qp = w, *Kp = w + one, *Vp = w + 2 * one, *Op = w + 3 * one;
-    auto padf = dtype == JH_BF16 ? pad<uint16_t> : pad<uint32_t>;
-    if ((e = padf(Qp, Q, rows, D, Dp, s)) || (e = padf(Kp, K, rows, D, Dp, s)) ||
-        (e = padf(Vp, V, rows, D, Dp, s)))
+    if ((e = move_rows<true>({{w, w + one, w + 2 * one}, {Q, K, V}}, 3, rows, D, Dp, es, s))) return e;
+    if ((e = launch_flash_fwd(dtype, causal, scale, w, w + one, w + 2 * one, w + 3 * one, lse, B, H, S, Dp, s)))
         return e;
-    if ((e = launch_flash_fwd(dtype, causal, scale, Qp, Kp, Vp, Op, lse, B, H, S, Dp, s))) return e;
-    return dtype == JH_BF16 ? unpad<uint16_t>(O, Op, rows, D, Dp, s) : unpad<uint32_t>(O, Op, rows, D, Dp, s);
+    return move_rows<false>({{O}, {w + 3 * one}}, 1, rows, D, Dp, es, s);
 }
 
 hipError_t launch_flash_bwd_padded(int dtype, int causal, float scale, const void* Q, const void* K,
@@ -125,21 +131,13 @@ hipError_t launch_flash_bwd_padded(int dtype, int causal, float scale, const voi
     WorkspaceLock lock;
     hipError_t e = stream_workspace(8 * one, s, &ws, &lock);
     if (e != hipSuccess) return e;
-    char* w = static_cast<char*>(ws);
-    void* p[8];
-    for (int i = 0; i < 8; ++i) p[i] = w + i * one;  // Q K V O dO dQ dK dV
-    auto padf = dtype == JH_BF16 ? pad<uint16_t> : pad<uint32_t>;
-    auto unpadf = dtype == JH_BF16 ? unpad<uint16_t> : unpad<uint32_t>;
-    const void* src[5] = {Q, K, V, O, dO};
-    for (int i = 0; i < 5; ++i)
-        if ((e = padf(p[i], src[i], rows, D, Dp, s))) return e;
+    char* p[8];
+    for (int i = 0; i < 8; ++i) p[i] = static_cast<char*>(ws) + i * one;  // Q K V O dO dQ dK dV
+    if ((e = move_rows<true>({{p[0], p[1], p[2], p[3], p[4]}, {Q, K, V, O, dO}}, 5, rows, D, Dp, es, s))) return e;
     if ((e = launch_flash_bwd(dtype, causal, scale, p[0], p[1], p[2], p[3], p[4], lse, p[5], p[6], p[7],
                               B, H, S, Dp, bwd_ws, s)))
         return e;
-    if ((e = unpadf(dQ, p[5], rows, D, Dp, s)) || (e = unpadf(dK, p[6], rows, D, Dp, s)) ||
-        (e = unpadf(dV, p[7], rows, D, Dp, s)))
-        return e;
-    return hipSuccess;
+    return move_rows<false>({{dQ, dK, dV}, {p[5], p[6], p[7]}}, 3, rows, D, Dp, es, s);
 }
 
 }  // namespace jh

@@ -142,7 +142,12 @@ hipError_t launch_hbm_read(const void* buf, int64_t bytes, uint32_t* out, int wo
                            hipStream_t s);
 
 
-// flash attention at head dims other than 64 and 128 (1 <= D <= 128): inputs
+// bf16 forward at a head dim the kernels read as it is (D < 128, a multiple of
+// 8, heads below 2^31 bytes), its columns up to 64 or 128 zeros on the way in
+bool flash_fwd_takes_rows(int dtype, int S, int D);
+hipError_t launch_flash_fwd_rows(int causal, float scale, const void* Q, const void* K, const void* V, void* O,
+                                 float* lse, int B, int H, int S, int D, hipStream_t s);
+// flash attention at other head dims than 64 and 128 (1 <= D <= 128): inputs
 // zero-padded to 64 or 128 in the per-stream workspace (flash_pad.hip)
 int flash_padded_dim(int D);
 hipError_t launch_flash_fwd_padded(int dtype, int causal, float scale, const void* Q, const void* K,
