@@ -16,9 +16,10 @@
 // All three are HBM-bound, and the row is held in registers so it is read
 // from HBM once and written once: one wave per row for N <= 4096 (four rows
 // per workgroup), one 1024-thread workgroup per row for N <= 65536 (up to 64
-// elements per thread).  With N % 4 == 0 and 16-byte aligned rows each
-// thread moves 16-byte pieces, otherwise single floats; either way every wave
-// instruction covers contiguous bytes.  Rows longer than 65536 get a
+// elements per thread).  Each thread moves 16-byte pieces of the row's whole
+// 16-float vectors, wherever the row starts, and the last N % 16 elements are
+// one float each of the first threads; rows up to 128 are moved as single
+// floats.  Every wave instruction covers contiguous bytes.  Rows longer than 65536 get a
 // 1024-thread workgroup that keeps the row's first 65536 elements on chip
 // (registers and LDS) and streams the rest in chunks of 16 elements per
 // thread, in the reference's own three passes (softmax and cross entropy:
@@ -80,9 +81,11 @@ __device__ __forceinline__ float row_norm(float e, float inv, float sum, int j, 
 
 // ---- a row held in the registers of a group of G threads (one wave, or
 // the BT threads of a block).  Thread `tid` holds ELEMS elements: with VEC,
-// 16-byte pieces f = tid + G*t, elements 4f .. 4f+3 (rows 16-byte aligned,
-// N % 4 == 0); without, elements j = tid + G*t.  Every load or store
-// instruction of a wave covers contiguous bytes.
+// 16-byte pieces f = tid + G*t, elements 4f .. 4f+3, of the row's first nv = N
+// & ~15 elements (at any 4-byte address: rows of 50257 floats moved one by one
+// took 222 us for 2048 of them, 183 us as pieces); without, elements j = tid +
+// G*t of the row.  Every load or store instruction of a wave covers contiguous
+// bytes.
 // The BT-thread rows use range-checked buffer accesses over the row (N * 4
 // bytes, N <= 65536): a store past the row's end is dropped without a
 // branch, and at 64 elements per thread the kernels fit in 128 registers.
@@ -95,6 +98,11 @@ struct RowRegs {
     static constexpr int NA = ELEMS / W;    // accesses per thread
     static constexpr bool BUF = G != 64;
     using Access = std::conditional_t<VEC, f32x4_t, float>;
+    struct __attribute__((packed, aligned(4))) Any {  // an Access at any 4-byte address
+        Access v;
+    };
+    // the part of a row of N that load, store and each cover
+    __device__ __forceinline__ static int part(int N) { return VEC ? N & ~15 : N; }
     float v[ELEMS];
     __device__ __forceinline__ static int elem(int tid, int a, int i) {
         return VEC ? 4 * (tid + G * a) + i : tid + G * a;
@@ -123,7 +131,7 @@ struct RowRegs {
             else
                 return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, o, 0, 0));
         } else {
-            return *reinterpret_cast<const Access*>(reinterpret_cast<const char*>(p) + o);
+            return reinterpret_cast<const Any*>(reinterpret_cast<const char*>(p) + o)->v;
         }
     }
     // one access stored at byte offset o; nothing if o is past the row
@@ -135,7 +143,7 @@ struct RowRegs {
             else
                 __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, q), dst, o, 0, 0);
         } else if (o < (uint32_t)N * 4u) {
-            *reinterpret_cast<Access*>(reinterpret_cast<char*>(p) + o) = q;
+            reinterpret_cast<Any*>(reinterpret_cast<char*>(p) + o)->v = q;
         }
     }
     // v[] = x[]; past the row's end, with LAST the row's last element (piece,
@@ -147,7 +155,7 @@ struct RowRegs {
     __device__ __forceinline__ void load(const float* x, int N, int tid) {
         const __amdgpu_buffer_rsrc_t src = row_rsrc(x, N);
         const uint32_t o0 = base_off(tid);
-        const uint32_t last = (uint32_t)(N - W) * 4u;  // N >= W: with VEC, N % 4 == 0
+        const uint32_t last = (uint32_t)(N - W) * 4u;  // N >= W: VEC rows have N > 128
 #pragma unroll
         for (int a = 0; a < NA; ++a) {
             const uint32_t o = o0 + 4u * (uint32_t)first(a);
@@ -187,42 +195,32 @@ struct RowRegs {
                 f(j, v[W * a + i], j < N);
             }
     }
-    // The row's tail [nv, N) (N % 16 elements; none when nv == N).  A thread
-    // holds at most one access inside it: the tail has fewer than 16
-    // elements and the group at least 64 threads (with VEC, nv % 16 == 0 and
-    // N % 4 == 0, so a piece is wholly in or out).
+    // The row's tail [nv, N): N % 16 elements, at most one a thread.  With VEC
+    // element nv + tid of the first threads, loaded on its own; without, the
+    // element u in [nv, N) with u % G == tid, which v[] holds.
     static constexpr uint32_t TAIL_NONE = 0x80000000u;  // past any row: no store
-    // byte offset of this thread's tail access, or TAIL_NONE: the one element
-    // (piece) u in [nv, N) (pieces [nv/4, N/4)) with u % G == tid
+    // byte offset of this thread's tail element, or TAIL_NONE
     __device__ __forceinline__ static uint32_t tail_off(int N, int nv, int tid) {
-        const int u0 = nv / W, u1 = N / W;
-        const int u = u0 + ((tid - u0) & (G - 1));
-        return u < u1 ? (uint32_t)u * (uint32_t)(4 * W) : TAIL_NONE;
+        const int u = VEC ? nv + tid : nv + ((tid - nv) & (G - 1));
+        return u < N ? (uint32_t)u * 4u : TAIL_NONE;
     }
-    // values of that access (0 without one)
-    __device__ __forceinline__ void tail(int N, int nv, int tid, float (&xt)[W]) const {
+    // its value (0 without one)
+    __device__ __forceinline__ float tail(const float* x, int N, int nv, int tid) const {
+        if constexpr (VEC) {
+            return tid < N - nv ? x[nv + tid] : 0.0f;
+        } else {
+            float xt = 0.0f;
 #pragma unroll
-        for (int i = 0; i < W; ++i) xt[i] = 0.0f;
-#pragma unroll
-        for (int a = 0; a < NA; ++a) {
-            const int j0 = elem(tid, a, 0);
-            const bool t = j0 >= nv && j0 < N;
-#pragma unroll
-            for (int i = 0; i < W; ++i) xt[i] = t ? v[W * a + i] : xt[i];
+            for (int a = 0; a < NA; ++a) {
+                const int j = elem(tid, a, 0);
+                xt = j >= nv && j < N ? v[a] : xt;
+            }
+            return xt;
         }
     }
     // y at byte offset off = q, one float, the same kind of access as store()
     __device__ __forceinline__ static void store1(float* y, int N, uint32_t off, float q) {
         RowRegs<G, 1, false>::store_at(y, row_rsrc(y, N), N, off, q);
-    }
-    // this thread's tail access, stored after store() (nothing for TAIL_NONE)
-    __device__ __forceinline__ static void store_tail(float* y, int N, uint32_t toff, const float (&q)[W]) {
-        Access w;
-        if constexpr (VEC)
-            w = f32x4_t{q[0], q[1], q[2], q[3]};
-        else
-            w = q[0];
-        store_at(y, row_rsrc(y, N), N, toff, w);
     }
 };
 
@@ -273,27 +271,26 @@ __device__ __forceinline__ float group_sum(float v, float* red) {
 // Leaves e = fast_exp(x - max) in R.v for the part of the row that fills
 // whole 16-float vectors (j < nv = N & ~15) and 0 elsewhere; the tail
 // [nv, N), where the reference takes expf and divides by the sum instead of
-// multiplying by its reciprocal, is this thread's et[] (its access there:
+// multiplying by its reciprocal, is this thread's *et (its element there:
 // RowRegs::tail_off), to be stored after R.  Each thread sums its own
-// elements, then its tail ones.  FULL: N % 16 == 0, no tail (a kernel of
+// elements, then its tail one.  FULL: N % 16 == 0, no tail (a kernel of
 // its own, which carries neither the tail's extraction nor its expf).
 template <bool FULL, int G, int ELEMS, bool VEC>
 __device__ __forceinline__ void softmax_held(RowRegs<G, ELEMS, VEC>& R, const float* x, int N,
                                              int tid, float* red, float* mx_out, float* s_out,
-                                             float (&et)[VEC ? 4 : 1]) {
+                                             float* et) {
     using RR = RowRegs<G, ELEMS, VEC>;
     const int nv = N & ~15;
-    R.template load<true>(x, N, tid);
+    const bool has_tail = !FULL && RR::tail_off(N, nv, tid) != RR::TAIL_NONE;
+    float xt = 0.0f;
+    if constexpr (!FULL && VEC) xt = R.tail(x, N, nv, tid);  // in flight with the row
+    R.template load<true>(x, RR::part(N), tid);
     float mx = -FLT_MAX;
 #pragma unroll
     for (int k = 0; k < ELEMS; ++k) mx = ref_max(mx, R.v[k]);
+    if constexpr (!FULL && VEC) mx = has_tail ? ref_max(mx, xt) : mx;
     mx = group_max<G>(mx, red);
-    if constexpr (FULL) {
-#pragma unroll
-        for (int i = 0; i < RR::W; ++i) et[i] = 0.0f;
-    } else {
-        R.tail(N, nv, tid, et);
-    }
+    if constexpr (!FULL && !VEC) xt = R.tail(x, N, nv, tid);
     // fast_exp clamps its argument to [-88, 88], so it is finite for every
     // element, pads included, and the select needs no branch
     float s = 0.0f;
@@ -306,13 +303,10 @@ __device__ __forceinline__ void softmax_held(RowRegs<G, ELEMS, VEC>& R, const fl
             e = RR::elem(tid, a, i) < nv ? f : 0.0f;
             s += e;
         }
+    *et = 0.0f;
     if constexpr (!FULL) {
-        const bool has_tail = RR::tail_off(N, nv, tid) != RR::TAIL_NONE;
-#pragma unroll
-        for (int i = 0; i < RR::W; ++i) {
-            et[i] = expf(et[i] - mx);
-            s += has_tail ? et[i] : 0.0f;
-        }
+        *et = expf(xt - mx);
+        s += has_tail ? *et : 0.0f;
     }
     *mx_out = mx;
     *s_out = group_sum<G>(s, red);
@@ -338,16 +332,13 @@ __global__ __launch_bounds__(G == 64 ? 64 * ROWS_PER_BLOCK : BT) void softmax_ke
     const int row = held_row<G>(&tid);
     if (row >= M) return;  // whole wave (G = 64) or whole block
     RowRegs<G, ELEMS, VEC> R;
-    float mx, s, pt[VEC ? 4 : 1];
-    softmax_held<FULL>(R, in + (int64_t)row * N, N, tid, red, &mx, &s, pt);
+    float mx, s, pt;
+    softmax_held<FULL>(R, in + (int64_t)row * N, N, tid, red, &mx, &s, &pt);
     const float inv = 1.0f / s;
     float* y = out + (int64_t)row * N;
-    R.store(y, N, tid, [&](float e) { return e * inv; });
-    if constexpr (!FULL) {
-#pragma unroll
-        for (int i = 0; i < (VEC ? 4 : 1); ++i) pt[i] = pt[i] / s;
-        R.store_tail(y, N, R.tail_off(N, N & ~15, tid), pt);  // after R's store of 0 there
-    }
+    R.store(y, R.part(N), tid, [&](float e) { return e * inv; });
+    // after R's store of 0 there (without VEC)
+    if constexpr (!FULL) R.store1(y, N, R.tail_off(N, N & ~15, tid), pt / s);
 }
 
 // ---- rows longer than a block holds: one BT-thread workgroup per row, the
@@ -563,27 +554,33 @@ __global__ __launch_bounds__(G == 64 ? 64 * ROWS_PER_BLOCK : BT) void layernorm_
     const int row = held_row<G>(&tid);
     if (row >= M) return;
     RowRegs<G, ELEMS, VEC> R;
-    R.template load<false>(in + (int64_t)row * N, N, tid);
+    using RR = RowRegs<G, ELEMS, VEC>;
+    const int nv = N & ~15, np = RR::part(N);
+    const bool has_tail = VEC && tid < N - nv;  // without VEC, R covers the whole row
+    const float* x = in + (int64_t)row * N;
+    const float xt = has_tail ? x[nv + tid] : 0.0f;
+    R.template load<false>(x, np, tid);
     float s = 0.0f;
 #pragma unroll
     for (int k = 0; k < ELEMS; ++k) s += R.v[k];
+    s += xt;
     const float mean = group_sum<G>(s, red) / (float)N;
     float q = 0.0f;
-    R.each(N, tid, [&](int, float& x, bool in) {
-        const float d = x - mean;
+    R.each(np, tid, [&](int, float& e, bool in) {
+        const float d = e - mean;
         q = in ? __builtin_fmaf(d, d, q) : q;
     });
+    q = has_tail ? __builtin_fmaf(xt - mean, xt - mean, q) : q;
     const float var = group_sum<G>(q, red) / (float)N;
     const float inv_std = 1.0f / sqrtf(var + eps);
-    using RR = RowRegs<G, ELEMS, VEC>;
     float* y = out + (int64_t)row * N;
-    const __amdgpu_buffer_rsrc_t gs = RR::row_rsrc(gamma, N), bs = RR::row_rsrc(beta, N),
-                                 ys = RR::row_rsrc(y, N);
+    const __amdgpu_buffer_rsrc_t gs = RR::row_rsrc(gamma, np), bs = RR::row_rsrc(beta, np),
+                                 ys = RR::row_rsrc(y, np);
     const uint32_t o0 = RR::fresh_base_off(tid);
-    const uint32_t last = (uint32_t)(N - RR::W) * 4u;
+    const uint32_t last = (uint32_t)(np - RR::W) * 4u;
 #pragma unroll
     for (int a = 0; a < RR::NA; ++a) {
-        if (RR::first(a) >= N) continue;  // the same for the whole group
+        if (RR::first(a) >= np) continue;  // the same for the whole group
         const uint32_t o = o0 + 4u * (uint32_t)RR::first(a), oc = o < last ? o : last;
         const typename RR::Access gq = RR::load_at(gamma, gs, oc), bq = RR::load_at(beta, bs, oc);
         typename RR::Access q;
@@ -593,8 +590,9 @@ __global__ __launch_bounds__(G == 64 ? 64 * ROWS_PER_BLOCK : BT) void layernorm_
         } else {
             q = __builtin_fmaf((R.v[a] - mean) * inv_std, gq, bq);
         }
-        RR::store_at(y, ys, N, o, q);  // nothing past the row
+        RR::store_at(y, ys, np, o, q);  // nothing past the row's part
     }
+    if (has_tail) y[nv + tid] = __builtin_fmaf((xt - mean) * inv_std, gamma[nv + tid], beta[nv + tid]);
 }
 
 // rows longer than a block holds: the reference's three passes (sum, sum of
@@ -671,31 +669,29 @@ __global__ __launch_bounds__(G == 64 ? 64 * ROWS_PER_BLOCK : BT) void cross_entr
     // the thread whose elements include t stores its gradient; x[t] is read
     // (by every thread, a scalar load) before any store of this row (grad may
     // alias logits)
-    const bool owner = valid && tid == (VEC ? (t >> 2) % G : t % G);
+    const int nv = N & ~15;
+    const bool owner = valid && tid == (!VEC ? t % G : t < nv ? (t >> 2) % G : t - nv);
     const float xt = valid ? x[t] : 0.0f;
     RowRegs<G, ELEMS, VEC> R;
-    float mx, s, ptl[VEC ? 4 : 1];
-    softmax_held<FULL>(R, x, N, tid, red, &mx, &s, ptl);
-    const int nv = N & ~15;
+    float mx, s, ptl;
+    softmax_held<FULL>(R, x, N, tid, red, &mx, &s, &ptl);
     const float inv = 1.0f / s;
     const float pt = row_norm(row_exp(xt - mx, t, nv), inv, s, t, nv);
     const float fm = (float)M;
-#pragma unroll
-    for (int i = 0; i < (VEC ? 4 : 1); ++i) ptl[i] = ptl[i] / s;
+    ptl = ptl / s;
     // grad = p / M as the reference's division; for a power-of-two M the
     // product with 1/M (exact) is the same single rounding of p * 2^-k, bit
     // for bit, at a tenth of the instructions
     if ((M & (M - 1)) == 0) {
         const float rm = 1.0f / fm;
-        R.store(g, N, tid, [&](float e) { return (e * inv) * rm; });
-#pragma unroll
-        for (int i = 0; i < (VEC ? 4 : 1); ++i) ptl[i] = ptl[i] * rm;
+        R.store(g, R.part(N), tid, [&](float e) { return (e * inv) * rm; });
+        ptl = ptl * rm;
     } else {
-        R.store(g, N, tid, [&](float e) { return (e * inv) / fm; });
-#pragma unroll
-        for (int i = 0; i < (VEC ? 4 : 1); ++i) ptl[i] = ptl[i] / fm;
+        R.store(g, R.part(N), tid, [&](float e) { return (e * inv) / fm; });
+        ptl = ptl / fm;
     }
-    if constexpr (!FULL) R.store_tail(g, N, R.tail_off(N, nv, tid), ptl);  // after R's store of 0 there
+    // after R's store of 0 there (without VEC)
+    if constexpr (!FULL) R.store1(g, N, R.tail_off(N, nv, tid), ptl);
     if (owner) {
         // after this thread's own stores of g[t], through the same buffer path
         R.store1(g, N, (uint32_t)t * 4u, (pt - 1.0f) / fm);
@@ -940,40 +936,32 @@ __global__ __launch_bounds__(RT) void cross_entropy_reduce_kernel(const float* _
 
 // Launch plan for a row length: the smallest register-held size that fits
 // (one wave per row up to MAX_CACHED, one BT-thread block per row up to
-// MAX_BLOCK_CACHED), 16-byte accesses when every row is 16-byte aligned, the
-// no-tail softmax when N % 16 == 0.  f(G, ELEMS, VEC, FULL) returns the
-// launch status; rows past MAX_BLOCK_CACHED are left to the caller
-// (streaming kernels).
+// MAX_BLOCK_CACHED), single floats up to 128, the no-tail softmax when N % 16
+// == 0.  f(G, ELEMS, VEC, FULL) returns the launch status; rows past
+// MAX_BLOCK_CACHED are left to the caller (streaming kernels).
 template <int G, int E, typename F>
-hipError_t with_flags(bool vec, bool full, F&& f) {
+hipError_t with_flags(bool full, F&& f) {
     using std::integral_constant;
     using g = integral_constant<int, G>;
     using e = integral_constant<int, E>;
-    if constexpr (E < 4) {
-        return full ? f(g{}, e{}, integral_constant<bool, false>{}, integral_constant<bool, true>{})
-                    : f(g{}, e{}, integral_constant<bool, false>{}, integral_constant<bool, false>{});
-    } else {
-        if (vec)
-            return full ? f(g{}, e{}, integral_constant<bool, true>{}, integral_constant<bool, true>{})
-                        : f(g{}, e{}, integral_constant<bool, true>{}, integral_constant<bool, false>{});
-        return full ? f(g{}, e{}, integral_constant<bool, false>{}, integral_constant<bool, true>{})
-                    : f(g{}, e{}, integral_constant<bool, false>{}, integral_constant<bool, false>{});
-    }
+    using v = integral_constant<bool, (E >= 4)>;
+    return full ? f(g{}, e{}, v{}, integral_constant<bool, true>{})
+                : f(g{}, e{}, v{}, integral_constant<bool, false>{});
 }
 template <typename F>
-hipError_t by_size(int N, bool vec, F&& f) {
+hipError_t by_size(int N, F&& f) {
     const bool full = N % 16 == 0;
-    if (N <= 64) return with_flags<64, 1>(vec, full, f);
-    if (N <= 128) return with_flags<64, 2>(vec, full, f);
-    if (N <= 256) return with_flags<64, 4>(vec, full, f);
-    if (N <= 512) return with_flags<64, 8>(vec, full, f);
-    if (N <= 1024) return with_flags<64, 16>(vec, full, f);
-    if (N <= 2048) return with_flags<64, 32>(vec, full, f);
-    if (N <= MAX_CACHED) return with_flags<64, 64>(vec, full, f);
-    if (N <= 8192) return with_flags<BT, 8>(vec, full, f);
-    if (N <= 16384) return with_flags<BT, 16>(vec, full, f);
-    if (N <= 32768) return with_flags<BT, 32>(vec, full, f);
-    return with_flags<BT, MAX_BLOCK_CACHED / BT>(vec, full, f);
+    if (N <= 64) return with_flags<64, 1>(full, f);
+    if (N <= 128) return with_flags<64, 2>(full, f);
+    if (N <= 256) return with_flags<64, 4>(full, f);
+    if (N <= 512) return with_flags<64, 8>(full, f);
+    if (N <= 1024) return with_flags<64, 16>(full, f);
+    if (N <= 2048) return with_flags<64, 32>(full, f);
+    if (N <= MAX_CACHED) return with_flags<64, 64>(full, f);
+    if (N <= 8192) return with_flags<BT, 8>(full, f);
+    if (N <= 16384) return with_flags<BT, 16>(full, f);
+    if (N <= 32768) return with_flags<BT, 32>(full, f);
+    return with_flags<BT, MAX_BLOCK_CACHED / BT>(full, f);
 }
 
 bool rows_vec4(int N, std::initializer_list<const void*> ptrs) {
@@ -1054,7 +1042,7 @@ hipError_t launch_softmax(float* out, const float* in, int M, int N, hipStream_t
             hipLaunchKernelGGL(softmax_long_kernel<false>, dim3(M), dim3(BT), HEAD_LDS, s, out, in, N);
         return hipGetLastError();
     }
-    return by_size(N, rows_vec4(N, {out, in}), [&](auto g, auto e, auto v, auto f) {
+    return by_size(N, [&](auto g, auto e, auto v, auto f) {
         constexpr int G = decltype(g)::value;
         hipLaunchKernelGGL((softmax_kernel<G, decltype(e)::value, decltype(v)::value, decltype(f)::value>),
                            dim3(row_blocks<G>(M)), dim3(G == 64 ? 64 * ROWS_PER_BLOCK : BT), 0, s,
@@ -1086,7 +1074,7 @@ hipError_t launch_layernorm(float* out, const float* in, const float* gamma, con
                                beta, N, eps);
         return hipGetLastError();
     }
-    return by_size(N, rows_vec4(N, {out, in, gamma, beta}), [&](auto g, auto e, auto v, auto) {
+    return by_size(N, [&](auto g, auto e, auto v, auto) {
         constexpr int G = decltype(g)::value;
         hipLaunchKernelGGL((layernorm_kernel<G, decltype(e)::value, decltype(v)::value, false>),
                            dim3(row_blocks<G>(M)), dim3(G == 64 ? 64 * ROWS_PER_BLOCK : BT), 0, s,
@@ -1121,7 +1109,7 @@ hipError_t launch_cross_entropy(const float* logits, const int32_t* targets, flo
                                    targets, grad, row_loss, M, N);
             e = hipGetLastError();
         } else {
-            e = by_size(N, rows_vec4(N, {logits, grad}), [&](auto g, auto el, auto v, auto f) {
+            e = by_size(N, [&](auto g, auto el, auto v, auto f) {
                 constexpr int G = decltype(g)::value;
                 hipLaunchKernelGGL((cross_entropy_kernel<G, decltype(el)::value, decltype(v)::value,
                                                          decltype(f)::value>),

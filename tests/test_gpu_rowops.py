@@ -279,3 +279,29 @@ def test_registry_row_kernels(dev):
     l64, g64 = po.cross_entropy64(x, np.arange(12, dtype=np.int32) * 5)
     assert abs(float(to_np(loss)[0]) - l64) < 1e-5 * max(1, abs(l64))
     assert I.rel_err(to_np(y), g64) < I.TOL["f32"]
+
+
+@pytest.mark.parametrize("M,N", [(5, 129), (7, 1023), (3, 4095), (3, 4097), (2, 16385), (2, 50257), (2, 65535)])
+def test_rows_at_any_address(dev, M, N):
+    """Rows that start between 16-byte addresses, and end with their
+    allocation's last element, give the bits of aligned ones."""
+    case(f"rows {M}x{N} misaligned")
+    x = torch.randn((M, N), device=dev)
+    t = torch.randint(0, N, (M,), device=dev, dtype=torch.int32)
+    t[0] = N - 1  # a target in the row's last N % 16 elements
+    g, b = torch.rand((N,), device=dev), torch.rand((N,), device=dev)
+
+    def off(v, k):
+        buf = torch.empty((v.numel() + k,), device=dev)
+        buf[k:] = v.reshape(-1)
+        return buf[k:].view(v.shape)
+
+    xm = off(x, 1)
+    assert torch.equal(ops.softmax(xm, out=off(x, 3)), ops.softmax(x))
+    assert torch.equal(ops.layernorm(xm, off(g, 2), off(b, 1), out=off(x, 3)), ops.layernorm(x, g, b))
+    (l0, g0), (l1, g1) = ops.cross_entropy(x, t), ops.cross_entropy(xm, t, grad=off(x, 3))
+    assert torch.equal(l0, l1) and torch.equal(g0, g1)
+    # in place, and against plain fp64
+    ref = torch.softmax(x.double(), 1)
+    y = ops.softmax(xm, out=xm)
+    assert ((y.double() - ref).abs().max() / ref.max()).item() < 2e-5
