@@ -626,10 +626,15 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_bf16_pad(
 
 // ---------------------------------------------------------------------------
 // fp32: same recurrence on v_mfma_f32_32x32x2_f32.  The 32x32x2 A/B operands
-// are one fp32 per lane (row/col = lane & 31, k = lane >> 5), so K and V are
-// read from LDS as [key][d] rows without any transpose: for the PV product
-// k-step (j, i) pairs keys 8j+i (lanes 0-31) and 8j+4+i (lanes 32-63), which
-// are exactly the score accumulator element 4j+i each lane already holds.
+// are one fp32 per lane (row/col = lane & 31, k = lane >> 5), and which k an
+// MFMA pairs is free as long as A and B agree, so K and V are read from LDS as
+// [key][d] rows without any transpose, 16 (or 8) bytes at a time: in QK^T MFMA
+// 4 i + e pairs columns 8 i + e and 8 i + 4 + e; in PV step (j, i) pairs keys
+// 8j+i (lanes 0-31) and 8j+4+i (lanes 32-63), which are exactly the score
+// accumulator element 4j+i each lane already holds, and a lane's D / 32
+// neighbouring columns of the key's row feed the D / 32 accumulators.
+// Against one 4-byte read per MFMA, a rescale of the accumulator on every tile
+// and an unpadded merge: [4,8,1024,64] causal 63.0 -> 55.0 us.
 //
 // Work split: a workgroup owns 32 queries, and its 4 waves split the key
 // range (wave w takes key tiles w, w+4, ...), each with its own running
@@ -659,8 +664,12 @@ __device__ __forceinline__ void flash_f32_body(
     float* __restrict__ O, float* __restrict__ lse, int BH, int S, float c_log2) {
     using C = F32Cfg<D>;
     constexpr int BKV = C::BKV;
+    constexpr int DT = D / 32;
+    typedef float VRow __attribute__((ext_vector_type(DT)));
     // K/V stages during the loop; the merge reuses the same memory
-    constexpr int MERGE_FLOATS = NWF * (BQF * D + 2 * BQF);
+    constexpr int MROW = D + 4;                        // padded row of a partial accumulator
+    constexpr int MSTATE = BQF * MROW + 2 * BQF;       // a wave's accumulator, then m[q], l[q]
+    constexpr int MERGE_FLOATS = NWF * MSTATE;
     constexpr int SMEM_FLOATS = NWF * C::WAVE_FLOATS > MERGE_FLOATS ? NWF * C::WAVE_FLOATS
                                                                        : MERGE_FLOATS;
     __shared__ __attribute__((aligned(16))) float smem[SMEM_FLOATS];
@@ -676,9 +685,14 @@ __device__ __forceinline__ void flash_f32_body(
     const float* Vh = V + hoff;
     const int qrow = q0 + col;
 
-    float qf[D / 2];  // Q[qrow][2 ks + g]
+    // Q[qrow][8 i + 4 g + 0..3]: MFMA 4 i + e pairs columns 8 i + e (lanes 0-31)
+    // and 8 i + 4 + e (lanes 32-63), so Q and K come as 16-byte reads
+    f32x4_t qf[D / 8];
+    {
+        const float* qp = Qh + (int64_t)min(qrow, S - 1) * D + 4 * g;  // rows past S are never stored
 #pragma unroll
-    for (int ks = 0; ks < D / 2; ++ks) qf[ks] = (qrow < S) ? Qh[(int64_t)qrow * D + 2 * ks + g] : 0.0f;
+        for (int i = 0; i < D / 8; ++i) qf[i] = *reinterpret_cast<const f32x4_t*>(qp + 8 * i);
+    }
 
     const int kv_end = CAUSAL ? min(S, q0 + BQF) : S;
     const int n_kv = (kv_end + BKV - 1) / BKV;
@@ -723,10 +737,13 @@ __device__ __forceinline__ void flash_f32_body(
 #pragma unroll
         for (int e = 0; e < 16; ++e) s[e] = s1[e] = 0.0f;
 #pragma unroll
-        for (int ks = 0; ks < D / 2; ks += 2) {
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(Ks[col * C::ROWF + 2 * ks + g], qf[ks], s, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(Ks[col * C::ROWF + 2 * ks + 2 + g], qf[ks + 1],
-                                                      s1, 0, 0, 0);
+        for (int i = 0; i < D / 8; ++i) {
+            const f32x4_t kf = *reinterpret_cast<const f32x4_t*>(Ks + col * C::ROWF + 8 * i + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[i][e], s, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e + 1], qf[i][e + 1], s1, 0, 0, 0);
+            }
         }
         s += s1;
         const bool need_mask = (k0 + BKV > S) || (CAUSAL && k0 + BKV - 1 > q0);
@@ -744,6 +761,7 @@ __device__ __forceinline__ void flash_f32_body(
         const float m_new = fmaxf(m_run, mx * c_log2);
         const float m_use = (m_new == kNegInf) ? 0.0f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        const bool moved = __builtin_amdgcn_ballot_w64(m_new != m_run) != 0;  // else alpha is 1 in every lane
         m_run = m_new;
         float ls = 0.0f;
 #pragma unroll
@@ -753,19 +771,23 @@ __device__ __forceinline__ void flash_f32_body(
             ls += p;
         }
         l_run = __builtin_fmaf(l_run, alpha, ls);
+        if (moved) {
 #pragma unroll
-        for (int i = 0; i < D / 32; ++i)
+            for (int i = 0; i < D / 32; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc_o[i][e] *= alpha;
+                for (int e = 0; e < 16; ++e) acc_o[i][e] *= alpha;
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
+                // columns DT col .. DT col + DT - 1 of the key's V row: row r of
+                // accumulator dt is column DT r + dt of O
                 const int key = 8 * j + 4 * g + i;
+                const VRow vf = *reinterpret_cast<const VRow*>(Vs + key * C::ROWF + DT * col);
 #pragma unroll
-                for (int dt = 0; dt < D / 32; ++dt)
-                    acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[key * C::ROWF + dt * 32 + col],
-                                                                     s[4 * j + i], acc_o[dt], 0, 0, 0);
+                for (int dt = 0; dt < DT; ++dt)
+                    acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[dt], s[4 * j + i], acc_o[dt], 0, 0, 0);
             }
     };
 
@@ -784,18 +806,22 @@ __device__ __forceinline__ void flash_f32_body(
     // ---- merge the four partial states: M = max m_w, O = sum acc_w 2^(m_w - M),
     // L = sum l_w 2^(m_w - M), in wave order ----
     __syncthreads();  // every wave is done with its K/V tile
-    float* macc = smem + wave * (BQF * D + 2 * BQF);  // [q][d] accumulator, then m[q], l[q]
+    // rows padded and moved 16 bytes at a time: a lane per row with a stride of D
+    // floats, every write met one bank 32 times over (1.4 us a workgroup)
+    float* macc = smem + wave * MSTATE;
     const float l_pair = l_run + xor32(l_run);
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
+    for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int d = dt * 32 + 8 * (e >> 2) + 4 * g + (e & 3);
-            macc[col * D + d] = acc_o[dt][e];
+        for (int h = 0; h < DT; ++h) {  // columns DT (8 b + 4 g) + 4 h .. + 3
+            f32x4_t v;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) v[x] = acc_o[(4 * h + x) % DT][4 * b + (4 * h + x) / DT];
+            *reinterpret_cast<f32x4_t*>(macc + col * MROW + DT * (8 * b + 4 * g) + 4 * h) = v;
         }
     if (g == 0) {
-        macc[BQF * D + col] = m_run;
-        macc[BQF * D + BQF + col] = l_pair;
+        macc[BQF * MROW + col] = m_run;
+        macc[BQF * MROW + BQF + col] = l_pair;
     }
     __syncthreads();
     // every wave merges D/4 of the d columns of all 32 queries: lane -> (q, 8 d)
@@ -804,7 +830,7 @@ __device__ __forceinline__ void flash_f32_body(
     float mw[NWF], mm = kNegInf;
 #pragma unroll
     for (int w = 0; w < NWF; ++w) {
-        mw[w] = smem[w * (BQF * D + 2 * BQF) + BQF * D + q];
+        mw[w] = smem[w * MSTATE + BQF * MROW + q];
         mm = fmaxf(mm, mw[w]);
     }
     const float m_ref = (mm == kNegInf) ? 0.0f : mm;
@@ -812,7 +838,7 @@ __device__ __forceinline__ void flash_f32_body(
 #pragma unroll
     for (int w = 0; w < NWF; ++w) {
         sc[w] = (mw[w] == kNegInf) ? 0.0f : __builtin_amdgcn_exp2f(mw[w] - m_ref);
-        L += smem[w * (BQF * D + 2 * BQF) + BQF * D + BQF + q] * sc[w];
+        L += smem[w * MSTATE + BQF * MROW + BQF + q] * sc[w];
     }
     const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
     const int orow = q0 + q;
@@ -820,15 +846,11 @@ __device__ __forceinline__ void flash_f32_body(
         float* Orow = O + hoff + (int64_t)orow * D;
 #pragma unroll
         for (int c4 = 0; c4 < D / 32; ++c4) {
-            f32x4_t v;
+            f32x4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int d = dbase + 4 * c4 + i;
-                float o = 0.0f;
-#pragma unroll
-                for (int w = 0; w < NWF; ++w) o += smem[w * (BQF * D + 2 * BQF) + q * D + d] * sc[w];
-                v[i] = o * inv;
-            }
+            for (int w = 0; w < NWF; ++w)
+                v += *reinterpret_cast<const f32x4_t*>(smem + w * MSTATE + q * MROW + dbase + 4 * c4) * sc[w];
+            v *= inv;
             *reinterpret_cast<f32x4_t*>(Orow + dbase + 4 * c4) = v;
         }
         if (lse && wave == 0 && (lane & 1) == 0)
