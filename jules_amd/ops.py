@@ -20,7 +20,9 @@ _DT = {torch.float32: F32, torch.bfloat16: BF16}
 
 
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the raw handle of torch.cuda.current_stream(t.device), without building
+    # the Stream object around it
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _ptr(t):
@@ -36,7 +38,7 @@ def _need(t, name, dtypes, shape=None, numel=None):
         raise ValueError(f"{name}: dtype {t.dtype} not in {dtypes}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    if shape is not None and tuple(t.shape) != tuple(shape):
+    if shape is not None and t.shape != shape:
         raise ValueError(f"{name}: shape {tuple(t.shape)}, expected {tuple(shape)}")
     if numel is not None and t.numel() != numel:
         raise ValueError(f"{name}: {t.numel()} elements, expected {numel}")
@@ -60,17 +62,17 @@ def _workspace(ws, name):
 def _on_device(**tensors):
     """Every given tensor (None entries skipped) is a GPU tensor on the device
     of the first one; returns that device."""
-    dev = None
+    first = None
     for name, t in tensors.items():
         if t is None:
             continue
         if not t.is_cuda:
             raise ValueError(f"{name} must be a GPU tensor")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"{name} is on {t.device}, expected {dev}")
-    return dev
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise ValueError(f"{name} is on {t.device}, expected {first.device}")
+    return None if first is None else first.device
 
 
 def _act(act):
