@@ -47,9 +47,9 @@ __device__ __forceinline__ void finish(const F32Gemm& g, Each&& each) {
     }
 }
 
-template <class CF, bool TA, bool TB, int V>
+template <class CF, bool TA, bool TB, int V, bool FOLD>
 __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Gemm g, int kc, int chunk, float* __restrict__ part) {
-    using T = F32Tile<CF::MF, CF::MT, CF::NT, CF::BK, CF::PF, TA, TB, V>;
+    using T = F32Tile<CF::MF, CF::MT, CF::NT, CF::BK, CF::PF, TA, TB, V, FOLD>;
     constexpr bool ACTS = !TA && !TB;
     __shared__ __attribute__((aligned(16))) float sm[2 * T::STAGE];
     const TileCoord t = tile_coord<8>((g.M + T::BM - 1) / T::BM, (g.N + T::BN - 1) / T::BN);
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Gemm g, int kc
         bias[j] = ACTS && g.bias ? g.bias[min(nw + j * CF::MF, g.N - 1)] : 0.0f;
 
     typename T::Mf::Acc acc[CF::MT][CF::NT];
-    T::run(g.A, g.lda, g.B, g.ldb, m0, g.M - (g.colsum ? 1 : 0), n0, g.N, kb, min(g.K, kb + kc), part ? 0 : chunk,
+    T::run(g.A, g.lda, g.B, g.ldb, m0, g.M - (g.colsum ? 1 : 0), n0, g.N, kb, min(g.K, kb + kc), chunk,
            g.colsum != nullptr, sm, acc);
 
     auto each = [&](auto&& f) {
@@ -97,29 +97,32 @@ using F32Cfg4 = F32Cfg<16, 1, 1, 128, 1>;
 
 template <bool TA, bool TB>
 void launch_f32_tile(int plan, int v, const F32Gemm& g, int splits, int kc, int chunk, float* part, hipStream_t s) {
-    auto go = [&](auto cfg, auto vec) {
+    using yes = std::integral_constant<bool, true>;
+    using no = std::integral_constant<bool, false>;
+    auto go = [&](auto cfg, auto vec, auto fold) {
         using CF = decltype(cfg);
         const int64_t wg =
             (((int64_t)g.M + CF::BM - 1) / CF::BM) * (((int64_t)g.N + CF::BN - 1) / CF::BN) * splits;
-        hipLaunchKernelGGL((gemm_f32_tile_kernel<CF, TA, TB, decltype(vec)::value>), dim3((unsigned)wg), dim3(256), 0,
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<CF, TA, TB, decltype(vec)::value, decltype(fold)::value>), dim3((unsigned)wg), dim3(256), 0,
                            s, g, kc, chunk, part);
     };
     auto pick = [&](auto vec) {
         switch (plan) {
-        case 0: go(F32Cfg0{}, vec); break;
-        case 1: go(F32Cfg1{}, vec); break;
-        case 2: go(F32Cfg2{}, vec); break;
+        case 0: chunk ? go(F32Cfg0{}, vec, yes{}) : go(F32Cfg0{}, vec, no{}); break;
+        case 1: go(F32Cfg1{}, vec, no{}); break;
+        case 2: go(F32Cfg2{}, vec, no{}); break;
         case 3:
             // a transposed B's fragments spill at 128 x 128 (64 x 128 is within 4 %)
-            if constexpr (TB) go(F32Cfg2{}, vec);
-            else go(F32Cfg3{}, vec);
+            if constexpr (TB) go(F32Cfg2{}, vec, no{});
+            else go(F32Cfg3{}, vec, no{});
             break;
-        default: go(F32Cfg4{}, vec); break;
+        default: chunk ? go(F32Cfg4{}, vec, yes{}) : go(F32Cfg4{}, vec, no{}); break;
         }
     };
     if (v == 4) pick(std::integral_constant<int, 4>{});
     else if (v == 1) pick(std::integral_constant<int, 1>{});
-    else go(F32Cfg0{}, std::integral_constant<int, 0>{});
+    else if (chunk) go(F32Cfg0{}, std::integral_constant<int, 0>{}, yes{});
+    else go(F32Cfg0{}, std::integral_constant<int, 0>{}, no{});
 }
 
 // gemm_f32_tile_t.hip: at least one of ta, tb

@@ -194,7 +194,7 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int MF, int MT, int NT, int BK, int PF, bool TA, bool TB, int V>
+template <int MF, int MT, int NT, int BK, int PF, bool TA, bool TB, int V, bool FOLD = false>
 struct F32Tile {
     using Mf = F32Mfma<MF>;
     static constexpr int BM = 2 * MT * MF, BN = 2 * NT * MF, KP = Mf::KP;
@@ -202,8 +202,9 @@ struct F32Tile {
     using SB = F32Slice<MF, BN, BK, TB, V, true>;
     static constexpr int STAGE = SA::FLOATS + SB::FLOATS;
 
-    // acc = the tile at (m0, n0) over k in [kb, ke).  chunk > 0 (a multiple of
-    // 16; one accumulator a wave only): the sum is taken over chunks of that
+    // acc = the tile at (m0, n0) over k in [kb, ke).  FOLD (chunk > 0, a
+    // multiple of 16; one accumulator a wave only; a kernel of its own, its test
+    // per four k-steps costs a chain 12 %): the sum is taken over chunks of that
     // many k, each its own chain, added in order, as a K split into ranges of
     // chunk would add its partial sums.  ones: row M of op(A) reads as 1, so
     // output row M is the column sum of op(B) (TA only).
@@ -225,6 +226,7 @@ struct F32Tile {
         // 128 1046 against 1374 us): slice t + PF loaded first, slice t + 1
         // stored last.
         constexpr bool AHEAD = MT * NT == 1;
+        static_assert(AHEAD || !FOLD, "one accumulator");
         SA ra[PF];
         SB rb[PF];
         typename SA::Src pa(A, lda, m0, M, kb);
@@ -292,18 +294,18 @@ struct F32Tile {
                                 acc[i][j] = Mf::run(a[g & 1][i][s], b[g & 1][j][s], acc[i][j]);
                     if constexpr (AHEAD) {
                         __builtin_amdgcn_sched_barrier(0);
-                        if (chunk && k0 + 4 * KP * g < ke && (left -= 4 * KP) == 0) fold();
+                        if constexpr (FOLD)
+                            if (k0 + 4 * KP * g < ke && (left -= 4 * KP) == 0) fold();
                     }
                 }
                 if (!AHEAD && k0 + BK < ke) store((u + 1) % PF, buf);
                 lds_barrier();
             }
         }
-        if constexpr (AHEAD)
-            if (chunk) {
-                if (left != chunk) fold();
-                acc[0][0] = tot[0][0];
-            }
+        if constexpr (FOLD) {
+            if (left != chunk) fold();
+            acc[0][0] = tot[0][0];
+        }
     }
 };
 
