@@ -433,9 +433,15 @@ inline TileChoice tile_plan(const TileModel& m, int M, int N, int K, hipStream_t
     TileChoice c = tile_choice(m, M, N, K, s != hipStreamPerThread);
     if (c.splits == 1) return c;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
-        stream_workspace((size_t)c.splits * M * N * 4, s, part, lock) == hipSuccess)
-        return c;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+        // another thread may be capturing: growing the workspace concerns this
+        // stream only, and must not end that capture
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        const hipError_t e = stream_workspace((size_t)c.splits * M * N * 4, s, part, lock);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (e == hipSuccess) return c;
+    }
     (void)hipGetLastError();
     *part = nullptr;
     return tile_choice(m, M, N, K, false);
