@@ -26,11 +26,11 @@ namespace kernel {
 // reference FusedKernels.h:61-67; Silu appended (value 5, C ABI JH_ACT_SILU)
 enum class ActivationType { None, Relu, Sigmoid, Tanh, Gelu, Silu };
 
-// reference TilePlanner.h:39-56.  On the GPU a TileConfig names one kernel of
-// the library's gfx950 tile table (jules_hip_gemm_tile): fp32 rows x 64 x K
-// with 4 or 8 rows (the row kernel), 32x32x32 or 64x64x32.  Every table tile
-// gives the same bits (each output is one fma chain over k in order), as in
-// the reference, whose results do not depend on the tile either.
+// reference TilePlanner.h:39-56.  On the GPU a TileConfig is one entry of the
+// library's gfx950 tile table (jules_hip_gemm_tile): fp32 rows x 64 x K with 4
+// or 8 rows, 32x32x32 or 64x64x32.  An entry is a class of shapes; the launch
+// picks its workgroup tile by the shape.  Results never depend on the tile
+// (each output is one fma chain over k in order), as in the reference.
 struct TileConfig {
     int tile_m;
     int tile_n;
@@ -61,16 +61,15 @@ struct ShapeSignature {
     };
 };
 
-// reference TilePlanner.h:74-294.  computeAnalytical returns the tile the
-// fp32 GEMM launch uses by default (the library's table); getTileConfig
-// caches per shape and, with auto-tuning on (the default, as in the
-// reference) and M, N >= 32, times every table kernel that can run the
-// shape on the current GPU (one warm-up and 10 timed launches each, HIP
-// events) and keeps the fastest.  Like the reference, one planner object is
-// not safe to use from two threads at once.
+// reference TilePlanner.h:74-294.  computeAnalytical returns the table's entry
+// for the shape; getTileConfig caches it per shape.  Auto-tuning (on by
+// default, as in the reference) times the function that setBenchmarkKernel
+// registered, for M, N >= 32; without one the entry stands, as the launch runs
+// the same kernel under every entry.  Like the reference, one planner object
+// is not safe to use from two threads at once.
 //
 // setBenchmarkKernel (reference TilePlanner.h:141-148) registers the function
-// that auto-tuning times instead: as in the reference it is called with HOST
+// that auto-tuning times: as in the reference it is called with HOST
 // buffers (A, B filled with 1.0f, C of M*N floats), M, N, K and each
 // candidate TileConfig, one warm-up and 10 timed calls per candidate on the
 // host clock, and must be synchronous.  The candidates stay the GPU table's
@@ -150,9 +149,8 @@ void fusedMatmulRelu(const float* X, const float* W, float* output, int M, int K
 // reference FusedKernels.h:265
 void fusedMatmulBiasRelu(const float* X, const float* W, const float* bias, float* output, int M,
                          int K, int N);
-// reference FusedKernels.h:378.  A cfg naming a kernel of the tile table
-// (what TilePlanner returns) runs that kernel; any other cfg runs the
-// table's default for the shape.  The bits are the same either way.
+// reference FusedKernels.h:378.  The launch picks its tile by the shape under
+// any cfg; the bits do not depend on it.
 void tiledMatmulWithActivation(const float* A, const float* B, float* C, int M, int N, int K,
                                const TileConfig& cfg, ActivationType act = ActivationType::None);
 // reference FusedKernels.h:633-644: C = alpha op(A) op(B) + beta C with the

@@ -61,25 +61,6 @@ int set_last_error(int status, const std::string& message) {
     g_last_error = message;
     return status;
 }
-
-// jules_hip_gemm_bias_act for fp32 with a chosen entry of the tile table
-// (variant < 0: the table's default for the shape), which must be able to
-// take the shape; the launch picks its own tile, every one with the same bits.
-int gemm_f32_with_variant(int variant, int act, const float* A, const float* B, const float* bias,
-                          float* C, int M, int N, int K, hipStream_t s) {
-    if (!valid_act(act)) return fail(JH_ERR_ACT, "gemm: activation code %d", act);
-    if (M < 0 || N < 0 || K < 0) return fail(JH_ERR_SHAPE, "gemm: M=%d N=%d K=%d", M, N, K);
-    if ((int64_t)M * K > kMaxElems || (int64_t)K * N > kMaxElems || (int64_t)M * N > kMaxElems)
-        return fail(JH_ERR_SHAPE, "gemm: M=%d N=%d K=%d too large", M, N, K);
-    if (variant < 0) variant = f32_gemm_tile(M, N, K).variant;
-    if (!f32_variant_valid(variant, K))
-        return fail(JH_ERR_ARG, "gemm f32: kernel variant %d cannot run K=%d", variant, K);
-    if (M == 0 || N == 0) return JH_OK;
-    if (!C || (K > 0 && (!A || !B))) return fail(JH_ERR_NULL, "gemm: null A, B or C");
-    if (!aligned(A, 4) || !aligned(B, 4) || !aligned(C, 4) || !aligned(bias, 4))
-        return fail(JH_ERR_ALIGN, "gemm f32: operands must be 4-byte aligned");
-    return check_hip(launch_gemm_f32(act, A, B, bias, C, M, N, K, s), "gemm f32 launch");
-}
 }  // namespace jh
 
 extern "C" {
@@ -112,13 +93,17 @@ int jules_hip_gemm_bias_act(int dtype, int act, const void* A, const void* B, co
     if ((int64_t)M * K > kMaxElems || (int64_t)K * N > kMaxElems || (int64_t)M * N > kMaxElems)
         return fail(JH_ERR_SHAPE, "gemm: M=%d N=%d K=%d too large", M, N, K);
     if (dtype != JH_F32 && dtype != JH_BF16) return fail(JH_ERR_DTYPE, "gemm: dtype %d", dtype);
-    if (dtype == JH_F32)
-        return jh::gemm_f32_with_variant(-1, act, static_cast<const float*>(A),
-                                         static_cast<const float*>(B), bias, static_cast<float*>(C),
-                                         M, N, K, static_cast<hipStream_t>(stream));
     if (M == 0 || N == 0) return JH_OK;
     if (!C || (K > 0 && (!A || !B))) return fail(JH_ERR_NULL, "gemm: null A, B or C");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == JH_F32) {
+        if (!aligned(A, 4) || !aligned(B, 4) || !aligned(C, 4) || !aligned(bias, 4))
+            return fail(JH_ERR_ALIGN, "gemm f32: operands must be 4-byte aligned");
+        return check_hip(jh::launch_gemm_f32(act, static_cast<const float*>(A),
+                                             static_cast<const float*>(B), bias,
+                                             static_cast<float*>(C), M, N, K, s),
+                         "gemm f32 launch");
+    }
     if (M % 8 || N % 8 || K % 8)
         return fail(JH_ERR_UNSUPPORTED, "gemm bf16: M, N, K must be multiples of 8 (got %d %d %d)",
                     M, N, K);

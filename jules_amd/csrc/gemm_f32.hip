@@ -8,7 +8,7 @@
 // :401-406), followed by + bias[j] and the vector-path activation.  The fp32
 // MFMAs compute that chain bit for bit (gemm_f32_tile.hpp), so the GEMM runs
 // on them, with no split of K.  Against thread tiles of v_fma_f32: 2000 x 3072
-// x 1024 305 -> 113 us, 512^3 12.3 -> 10.1 us with its operands cold.
+// x 1024 305 -> 113 us, 512^3 12.3 -> 8.0 us with its operands cold.
 #include "common.hpp"
 #include "launch.hpp"
 

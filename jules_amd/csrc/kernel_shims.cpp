@@ -83,33 +83,19 @@ private:
     bool ok_ = true;
 };
 
-// variant: a kernel of the tile table, or -1 for the table's default
 void run_gemm(const float* A, const float* B, const float* bias, float* C, int M, int N, int K,
-              int act, int variant = -1) {
+              int act) {
     if (M < 0 || N < 0 || K < 0) return record(JH_ERR_SHAPE);
     DevBuf a(A, sizeof(float) * (size_t)M * K, true, false);
     DevBuf b(B, sizeof(float) * (size_t)K * N, true, false);
     DevBuf bi(bias, bias ? sizeof(float) * (size_t)N : 0, true, false);
     DevBuf c(C, sizeof(float) * (size_t)M * N, false, true);
     if (!a.ok() || !b.ok() || !bi.ok() || !c.ok()) return record(JH_ERR_HIP);
-    int st = jh::gemm_f32_with_variant(variant, act, static_cast<const float*>(a.get()),
-                                       static_cast<const float*>(b.get()),
-                                       static_cast<const float*>(bi.get()),
-                                       static_cast<float*>(c.get()), M, N, K, nullptr);
+    int st = jules_hip_gemm_bias_act(JH_F32, act, a.get(), b.get(), static_cast<const float*>(bi.get()),
+                                     c.get(), M, N, K, nullptr);
     if (st == JH_OK && hipDeviceSynchronize() != hipSuccess) st = JH_ERR_HIP;
     if (st == JH_OK && !c.finish()) st = JH_ERR_HIP;
     record(st);
-}
-
-// the table kernel a TileConfig names at depth K, or -1
-int variant_of(const TileConfig& cfg, int K) {
-    for (int v = jh::GV_F32_ROWS1; v <= jh::GV_F32_T64; ++v) {
-        const jh::GemmTile t = jh::f32_variant_tile(v, K);
-        if (jh::f32_variant_valid(v, K) && t.tile_m == cfg.tile_m && t.tile_n == cfg.tile_n &&
-            t.tile_k == cfg.tile_k)
-            return v;
-    }
-    return -1;
 }
 
 TileConfig to_config(const jh::GemmTile& t) { return TileConfig{t.tile_m, t.tile_n, t.tile_k}; }
@@ -245,7 +231,7 @@ void fusedMatmulBiasRelu(const float* X, const float* W, const float* bias, floa
 }
 
 void tiledMatmulWithActivation(const float* A, const float* B, float* C, int M, int N, int K,
-                               const TileConfig& cfg, ActivationType act) {
+                               const TileConfig&, ActivationType act) {
     if (K == 0 && M > 0 && N > 0) {
         // The reference zeroes C (FusedKernels.h:382) and applies the
         // activation only inside its K-slice loop (:407), which K = 0 never
@@ -266,7 +252,7 @@ void tiledMatmulWithActivation(const float* A, const float* B, float* C, int M, 
                                                      : "tiledMatmulWithActivation: zeroing C failed");
         return record(st);
     }
-    run_gemm(A, B, nullptr, C, M, N, K, static_cast<int>(act), variant_of(cfg, K));
+    run_gemm(A, B, nullptr, C, M, N, K, static_cast<int>(act));
 }
 
 void blasMatmul(const float* A, const float* B, float* C, int M, int N, int K, float alpha,

@@ -42,10 +42,6 @@ struct F32Gemm {
     float* colsum;
 };
 hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s);
-// the fp32 GEMM entry point's validation and launch with a chosen table
-// variant (-1: the table's default), for jules::kernel::tiledMatmulWithActivation
-int gemm_f32_with_variant(int variant, int act, const float* A, const float* B, const float* bias,
-                          float* C, int M, int N, int K, hipStream_t s);
 // C = alpha op(A) op(B) + beta C, fp32 on MFMA (mlp.hip); op(X) = X^T when
 // the trans flag is set; row-major with leading dimensions lda, ldb, ldc
 hipError_t launch_sgemm(bool transA, bool transB, int M, int N, int K, float alpha, const float* A,
