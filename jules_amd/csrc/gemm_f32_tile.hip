@@ -56,6 +56,28 @@ int f32_plan(int M, int N, int kc, int splits, float* us_out) {
     return best;
 }
 
+struct F32Dims {
+    int bm, bn, bk;
+};
+template <class CF>
+constexpr F32Dims f32_dims() {
+    return {CF::BM, CF::BN, CF::BK};
+}
+constexpr F32Dims kF32Dims[5] = {f32_dims<F32Cfg0>(), f32_dims<F32Cfg1>(), f32_dims<F32Cfg2>(),
+                                 f32_dims<F32Cfg3>(), f32_dims<F32Cfg4>()};
+
+// Whether every byte offset that the plan's tile forms (F32Slice::Src) is below
+// 2^32: to each k of a slice, those past K among them, where k is the outer
+// dimension in memory, and to each row that exists where it is not.
+bool f32_fits(const F32Gemm& g, int plan) {
+    const F32Dims& t = kF32Dims[g.tb && plan == 3 ? 2 : plan];  // as launch_f32_tile
+    const auto span = [&](bool k_outer, int x, int rows, int64_t ld) {
+        const int64_t xs = std::min(x, rows);
+        return 4 * (k_outer ? (t.bk - 1) * ld + xs : (xs - 1) * ld + t.bk);
+    };
+    return std::max(span(g.ta, t.bm, g.M, g.lda), span(!g.tb, t.bn, g.N, g.ldb)) <= int64_t(1) << 32;
+}
+
 }  // namespace
 
 hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
@@ -85,13 +107,11 @@ hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hi
         part = nullptr;
         if (!chunk) plan = f32_plan(g.M, g.N, kc, 1, &us);
     }
-    // whole 16-byte pieces of the operands whose k is the outer dimension; 32-bit
-    // offsets within a tile (128 rows, or the rows there are, or a slice's 64)
-    const auto spans = [](bool rows_are_k, int rows, int64_t ld) {
-        return (int64_t)std::min(rows, rows_are_k ? 64 : 128) * ld * 4 >= (int64_t(1) << 32);
-    };
-    const bool big = spans(g.ta, g.ta ? g.K : g.M, g.lda) || spans(!g.tb, g.tb ? g.N : g.K, g.ldb);
-    const int v = big ? 0 : (!g.ta || (g.M - (g.colsum ? 1 : 0)) % 4 == 0) && (g.tb || g.N % 4 == 0) ? 4 : 1;
+    // a tile whose offsets pass 32 bits gives way to 32 x 32, then to 64-bit ones
+    if (!f32_fits(g, plan)) plan = 0;
+    // whole 16-byte pieces of the operands whose k is the outer dimension
+    const int v = !f32_fits(g, plan) ? 0
+                  : (!g.ta || (g.M - (g.colsum ? 1 : 0)) % 4 == 0) && (g.tb || g.N % 4 == 0) ? 4 : 1;
     if (g.ta || g.tb) launch_f32_tile_trans(plan, v, g, splits, kc, chunk, part, s);
     else launch_f32_tile<false, false>(plan, v, g, splits, kc, chunk, part, s);
     if (part) {

@@ -1,0 +1,120 @@
+// host_launch.cpp - what the library's entry points launch, and what they do
+// with the workspaces they hold, checked without a GPU: the library's objects
+// linked against hip_stub.cpp, its host sources built with AddressSanitizer and
+// UndefinedBehaviorSanitizer.  `host_launch <check>` runs one check and prints
+// "<check> ok"; run by tests/test_host_launch.py.
+#include <algorithm>
+#include <cstdint>
+#include <cstdio>
+#include <cstring>
+#include <string>
+
+#include "hip_stub.hpp"
+#include "jules_hip.h"
+#include "launch.hpp"
+
+static int g_fail = 0;
+#define EXPECT(cond, ...)                                                            \
+    do {                                                                             \
+        if (!(cond)) {                                                               \
+            if (++g_fail <= 20) {                                                    \
+                std::fprintf(stderr, "line %d: expected %s: ", __LINE__, #cond);     \
+                std::fprintf(stderr, __VA_ARGS__);                                   \
+                std::fprintf(stderr, "\n");                                          \
+            }                                                                        \
+        }                                                                            \
+    } while (0)
+
+// an operand that no check lets anything read
+template <typename T = float>
+static T* fake(int i) {
+    return reinterpret_cast<T*>((uintptr_t(1) << 46) + (uintptr_t(i) << 42));
+}
+
+// A launch of the fp32 tile kernel: its tile and variant, from its name.
+struct F32Launch {
+    int mf, mt, nt, bk, pf, v;
+    bool ta, tb, fold;
+};
+static bool f32_launch(const std::string& name, F32Launch* f) {
+    char ta[8], tb[8], fold[8];
+    const int n = std::sscanf(name.c_str(),
+                              "void jh::gemm_f32_tile_kernel<jh::F32Cfg<%d, %d, %d, %d, %d>, %5[a-z], %5[a-z], %d, %5[a-z]>",
+                              &f->mf, &f->mt, &f->nt, &f->bk, &f->pf, ta, tb, &f->v, fold);
+    f->ta = !std::strcmp(ta, "true");
+    f->tb = !std::strcmp(tb, "true");
+    f->fold = !std::strcmp(fold, "true");
+    return n == 9;
+}
+
+// Every fp32 product whose tile spans 2^32 bytes of an operand takes the 64-bit
+// offsets (V = 0).  The kernel forms an offset for each k of a slice, also those
+// past K, of an operand whose k is the outer dimension, and for each row that
+// exists of the others.
+static void f32_offsets() {
+    int tiles = 0, wide = 0;
+    stub::on_launch = [&](const stub::Launch& l) {
+        F32Launch f;
+        if (!f32_launch(l.kernel, &f)) return;
+        ++tiles;
+        wide += f.v == 0;
+        const auto g = l.arg<jh::F32Gemm>(0);
+        const auto last = [&](bool k_outer, int x, int rows, int64_t ld) {
+            const int64_t xs = std::min(x, rows);
+            return 4 * (k_outer ? (f.bk - 1) * ld + xs : (xs - 1) * ld + f.bk);
+        };
+        const int64_t a = last(f.ta, 2 * f.mt * f.mf, g.M - (g.colsum ? 1 : 0), g.lda);
+        const int64_t b = last(!f.tb, 2 * f.nt * f.mf, g.N, g.ldb);
+        EXPECT(f.v == 0 || std::max(a, b) <= int64_t(1) << 32, "%s M=%d N=%d K=%d lda=%ld ldb=%ld", l.kernel.c_str(),
+               g.M, g.N, g.K, (long)g.lda, (long)g.ldb);
+        // and an ordinary row keeps the 32-bit ones
+        EXPECT(f.v != 0 || std::max(g.lda, g.ldb) > 1 << 20, "%s lda=%ld ldb=%ld", l.kernel.c_str(), (long)g.lda,
+               (long)g.ldb);
+    };
+    const int lds[] = {4096,     1 << 20,  8300000,  8388607,  8388608,   8400000,  8454659,  8454661, 9000000, 10000000,
+                       16777215, 16777216, 16909321, 20000000, 33554432,  34636833, 67108863, 70000000, 71582789,
+                       80000000, 300000000, 1 << 30, INT32_MAX};
+    for (int ta : {0, 1})
+        for (int tb : {0, 1})
+            for (int M : {1, 3, 32, 33, 100, 512, 2048})
+                for (int N : {1, 32, 33, 130, 2048})
+                    for (int K : {1, 4, 10, 15, 17, 63, 64, 129, 256, 1024})
+                        for (int ld : lds)
+                            for (int other : {4096, ld}) {
+                                const int lda = std::max(ld, ta ? M : K), ldb = std::max(other, tb ? K : N);
+                                (void)jules_hip_sgemm(ta, tb, M, N, K, 1.0f, fake(0), lda, fake(1), ldb, 0.0f, fake(2),
+                                                      N, nullptr);
+                                const int la = std::max(other, ta ? M : K), lb = std::max(ld, tb ? K : N);
+                                (void)jules_hip_sgemm(ta, tb, M, N, K, 1.0f, fake(0), la, fake(1), lb, 1.0f, fake(2),
+                                                      N, nullptr);
+                            }
+    for (int M : {1, 8, 200})
+        for (int K : {1, 4, 17, 40})
+            for (int N : lds)
+                (void)jules_hip_gemm_bias_act(JH_F32, JH_ACT_NONE, fake(0), fake(1), nullptr, fake(2), M, N, K, nullptr);
+    for (int N : {1, 8, 200})
+        for (int M : {1, 8, 200})
+            for (int K : lds)
+                (void)jules_hip_gemm_bias_act(JH_F32, JH_ACT_NONE, fake(0), fake(1), nullptr, fake(2), M, N, K, nullptr);
+    EXPECT(tiles > 10000 && wide > 1000, "%d launches, %d with 64-bit offsets", tiles, wide);
+}
+
+static const struct {
+    const char* name;
+    void (*run)();
+} kChecks[] = {
+    {"f32_offsets", f32_offsets},
+};
+
+int main(int argc, char** argv) {
+    for (const auto& c : kChecks)
+        if (argc == 2 && !std::strcmp(argv[1], c.name)) {
+            c.run();
+            stub::on_launch = nullptr;
+            if (g_fail) std::fprintf(stderr, "%d failed expectations\n", g_fail);
+            else std::printf("%s ok\n", c.name);
+            return g_fail ? 1 : 0;
+        }
+    std::fprintf(stderr, "usage: host_launch <check>\n");
+    return 2;
+}
