@@ -13,27 +13,24 @@
 // used as given (its default is 1/sqrt(D) of the real D).
 #include <map>
 #include <mutex>
+#include <tuple>
 
 #include "common.hpp"
 #include "launch.hpp"
 
 namespace jh {
 
-// One workspace per (device, stream), kept for the process: calls on one
-// stream run in order and may share it, calls on other streams get their
-// own.  A larger need replaces it once the stream is done with the old one.
-// The lock is the caller's until it has enqueued every kernel that uses the
-// workspace, so that threads sharing a stream neither interleave their kernels
-// nor replace the buffer under each other; recursive, since a registry call
-// holds it around entry points of the library.
-hipError_t stream_workspace(size_t need, hipStream_t s, void** ws, WorkspaceLock* lock) {
+namespace {
+enum BufferUse { BUFFER_CALL, BUFFER_PARTIALS };
+
+hipError_t stream_buffer(BufferUse use, size_t need, hipStream_t s, void** ws, WorkspaceLock* lock) {
     static std::recursive_mutex mu;
-    static std::map<std::pair<int, hipStream_t>, std::pair<void*, size_t>> cache;
+    static std::map<std::tuple<int, hipStream_t, BufferUse>, std::pair<void*, size_t>> cache;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     *lock = WorkspaceLock(mu);
-    auto& slot = cache[{dev, s}];
+    auto& slot = cache[{dev, s, use}];
     if (slot.second < need) {
         if (slot.first) {
             if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
@@ -46,6 +43,25 @@ hipError_t stream_workspace(size_t need, hipStream_t s, void** ws, WorkspaceLock
     }
     *ws = slot.first;
     return hipSuccess;
+}
+}  // namespace
+
+// One workspace per (device, stream), kept for the process: calls on one
+// stream run in order and may share it, calls on other streams get their
+// own.  A larger need replaces it once the stream is done with the old one.
+// The lock is the caller's until it has enqueued every kernel that uses the
+// workspace, so that threads sharing a stream neither interleave their kernels
+// nor replace the buffer under each other; recursive, since a registry call
+// holds it around entry points of the library.
+hipError_t stream_workspace(size_t need, hipStream_t s, void** ws, WorkspaceLock* lock) {
+    return stream_buffer(BUFFER_CALL, need, s, ws, lock);
+}
+
+// A graph captured after a warm-up holds the workspace's address.  A GEMM only
+// splits K outside of captures, and with a buffer apart it neither writes nor
+// replaces what such a graph replays into.
+hipError_t stream_partials(hipStream_t s, void** ws, WorkspaceLock* lock) {
+    return stream_buffer(BUFFER_PARTIALS, kMaxPartialBytes, s, ws, lock);
 }
 
 namespace {

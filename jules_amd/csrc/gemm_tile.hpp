@@ -392,7 +392,6 @@ struct TileModel {
 struct TileChoice {
     int plan, splits, kc;
 };
-constexpr int64_t kMaxPartialBytes = int64_t(64) << 20;  // bound of the split's workspace
 
 inline TileChoice tile_choice(const TileModel& m, int M, int N, int K, bool may_split) {
     TileChoice best{0, 1, 0};
@@ -403,7 +402,7 @@ inline TileChoice tile_choice(const TileModel& m, int M, int N, int K, bool may_
         const int slices = (K + p.bk - 1) / p.bk;
         for (int S : {1, 2, 3, 4, 6, 8}) {
             if (S > 1 && (!may_split || slices < 2 * S || tiles * S > 512 ||
-                          (int64_t)S * M * N * 4 > kMaxPartialBytes))
+                          (int64_t)S * M * N * 4 > (int64_t)kMaxPartialBytes))
                 break;
             const int per = (slices + S - 1) / S;
             const int z = slices ? (slices + per - 1) / per : 1;
@@ -422,11 +421,12 @@ inline TileChoice tile_choice(const TileModel& m, int M, int N, int K, bool may_
     return best;
 }
 
-// tile_choice with the partial sums' memory: the stream's workspace, under its
-// lock until the caller has enqueued the reduction.  It may not be allocated
-// while a graph is being captured, nor kept by the graph (a later call may
-// replace it), and hipStreamPerThread is one handle for many streams: there,
-// and without memory for it, K is not split.
+// tile_choice with the partial sums' memory: the stream's buffer for them,
+// under its lock until the caller has enqueued the reduction.  It may not be
+// allocated while a graph is being captured, nor kept by the graph (eager calls
+// on the stream write it while the graph may run on another), and
+// hipStreamPerThread is one handle for many streams: there, and without memory
+// for it, K is not split.
 inline TileChoice tile_plan(const TileModel& m, int M, int N, int K, hipStream_t s, void** part,
                             WorkspaceLock* lock) {
     *part = nullptr;
@@ -434,11 +434,11 @@ inline TileChoice tile_plan(const TileModel& m, int M, int N, int K, hipStream_t
     if (c.splits == 1) return c;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
-        // another thread may be capturing: growing the workspace concerns this
+        // another thread may be capturing: allocating the buffer concerns this
         // stream only, and must not end that capture
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         (void)hipThreadExchangeStreamCaptureMode(&mode);
-        const hipError_t e = stream_workspace((size_t)c.splits * M * N * 4, s, part, lock);
+        const hipError_t e = stream_partials(s, part, lock);
         (void)hipThreadExchangeStreamCaptureMode(&mode);
         if (e == hipSuccess) return c;
     }

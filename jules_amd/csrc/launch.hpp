@@ -158,6 +158,10 @@ hipError_t launch_flash_bwd_padded(int dtype, int causal, float scale, const voi
 // lock under which the caller enqueues what uses it
 using WorkspaceLock = std::unique_lock<std::recursive_mutex>;
 hipError_t stream_workspace(size_t need, hipStream_t s, void** ws, WorkspaceLock* lock);
+// the same for the partial sums of a GEMM whose K is split: a buffer of their
+// own, of kMaxPartialBytes whatever the call needs
+constexpr size_t kMaxPartialBytes = size_t(64) << 20;
+hipError_t stream_partials(hipStream_t s, void** ws, WorkspaceLock* lock);
 // the library's static device scratch (scratch.hip): its size, and the
 // device address of the current device's copy (looked up once per device;
 // allocates nothing)

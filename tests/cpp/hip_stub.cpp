@@ -9,7 +9,6 @@
 
 #include <cstdlib>
 #include <cstring>
-#include <map>
 #include <mutex>
 
 namespace stub {
@@ -53,6 +52,10 @@ bool allocated(const void* p) {
     if (it == blocks().begin()) return false;
     --it;
     return c < it->first + it->second;
+}
+std::map<const char*, size_t> allocations() {
+    std::lock_guard<std::mutex> lock(mu());
+    return blocks();
 }
 }  // namespace stub
 

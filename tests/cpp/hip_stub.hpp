@@ -7,6 +7,7 @@
 
 #include <cstddef>
 #include <functional>
+#include <map>
 #include <set>
 #include <string>
 
@@ -25,5 +26,6 @@ extern std::function<void(const Launch&)> on_launch;
 extern std::function<void(hipStream_t)> on_synchronize;  // before hipStreamSynchronize returns
 extern std::set<hipStream_t> capturing;                  // streams under capture
 bool allocated(const void* p);  // p lies in device memory that has not been freed
+std::map<const char*, size_t> allocations();
 
 }  // namespace stub

@@ -99,11 +99,55 @@ static void f32_offsets() {
     EXPECT(tiles > 10000 && wide > 1000, "%d launches, %d with 64-bit offsets", tiles, wide);
 }
 
+// Calls that keep a workspace of the stream are run once, captured (their
+// address is then the graph's) and followed by eager GEMMs that split K on the
+// same stream: these may neither free nor use the memory that the graph holds.
+static void graph_workspace() {
+    const auto s = reinterpret_cast<hipStream_t>(uintptr_t(0x1230));
+    const auto held = [&] {
+        (void)jules_hip_flash_attn_fwd(JH_F32, 0, 0.1f, fake(0), fake(1), fake(2), fake(3), nullptr, 1, 2, 100, 80, s);
+        (void)jules_hip_flash_attn_bwd(JH_BF16, 0, 0.1f, fake(0), fake(1), fake(2), fake(3), fake(4), fake(5), fake(6),
+                                       fake(7), fake(8), 1, 2, 50, 80, fake(9), 1 << 20, s);
+        (void)jules_hip_softmax(fake(0), fake(1), 2, 70000, s);
+        (void)jules_hip_sgemm(0, 0, 64, 64, 4096, 1.0f, fake(0), 4096, fake(1), 64, 0.0f, fake(2), 64, s);
+        (void)jules_hip_matmul_int8(fake<int8_t>(0), fake<int8_t>(1), fake(2), 8, 512, 1024, 1.0f, 1.0f, nullptr, s);
+    };
+    held();
+    const auto before = stub::allocations();
+    EXPECT(!before.empty(), "no workspace was allocated");
+    stub::capturing.insert(s);
+    int captured = 0;
+    stub::on_launch = [&](const stub::Launch&) { ++captured; };
+    held();
+    EXPECT(captured > 10 && stub::allocations() == before, "%d launches captured", captured);
+    stub::capturing.clear();
+
+    int split = 0;
+    stub::on_launch = [&](const stub::Launch& l) {
+        const char* part = l.kernel.find("gemm_bf16_tile_kernel") != std::string::npos ? l.arg<const char*>(4)
+                           : l.kernel.find("int8_tile_kernel") != std::string::npos    ? l.arg<const char*>(3)
+                                                                                       : nullptr;
+        if (!part) return;
+        ++split;
+        EXPECT(stub::allocated(part), "%s", l.kernel.c_str());
+        for (const auto& b : before)
+            EXPECT(part < b.first || part >= b.first + b.second, "%s writes the graph's workspace", l.kernel.c_str());
+    };
+    for (int N : {504, 1504, 4104}) {
+        (void)jules_hip_gemm_bias_act(JH_BF16, JH_ACT_NONE, fake(0), fake(1), nullptr, fake(2), 24, N, 4352, s);
+        (void)jules_hip_matmul_int8(fake<int8_t>(0), fake<int8_t>(1), fake(2), 72, N / 16 * 16, 4368, 1.0f, 1.0f,
+                                    nullptr, s);
+    }
+    EXPECT(split >= 4, "%d GEMMs split K", split);
+    for (const auto& b : before) EXPECT(stub::allocated(b.first), "the graph's workspace was freed");
+}
+
 static const struct {
     const char* name;
     void (*run)();
 } kChecks[] = {
     {"f32_offsets", f32_offsets},
+    {"graph_workspace", graph_workspace},
 };
 
 int main(int argc, char** argv) {

@@ -88,6 +88,32 @@ def test_bf16_split_under_capture(dev):
         _check(eager, A, B, bias, "silu")
 
 
+def test_split_leaves_a_graphs_workspace(dev):
+    """A graph captured from a call that keeps the stream's workspace replays
+    between eager GEMMs that split K on that stream."""
+    case("gemm bf16 split on the stream of a captured int8 decode")
+    g = torch.Generator(device=dev).manual_seed(2)
+    a8 = torch.randint(-128, 128, (8, 1024), generator=g, device=dev, dtype=torch.int8)
+    b8 = torch.randint(-128, 128, (1024, 512), generator=g, device=dev, dtype=torch.int8)
+    one = torch.ones((), device=dev)
+    A, B, _ = _operands(dev, 24, 4104, 4352, 11)
+    y8 = torch.empty((8, 512), device=dev)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        ops.matmul_int8(a8, b8, 1.0, 1.0, out=y8)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            ops.matmul_int8(a8, b8, 1.0, 1.0, out=y8)
+        for _ in range(3):
+            y = ops.gemm_bias_act(A, B, None, "none")
+            a8.copy_(torch.randint(-128, 128, a8.shape, generator=g, device=dev, dtype=torch.int8))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y8, _int8_ref(a8, b8, one, one, None))
+            _check(y, A, B, None, "none")
+
+
 def _int8_ref(A, B, rs, cs, bias):
     """The scalar path's arithmetic on the exact integer sums (each below
     2^31, so the float64 product holds it exactly)."""
