@@ -23,25 +23,40 @@ namespace jh {
 namespace {
 enum BufferUse { BUFFER_CALL, BUFFER_PARTIALS };
 
+// A lock of its own: a call that waits for its stream to replace a buffer
+// keeps no other stream's calls waiting.
+struct StreamBuffer {
+    std::recursive_mutex mu;
+    void* ptr = nullptr;
+    size_t bytes = 0;
+};
+
 hipError_t stream_buffer(BufferUse use, size_t need, hipStream_t s, void** ws, WorkspaceLock* lock) {
-    static std::recursive_mutex mu;
-    static std::map<std::tuple<int, hipStream_t, BufferUse>, std::pair<void*, size_t>> cache;
+    static std::mutex mu;  // of the map only; its elements stay where they are
+    static std::map<std::tuple<int, hipStream_t, BufferUse>, StreamBuffer> buffers;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    *lock = WorkspaceLock(mu);
-    auto& slot = cache[{dev, s, use}];
-    if (slot.second < need) {
-        if (slot.first) {
-            if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
-            (void)hipFree(slot.first);
-        }
-        slot = {nullptr, 0};
-        void* p = nullptr;
-        if ((e = hipMalloc(&p, need)) != hipSuccess) return e;
-        slot = {p, need};
+    StreamBuffer* b;
+    {
+        std::lock_guard<std::mutex> map_lock(mu);
+        b = &buffers[{dev, s, use}];
     }
-    *ws = slot.first;
+    *lock = WorkspaceLock(b->mu);
+    if (b->bytes < need) {
+        if (b->ptr) {
+            if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+            (void)hipFree(b->ptr);
+        }
+        b->ptr = nullptr;
+        b->bytes = 0;
+        if ((e = hipMalloc(&b->ptr, need)) != hipSuccess) {
+            b->ptr = nullptr;
+            return e;
+        }
+        b->bytes = need;
+    }
+    *ws = b->ptr;
     return hipSuccess;
 }
 }  // namespace

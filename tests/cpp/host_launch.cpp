@@ -4,9 +4,12 @@
 // UndefinedBehaviorSanitizer.  `host_launch <check>` runs one check and prints
 // "<check> ok"; run by tests/test_host_launch.py.
 #include <algorithm>
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <future>
 #include <string>
 
 #include "hip_stub.hpp"
@@ -142,12 +145,41 @@ static void graph_workspace() {
     for (const auto& b : before) EXPECT(stub::allocated(b.first), "the graph's workspace was freed");
 }
 
+// While a call waits for its stream to replace a workspace, calls of another
+// thread on another stream go on.
+static void stream_locks() {
+    const auto a = reinterpret_cast<hipStream_t>(uintptr_t(0x1230)), b = reinterpret_cast<hipStream_t>(uintptr_t(0x4560));
+    const auto decode = [](int N, hipStream_t s) {
+        return jules_hip_matmul_int8(fake<int8_t>(0), fake<int8_t>(1), fake(2), 8, N, 1024, 1.0f, 1.0f, nullptr, s);
+    };
+    EXPECT(decode(512, a) == JH_OK, "first call");
+    bool waited = false;
+    stub::on_synchronize = [&](hipStream_t s) {
+        if (s != a || waited) return;
+        waited = true;
+        auto other = std::async(std::launch::async, [&] {
+            int st = decode(512, b);
+            if (st == JH_OK) st = jules_hip_gemm_bias_act(JH_BF16, 0, fake(0), fake(1), nullptr, fake(2), 24, 504, 4352, b);
+            return st;
+        });
+        if (other.wait_for(std::chrono::seconds(5)) != std::future_status::ready) {
+            std::fprintf(stderr, "the other stream's calls wait too\n");
+            std::_Exit(1);
+        }
+        EXPECT(other.get() == JH_OK, "calls on the other stream");
+    };
+    EXPECT(decode(8192, a) == JH_OK, "call that replaces its workspace");
+    EXPECT(waited, "no workspace was replaced");
+    stub::on_synchronize = nullptr;
+}
+
 static const struct {
     const char* name;
     void (*run)();
 } kChecks[] = {
     {"f32_offsets", f32_offsets},
     {"graph_workspace", graph_workspace},
+    {"stream_locks", stream_locks},
 };
 
 int main(int argc, char** argv) {
