@@ -25,6 +25,13 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+// 16 bytes at any 4-byte address, at any 2-byte address
+struct f32x4_any_t {
+    f32x4_t v;
+} __attribute__((packed, aligned(4)));
+struct u32x4_any2_t {
+    u32x4_t v;
+} __attribute__((packed, aligned(2)));
 
 // ---- activation epilogue ---------------------------------------------------
 

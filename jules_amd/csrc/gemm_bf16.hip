@@ -550,7 +550,7 @@ __device__ __forceinline__ u32x4_t act_pack8(const float (&v)[8]) {
 }
 
 // C = act(sum over z of part[z], in z order, + bias): 8 columns per thread
-// (N % 8 == 0)
+// (N % 8 == 0), at any address that C may have
 __global__ __launch_bounds__(256) void gemm_bf16_reduce_kernel(const float* __restrict__ part, int S,
                                                                const float* __restrict__ bias,
                                                                uint16_t* __restrict__ C, int act,
@@ -569,7 +569,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_reduce_kernel(const float* __re
     const int col = (int)(i % N);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (j < 4 ? lo[j] : hi[j - 4]) + (bias ? bias[col + j] : 0.0f);
-    JH_DISPATCH_ACT(act, ACT, *reinterpret_cast<u32x4_t*>(C + i) = act_pack8<ACT>(v));
+    JH_DISPATCH_ACT(act, ACT, reinterpret_cast<u32x4_any2_t*>(C + i)->v = act_pack8<ACT>(v));
 }
 
 // The tile kernel's tiles, with the waves, slice bytes and ring depth measured

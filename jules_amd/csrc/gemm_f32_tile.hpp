@@ -56,10 +56,6 @@ struct F32Mfma<16> {
     static __device__ __forceinline__ int row(int lane, int e) { return 4 * (lane >> 4) + e; }
 };
 
-struct f32x4_any_t {  // 16 bytes at any 4-byte address
-    f32x4_t v;
-} __attribute__((packed, aligned(4)));
-
 // One operand's slice, X rows (columns) of the tile by BK k.  CONTIG: k is the
 // contiguous dimension in memory, loaded 4 floats at a time wherever the rows
 // start (only the last slice, one float at a time, can reach past a row).  Else

@@ -92,7 +92,8 @@ __global__ __launch_bounds__(T::THREADS) void int8_tile_kernel(
     }
 }
 
-// C = scale(sum over z of part[z]): 4 columns per thread (N % 16 == 0)
+// C = scale(sum over z of part[z]): 4 columns per thread (N % 16 == 0), at any
+// address that C may have
 __global__ __launch_bounds__(256) void int8_reduce_kernel(
     const int* __restrict__ part, int S, float* __restrict__ C, int64_t total, int N, float scale_a,
     float scale_b, const float* __restrict__ row_scale, const float* __restrict__ col_scale,
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(256) void int8_reduce_kernel(
     f32x4_t o;
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = i8_scale(v[j], rs, col_scale ? col_scale[n + j] : scale_b, bias, n + j);
-    *reinterpret_cast<f32x4_t*>(C + i) = o;
+    reinterpret_cast<f32x4_any_t*>(C + i)->v = o;
 }
 
 // As in gemm_bf16.hip; the fit is over 150 shapes (M 1-4096, N and K

@@ -88,6 +88,28 @@ def test_bf16_split_under_capture(dev):
         _check(eager, A, B, bias, "silu")
 
 
+@pytest.mark.parametrize("k", [1, 3])
+def test_split_into_misaligned_outputs(dev, k):
+    """Where K is split, an output that starts k elements past a 16-byte
+    address holds the bits of an aligned one, and nothing around it is
+    written."""
+    case(f"split GEMMs into outputs off by {k}")
+
+    def off(M, N, dtype):
+        buf = torch.full((M * N + k + 8,), 7, dtype=dtype, device=dev)
+        return buf, buf[k:k + M * N].view(M, N)
+
+    A, B, bias = _operands(dev, 24, 504, 4352, 9)
+    buf, out = off(24, 504, torch.bfloat16)
+    assert torch.equal(ops.gemm_bias_act(A, B, bias, "silu", out=out), ops.gemm_bias_act(A, B, bias, "silu"))
+    assert (buf[:k] == 7).all() and (buf[k + out.numel():] == 7).all()
+    a8 = torch.randint(-128, 128, (72, 4368), device=dev, dtype=torch.int8)
+    b8 = torch.randint(-128, 128, (4368, 1104), device=dev, dtype=torch.int8)
+    buf, out = off(72, 1104, torch.float32)
+    assert torch.equal(ops.matmul_int8(a8, b8, 0.5, 0.25, bias=None, out=out), ops.matmul_int8(a8, b8, 0.5, 0.25))
+    assert (buf[:k] == 7).all() and (buf[k + out.numel():] == 7).all()
+
+
 def test_split_leaves_a_graphs_workspace(dev):
     """A graph captured from a call that keeps the stream's workspace replays
     between eager GEMMs that split K on that stream."""
