@@ -578,12 +578,12 @@ __global__ __launch_bounds__(256) void gemm_bf16_reduce_kernel(const float* __re
 // best of them on average.  Larger tiles move fewer bytes per output (per_k /
 // (bm bn) falls from 1.2 to 0.34 ps), smaller ones fill the chip sooner.
 constexpr TileModel kBf16Model = {
-    {{32, 64, 64, 5.0f, 0.0024f, 1.2f, 0.79f},
-     {64, 64, 64, 5.9f, 0.0025f, 0.4f, 1.1f},
-     {64, 128, 64, 2.0f, 0.0039f, 4.2f, 1.0f},
-     {128, 128, 64, 0.7f, 0.0062f, 6.0f, 1.0f},
-     {128, 256, 32, 0.5f, 0.0126f, 7.2f, 1.0f},
-     {256, 256, 32, 1.7f, 0.0222f, 8.1f, 1.0f}},
+    {{32, 64, 64, 128, 5.0f, 0.0024f, 1.2f, 0.79f},
+     {64, 64, 64, 256, 5.9f, 0.0025f, 0.4f, 1.1f},
+     {64, 128, 64, 512, 2.0f, 0.0039f, 4.2f, 1.0f},
+     {128, 128, 64, 512, 0.7f, 0.0062f, 6.0f, 1.0f},
+     {128, 256, 32, 512, 0.5f, 0.0126f, 7.2f, 1.0f},
+     {256, 256, 32, 512, 1.7f, 0.0222f, 8.1f, 1.0f}},
     0.0f, 1.75f, 0.19f, 1.2e-6f};
 
 template <class T>

@@ -78,6 +78,29 @@ bool f32_fits(const F32Gemm& g, int plan) {
     return std::max(span(g.ta, t.bm, g.M, g.lda), span(!g.tb, t.bn, g.N, g.ldb)) <= int64_t(1) << 32;
 }
 
+// One half of g's columns or, where there are more of them, its rows, whole
+// 128 x 128 tiles in the first.
+F32Gemm f32_half(F32Gemm g, bool second) {
+    const bool cols = g.N >= g.M;
+    const int at = (cols ? g.N : g.M) / 2 & ~127;
+    if (!second) {
+        (cols ? g.N : g.M) = at;
+        if (!cols) g.colsum = nullptr;  // the last row of the second
+        return g;
+    }
+    (cols ? g.N : g.M) -= at;
+    if (cols) {
+        g.B += g.tb ? at * g.ldb : at;
+        if (g.bias) g.bias += at;
+        if (g.colsum) g.colsum += at;
+    } else {
+        g.A += g.ta ? at : at * g.lda;
+    }
+    g.C += cols ? at : at * g.ldc;
+    if (g.mask) g.mask += cols ? at : at * g.ldm;
+    return g;
+}
+
 }  // namespace
 
 hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
@@ -112,6 +135,12 @@ hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hi
     // whole 16-byte pieces of the operands whose k is the outer dimension
     const int v = !f32_fits(g, plan) ? 0
                   : (!g.ta || (g.M - (g.colsum ? 1 : 0)) % 4 == 0) && (g.tb || g.N % 4 == 0) ? 4 : 1;
+    // the runtime takes fewer than 2^32 threads a launch
+    const F32Dims& t = kF32Dims[g.tb && plan == 3 ? 2 : plan];  // as launch_f32_tile
+    if (splits <= 1 && (((int64_t)g.M + t.bm - 1) / t.bm) * (((int64_t)g.N + t.bn - 1) / t.bn) >= int64_t(1) << 24) {
+        const hipError_t e = launch_f32_gemm(f32_half(g, false), 1, 0, nullptr, s);
+        return e != hipSuccess ? e : launch_f32_gemm(f32_half(g, true), 1, 0, nullptr, s);
+    }
     if (g.ta || g.tb) launch_f32_tile_trans(plan, v, g, splits, kc, chunk, part, s);
     else launch_f32_tile<false, false>(plan, v, g, splits, kc, chunk, part, s);
     if (part) {

@@ -382,7 +382,7 @@ __device__ __forceinline__ TileCoord tile_coord(int tiles_m, int tiles_n) {
 // sums and their reduction.  Each operand type has its own constants, fitted
 // to measured times (gemm_bf16.hip, matmul_int8.hip).
 struct TilePlan {
-    int bm, bn, bk;
+    int bm, bn, bk, threads;
     float base, per_k, round, shared;
 };
 struct TileModel {
@@ -399,6 +399,8 @@ inline TileChoice tile_choice(const TileModel& m, int M, int N, int K, bool may_
     for (int c = 0; c < 6; ++c) {
         const TilePlan& p = m.plan[c];
         const int64_t tiles = (((int64_t)M + p.bm - 1) / p.bm) * (((int64_t)N + p.bn - 1) / p.bn);
+        // the runtime takes fewer than 2^32 threads a launch (split ones are few)
+        if (tiles * p.threads >= int64_t(1) << 32 && c < 5) continue;
         const int slices = (K + p.bk - 1) / p.bk;
         for (int S : {1, 2, 3, 4, 6, 8}) {
             if (S > 1 && (!may_split || slices < 2 * S || tiles * S > 512 ||

@@ -114,12 +114,12 @@ __global__ __launch_bounds__(256) void int8_reduce_kernel(
 // As in gemm_bf16.hip; the fit is over 150 shapes (M 1-4096, N and K
 // 256-8192), its choice 3 % off the best on average.
 constexpr TileModel kInt8Model = {
-    {{32, 64, 128, 2.1f, 0.00079f, 4.0f, 0.56f},
-     {64, 64, 128, 4.5f, 0.00086f, 1.4f, 0.82f},
-     {64, 128, 128, 2.6f, 0.00135f, 3.4f, 1.0f},
-     {128, 128, 128, 1.5f, 0.0022f, 4.7f, 1.0f},
-     {128, 256, 64, 5.1f, 0.0042f, 2.7f, 1.0f},
-     {256, 256, 64, 10.4f, 0.0071f, 0.6f, 1.0f}},
+    {{32, 64, 128, 128, 2.1f, 0.00079f, 4.0f, 0.56f},
+     {64, 64, 128, 256, 4.5f, 0.00086f, 1.4f, 0.82f},
+     {64, 128, 128, 512, 2.6f, 0.00135f, 3.4f, 1.0f},
+     {128, 128, 128, 512, 1.5f, 0.0022f, 4.7f, 1.0f},
+     {128, 256, 64, 512, 5.1f, 0.0042f, 2.7f, 1.0f},
+     {256, 256, 64, 512, 10.4f, 0.0071f, 0.6f, 1.0f}},
     1.09f, 1.55f, 0.07f, 1.4e-6f};
 
 // ---------------------------------------------------------------------------

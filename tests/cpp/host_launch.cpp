@@ -173,6 +173,66 @@ static void stream_locks() {
     stub::on_synchronize = nullptr;
 }
 
+// Products of very many rows or columns are launched, in grids that the runtime
+// takes (below 2^32 threads): the stand-in refuses the others as it does.
+static void grid_limits() {
+    uint64_t outputs = 0;
+    stub::on_launch = [&](const stub::Launch& l) {
+        F32Launch f;
+        if (!f32_launch(l.kernel, &f)) return;
+        const auto g = l.arg<jh::F32Gemm>(0);
+        outputs += (uint64_t)g.M * g.N;
+        // the part of the product that a launch writes, and its operands' parts
+        const int64_t at = g.C - fake(2), m0 = at / g.ldc, n0 = at % g.ldc;
+        EXPECT(g.A - fake(0) == (g.ta ? m0 : m0 * g.lda) && g.B - fake(1) == (g.tb ? n0 * g.ldb : n0) &&
+                   (!g.bias || g.bias - fake(3) == n0),
+               "rows from %ld, columns from %ld: A + %ld, B + %ld", (long)m0, (long)n0, (long)(g.A - fake(0)),
+               (long)(g.B - fake(1)));
+    };
+    const int kTop = INT32_MAX;
+    for (int big : {1 << 22, (1 << 28) + 8, 1 << 29, (1 << 29) + 40, 1 << 30, kTop - 255}) {
+        for (int small : {8, 16, 64, 200, 520}) {
+            if ((int64_t)big * small > int64_t(1) << 37) continue;  // beyond a card's memory
+            for (int K : {8, 64}) {
+                EXPECT(jules_hip_gemm_bias_act(JH_BF16, JH_ACT_NONE, fake(0), fake(1), nullptr, fake(2), big, small, K,
+                                               nullptr) == JH_OK,
+                       "bf16 %d x %d x %d: %s", big, small, K, jules_hip_last_error());
+                EXPECT(jules_hip_gemm_bias_act(JH_BF16, JH_ACT_NONE, fake(0), fake(1), nullptr, fake(2), small, big, K,
+                                               nullptr) == JH_OK,
+                       "bf16 %d x %d x %d: %s", small, big, K, jules_hip_last_error());
+            }
+            if (big % 16 == 0 && small % 16 == 0)
+                EXPECT(jules_hip_matmul_int8(fake<int8_t>(0), fake<int8_t>(1), fake(2), big, small, 64, 1.0f, 1.0f,
+                                             nullptr, nullptr) == JH_OK,
+                       "int8 %d x %d: %s", big, small, jules_hip_last_error());
+        }
+        for (int n : {big, big + (big < kTop - 255 ? 0 : 255)})
+            for (int small : {1, 3, 33, 100})
+                for (int K : {1, 4, 64, 130}) {
+                    if ((int64_t)n * std::max(small, K) > int64_t(1) << 37) continue;
+                    outputs = 0;
+                    EXPECT(jules_hip_gemm_bias_act(JH_F32, JH_ACT_RELU, fake(0), fake(1), fake(3), fake(2), n, small, K,
+                                                   nullptr) == JH_OK,
+                           "fp32 %d x %d x %d: %s", n, small, K, jules_hip_last_error());
+                    EXPECT(jules_hip_gemm_bias_act(JH_F32, JH_ACT_RELU, fake(0), fake(1), fake(3), fake(2), small, n, K,
+                                                   nullptr) == JH_OK,
+                           "fp32 %d x %d x %d: %s", small, n, K, jules_hip_last_error());
+                    EXPECT(outputs == 2 * (uint64_t)n * small, "%d x %d: %llu outputs", n, small,
+                           (unsigned long long)outputs);
+                    outputs = 0;
+                    for (int t = 0; t < 4; ++t)
+                        for (int flip : {0, 1}) {
+                            const int M = flip ? small : n, N = flip ? n : small, ta = t & 1, tb = t >> 1;
+                            EXPECT(jules_hip_sgemm(ta, tb, M, N, K, 1.0f, fake(0), ta ? M : K, fake(1), tb ? K : N, 1.0f,
+                                                   fake(2), N, nullptr) == JH_OK,
+                                   "sgemm %d x %d x %d ta=%d tb=%d: %s", M, N, K, ta, tb, jules_hip_last_error());
+                        }
+                    EXPECT(outputs == 8 * (uint64_t)n * small, "sgemm %d x %d: %llu outputs", n, small,
+                           (unsigned long long)outputs);
+                }
+    }
+}
+
 static const struct {
     const char* name;
     void (*run)();
@@ -180,6 +240,7 @@ static const struct {
     {"f32_offsets", f32_offsets},
     {"graph_workspace", graph_workspace},
     {"stream_locks", stream_locks},
+    {"grid_limits", grid_limits},
 };
 
 int main(int argc, char** argv) {

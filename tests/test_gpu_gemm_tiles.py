@@ -57,6 +57,19 @@ def test_bf16_long_rows(dev, M, N, K):
     _check(ops.gemm_bias_act(A, B, None, "none"), A, B, None, "none")
 
 
+def test_bf16_very_many_rows(dev):
+    """2^30 rows: the smaller tiles would need more threads than a launch has."""
+    case("gemm bf16 2^30 x 8 x 8")
+    M, part = 1 << 30, 1 << 26
+    A = torch.empty((M, 8), dtype=torch.bfloat16, device=dev)
+    for i in range(0, M, part):
+        A[i:i + part] = torch.rand((part, 1), device=dev) - 0.5
+    B = torch.randn((8, 8), device=dev).bfloat16()
+    y = ops.gemm_bias_act(A, B, None, "none")
+    for i in range(0, M, part):
+        _check(y[i:i + part], A[i:i + part], B, None, "none")
+
+
 @pytest.mark.parametrize("K", [8, 40, 72, 4360])
 def test_bf16_k_tail_keeps_rows_apart(dev, K):
     """An infinity in one row of A may not reach the row before it through

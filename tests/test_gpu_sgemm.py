@@ -35,6 +35,11 @@ def _check_sgemm(dev, ta, tb, M, N, K, lda=None, ldb=None, ldc=None, alpha=1.0, 
     assert ((C.double() - ref).abs() <= (K + 2) * 2.0 ** -24 * terms).all()
 
 
+@pytest.mark.parametrize("ta,tb,M,N", [(0, 0, 1, (1 << 29) + 40), (1, 0, (1 << 29) + 41, 1), (0, 1, 1, (1 << 29) + 3)])
+def test_more_tiles_than_a_launch_has(dev, ta, tb, M, N):
+    _check_sgemm(dev, ta, tb, M, N, 3, alpha=0.5, beta=-1.0)
+
+
 @pytest.mark.parametrize("ta,tb,M,N,K,lda,ldb", [
     # slices that span 2^32 bytes of an operand: 64-bit offsets within a tile
     (0, 0, 33, 40, 70, 70, 17_200_000), (1, 0, 33, 40, 70, 17_200_000, 40),

@@ -23,7 +23,7 @@ def _binary():
     return BINARY
 
 
-@pytest.mark.parametrize("check", ["f32_offsets", "graph_workspace", "stream_locks"])
+@pytest.mark.parametrize("check", ["f32_offsets", "graph_workspace", "stream_locks", "grid_limits"])
 def test_host_launch(check, tmp_path):
     if subprocess.run(["g++", "--version"], capture_output=True).returncode != 0:
         pytest.skip("no g++")
