@@ -129,11 +129,15 @@ int flash_padded_dim(int D) { return D <= 64 ? 64 : 128; }
 hipError_t launch_flash_fwd_padded(int dtype, int causal, float scale, const void* Q, const void* K,
                                    const void* V, void* O, float* lse, int B, int H, int S, int D,
                                    hipStream_t s) {
-    // the workspace holds copies of K and V, so there O may lie over them
-    const char *o = static_cast<const char*>(O), *k = static_cast<const char*>(K), *v = static_cast<const char*>(V);
-    const int64_t bytes = (int64_t)B * H * S * D * 2;
-    const bool apart = (o + bytes <= k || k + bytes <= o) && (o + bytes <= v || v + bytes <= o);
-    if (apart && flash_fwd_takes_rows(dtype, S, D))
+    // the workspace holds copies of Q, K and V, so there O may lie over them;
+    // without it O may be Q itself (a workgroup writes the rows that it alone
+    // has read), but lies apart from Q otherwise and from K and V
+    const auto apart = [&](const void* in) {
+        const char *o = static_cast<const char*>(O), *i = static_cast<const char*>(in);
+        const int64_t bytes = (int64_t)B * H * S * D * 2;
+        return o + bytes <= i || i + bytes <= o;
+    };
+    if (flash_fwd_takes_rows(dtype, S, D) && (O == Q || apart(Q)) && apart(K) && apart(V))
         return launch_flash_fwd_rows(causal, scale, Q, K, V, O, lse, B, H, S, D, s);
     const int Dp = flash_padded_dim(D);
     const int64_t rows = (int64_t)B * H * S;

@@ -233,6 +233,26 @@ static void grid_limits() {
     }
 }
 
+// bf16 attention at a padded head dim reads its rows in place only where O lies
+// apart from them (or is Q); any other overlap goes through copies.
+static void overlapping_outputs() {
+    bool in_place = false;
+    stub::on_launch = [&](const stub::Launch& l) {
+        in_place |= l.kernel.find("flash_fwd_bf16_pad") != std::string::npos;
+    };
+    const int64_t bytes = 1 * 2 * 100 * 80 * 2;
+    for (int operand = 0; operand < 3; ++operand)
+        for (int64_t off : {-bytes - 16, -bytes, -bytes + 16, int64_t(-160), int64_t(-16), int64_t(0), int64_t(16),
+                            int64_t(160), bytes - 16, bytes, bytes + 16}) {
+            in_place = false;
+            EXPECT(jules_hip_flash_attn_fwd(JH_BF16, 0, 0.1f, fake(0), fake(1), fake(2), fake<char>(operand) + off,
+                                            nullptr, 1, 2, 100, 80, nullptr) == JH_OK,
+                   "%s", jules_hip_last_error());
+            const bool sound = off <= -bytes || off >= bytes || (operand == 0 && off == 0);
+            EXPECT(in_place == sound, "O at operand %d %+ld bytes", operand, (long)off);
+        }
+}
+
 static const struct {
     const char* name;
     void (*run)();
@@ -241,6 +261,7 @@ static const struct {
     {"graph_workspace", graph_workspace},
     {"stream_locks", stream_locks},
     {"grid_limits", grid_limits},
+    {"overlapping_outputs", overlapping_outputs},
 };
 
 int main(int argc, char** argv) {

@@ -172,3 +172,17 @@ def _fill(d, t):
         d.sizes[i] = t.shape[i]
         d.strides[i] = t.stride(i)
     d.dtype = {torch.float32: 0, torch.bfloat16: 1, torch.int8: 2}[t.dtype]
+
+
+@pytest.mark.parametrize("operand,off", [(0, 0), (0, 8), (0, -80), (1, 0), (2, 160)])
+def test_padded_output_over_an_input(dev, operand, off):
+    """bf16 at a padded head dim with O on one of its inputs, or shifted from
+    it by some elements, gives the bits of an O apart."""
+    B, H, S, D = 1, 3, 300, 80
+    case(f"flash bf16 {B}x{H}x{S}x{D}, O at input {operand} + {off}")
+    n = B * H * S * D
+    bufs = [torch.randn((n + 512,), device=dev).bfloat16() for _ in range(3)]
+    q, k, v = (b[256:256 + n].view(B, H, S, D) for b in bufs)
+    ref = ops.flash_attention(q, k, v)
+    out = bufs[operand][256 + off:256 + off + n].view(B, H, S, D)
+    assert torch.equal(ops.flash_attention(q, k, v, out=out), ref)

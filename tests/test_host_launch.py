@@ -23,7 +23,8 @@ def _binary():
     return BINARY
 
 
-@pytest.mark.parametrize("check", ["f32_offsets", "graph_workspace", "stream_locks", "grid_limits"])
+@pytest.mark.parametrize("check", ["f32_offsets", "graph_workspace", "stream_locks", "grid_limits",
+                                   "overlapping_outputs"])
 def test_host_launch(check, tmp_path):
     if subprocess.run(["g++", "--version"], capture_output=True).returncode != 0:
         pytest.skip("no g++")
