@@ -84,7 +84,7 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_bf16_kernel(
     const int wave = tid >> 6;
 
     // ---- XCD-aware tile order ----
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const int tiles_m = (M + (BM - 1)) / BM, tiles_n = (N + (BN - 1)) / BN;
     const int nblk = tiles_m * tiles_n;
     int t = blockIdx.x;
     if ((nblk & 7) == 0) t = (t & 7) * (nblk >> 3) + (t >> 3);
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_bf16_tile_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, const float* __restrict__ bias,
     uint16_t* __restrict__ C, float* __restrict__ part, int act, int M, int N, int K, int kc) {
     __shared__ __attribute__((aligned(1024))) uint8_t sm[T::LDS];
-    const TileCoord t = tile_coord<8>((M + T::BM - 1) / T::BM, (N + T::BN - 1) / T::BN);
+    const TileCoord t = tile_coord<8>((M + (T::BM - 1)) / T::BM, (N + (T::BN - 1)) / T::BN);
     const int m0 = t.tm * T::BM, n0 = t.tn * T::BN, kb = t.z * kc;
     typename T::Acc own[T::OWN];
     T::run(reinterpret_cast<const uint8_t*>(A + (int64_t)m0 * K + kb), (int64_t)K * 2, min(T::BM, M - m0),
@@ -589,7 +589,7 @@ constexpr TileModel kBf16Model = {
 template <class T>
 void launch_tile(int act, const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C, float* part,
                  int M, int N, int K, const TileChoice& c, hipStream_t s) {
-    const int64_t tiles = ((int64_t)(M + T::BM - 1) / T::BM) * ((N + T::BN - 1) / T::BN);
+    const int64_t tiles = ((int64_t)(M + (T::BM - 1)) / T::BM) * ((N + (T::BN - 1)) / T::BN);
     hipLaunchKernelGGL(gemm_bf16_tile_kernel<T>, dim3((unsigned)(tiles * c.splits)), dim3(T::THREADS), 0, s,
                        A, B, bias, C, part, act, M, N, K, c.kc);
 }
@@ -600,7 +600,7 @@ hipError_t launch_gemm_bf16(int act, const uint16_t* A, const uint16_t* B, const
                             uint16_t* C, int M, int N, int K, hipStream_t s) {
     // byte offsets within a tile (256 rows of A, 64 of B) below 2^31
     if (K >= (1 << 22) || N >= (1 << 24)) {
-        const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+        const int tiles = ((M + (BM - 1)) / BM) * ((N + (BN - 1)) / BN);
         JH_DISPATCH_ACT(act, ACT, hipLaunchKernelGGL(gemm_bf16_kernel<ACT>, dim3(tiles), dim3(THREADS), 0, s,
                                                      A, B, bias, C, M, N, K));
         return hipGetLastError();

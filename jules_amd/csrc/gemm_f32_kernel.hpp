@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Gemm g, int kc
     using T = F32Tile<CF::MF, CF::MT, CF::NT, CF::BK, CF::PF, TA, TB, V, FOLD>;
     constexpr bool ACTS = !TA && !TB;
     __shared__ __attribute__((aligned(16))) float sm[2 * T::STAGE];
-    const TileCoord t = tile_coord<8>((g.M + T::BM - 1) / T::BM, (g.N + T::BN - 1) / T::BN);
+    const TileCoord t = tile_coord<8>((g.M + (T::BM - 1)) / T::BM, (g.N + (T::BN - 1)) / T::BN);
     const int m0 = t.tm * T::BM, n0 = t.tn * T::BN, kb = t.z * kc;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int mw = m0 + (wave >> 1) * CF::MT * CF::MF, nw = n0 + (wave & 1) * CF::NT * CF::MF + lane % CF::MF;

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(T::THREADS) void int8_tile_kernel(
     const float* __restrict__ row_scale, const float* __restrict__ col_scale,
     const float* __restrict__ bias) {
     __shared__ __attribute__((aligned(1024))) uint8_t sm[T::LDS];
-    const TileCoord t = tile_coord<8>((M + T::BM - 1) / T::BM, (N + T::BN - 1) / T::BN);
+    const TileCoord t = tile_coord<8>((M + (T::BM - 1)) / T::BM, (N + (T::BN - 1)) / T::BN);
     const int m0 = t.tm * T::BM, n0 = t.tn * T::BN, kb = t.z * kc;
     typename T::Acc own[T::OWN];
     T::run(reinterpret_cast<const uint8_t*>(A + (int64_t)m0 * K + kb), K, min(T::BM, M - m0),

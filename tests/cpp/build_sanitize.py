@@ -1,10 +1,15 @@
-"""Build tests/cpp/host_sanitize and tests/cpp/host_launch: the library's host
-sources (capi.cpp, kernel_shims.cpp, pjrt.cpp, cblas_sgemm.cpp) and a driver
-compiled by g++ with AddressSanitizer and UndefinedBehaviorSanitizer, linked
-with the library's compiled .hip objects (device code and launchers, built by
-jules_amd/build.py into _build/, not sanitized).  host_sanitize runs on the HIP
-runtime, host_launch on the stand-in hip_stub.cpp.  Host code only: no GPU code
-is built with a sanitizer."""
+"""Build the CPU suite's programs with AddressSanitizer and
+UndefinedBehaviorSanitizer.  Host code only: no GPU code is built with a
+sanitizer.
+
+tests/cpp/host_sanitize: the library's host sources (capi.cpp,
+kernel_shims.cpp, pjrt.cpp, cblas_sgemm.cpp) and a driver compiled by g++,
+linked with the library's compiled .hip objects (device code and launchers,
+built by jules_amd/build.py into _build/, not sanitized) and the HIP runtime.
+
+tests/cpp/host_launch: those sources, the host side of every .hip source
+(launchers and kernel stubs, without device code) and a driver compiled by
+ROCm's clang, linked with hip_stub.cpp in the place of the HIP runtime."""
 import concurrent.futures as cf
 import os
 import subprocess
@@ -16,6 +21,7 @@ CSRC = os.path.join(ROOT, "jules_amd", "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 OBJDIR = os.path.join(ROOT, "_build")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+CLANG = f"{ROCM}/lib/llvm/bin/clang++"
 BINARY = os.path.join(HERE, "host_sanitize")
 LAUNCH_BINARY = os.path.join(HERE, "host_launch")
 HOST_SOURCES = ["capi.cpp", "kernel_shims.cpp", "pjrt.cpp", "cblas_sgemm.cpp"]
@@ -42,23 +48,32 @@ def build(verbose=False):
     if missing:
         raise RuntimeError(f"library objects missing (run jules_amd/build.py first): {missing}")
     host = [os.path.join(CSRC, s) for s in HOST_SOURCES]
-    drivers = [os.path.join(HERE, s) for s in ("host_sanitize.cpp", "host_launch.cpp", "hip_stub.cpp")]
+    hips = [os.path.join(CSRC, s) for s in lib_build.SOURCES if s.endswith(".hip")]
+    cpp = [os.path.join(HERE, s) for s in ("host_launch.cpp", "hip_stub.cpp")]
 
-    def compile_one(src):
+    def gxx(src):
         obj = os.path.join(OBJDIR, "san_" + os.path.basename(src) + ".o")
         _run(["g++", *CXXFLAGS, *SANITIZE, "-c", src, "-o", obj], verbose)
         return obj
 
-    def link(objs, libs, out):
+    def clang(src):
+        obj = os.path.join(OBJDIR, "stub_" + os.path.basename(src) + ".o")
+        hip = [f"--offload-arch={lib_build.ARCH}", "--cuda-host-only", "-fuse-cuid=none", "-Wno-unused-function", "-x", "hip"]
+        _run([CLANG, *CXXFLAGS, *SANITIZE, *(hip if src.endswith(".hip") else []), "-c", src, "-o", obj], verbose)
+        return obj
+
+    def link(cxx, objs, libs, out):
         tmp = out + ".tmp"
-        _run(["g++", *SANITIZE, *objs, *dev_objs, *libs, "-o", tmp], verbose)
+        _run([cxx, *SANITIZE, *objs, *libs, "-o", tmp], verbose)
         os.replace(tmp, out)
 
-    with cf.ThreadPoolExecutor(max_workers=7) as ex:
-        objs = list(ex.map(compile_one, host + drivers))
-    host_objs, (sanitize, launch, hip_stub) = objs[:len(host)], objs[len(host):]
-    link([*host_objs, sanitize], [f"-L{ROCM}/lib", "-lamdhip64", f"-Wl,-rpath,{ROCM}/lib"], BINARY)
-    link([*host_objs, launch, hip_stub], ["-lpthread"], LAUNCH_BINARY)
+    with cf.ThreadPoolExecutor(max_workers=8) as ex:
+        san = ex.map(gxx, [*host, os.path.join(HERE, "host_sanitize.cpp")])
+        stub = ex.map(clang, [*hips, *host, *cpp])
+        san, stub = list(san), list(stub)
+    link("g++", [*san, *dev_objs], [f"-L{ROCM}/lib", "-lamdhip64", f"-Wl,-rpath,{ROCM}/lib"], BINARY)
+    # the objects share the name of the device code that they are without
+    link(CLANG, stub, ["-Wl,--allow-multiple-definition", "-lpthread"], LAUNCH_BINARY)
     return BINARY
 
 

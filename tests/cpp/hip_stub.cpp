@@ -63,6 +63,8 @@ using namespace stub;
 
 extern "C" {
 
+extern const char __hip_fatbin[] = "";  // where the device code would be
+
 void** __hipRegisterFatBinary(const void*) {
     static void* handle;
     return &handle;

@@ -1,7 +1,7 @@
 // host_launch.cpp - what the library's entry points launch, and what they do
-// with the workspaces they hold, checked without a GPU: the library's objects
-// linked against hip_stub.cpp, its host sources built with AddressSanitizer and
-// UndefinedBehaviorSanitizer.  `host_launch <check>` runs one check and prints
+// with the workspaces they hold, checked without a GPU: the library's host code,
+// launchers included, built with AddressSanitizer and UndefinedBehaviorSanitizer
+// and linked against hip_stub.cpp.  `host_launch <check>` runs one check and prints
 // "<check> ok"; run by tests/test_host_launch.py.
 #include <algorithm>
 #include <chrono>

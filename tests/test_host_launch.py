@@ -1,8 +1,8 @@
 """What the library's entry points launch, and how they hold their workspaces,
 checked without a GPU: tests/cpp/host_launch (built by
-tests/cpp/build_sanitize.py) links the library's objects against a stand-in for
-the HIP host calls that records launches, with the host sources under
-AddressSanitizer and UndefinedBehaviorSanitizer.  Each check says in
+tests/cpp/build_sanitize.py) links the library's host code, launchers included,
+under AddressSanitizer and UndefinedBehaviorSanitizer against a stand-in for the
+HIP host calls that records launches.  Each check says in
 tests/cpp/host_launch.cpp what it holds the library to."""
 import os
 import subprocess
