@@ -11,9 +11,11 @@
 #include <cstring>
 #include <future>
 #include <string>
+#include <vector>
 
 #include "hip_stub.hpp"
 #include "jules_hip.h"
+#include "jules_hip_kernel.hpp"
 #include "launch.hpp"
 
 static int g_fail = 0;
@@ -253,6 +255,44 @@ static void overlapping_outputs() {
         }
 }
 
+// The C++ training step and forward on host buffers: staged, launched, copied
+// back and given back, at shapes with and without ranges of K, and after errors.
+static void mlp_wrappers() {
+    using namespace jules::kernel;
+    int launches = 0;
+    stub::on_launch = [&](const stub::Launch&) { ++launches; };
+    const auto before = stub::allocations();
+    {
+        ExecutionArena arena;
+        TilePlanner planner;
+        const auto with_arena = stub::allocations();
+        for (int M : {0, 1, 19, 64, 300})
+            for (int K1 : {1, 23, 784})
+                for (int N1 : {1, 17, 256})
+                    for (int N2 : {1, 5, 10}) {
+                        std::vector<float> X(M * K1), W1(K1 * N1), b1(N1), W2(N1 * N2), b2(N2), out(M * N2);
+                        std::vector<float> dW1(K1 * N1), db1(N1), dW2(N1 * N2), db2(N2), dX(M * K1);
+                        std::vector<int32_t> t(M);
+                        for (float* dx : {dX.data(), (float*)nullptr}) {
+                            launches = 0;
+                            const auto r = interleavedMLPForwardBackward(
+                                X.data(), W1.data(), b1.data(), W2.data(), b2.data(), t.data(), out.data(), dW1.data(),
+                                db1.data(), dW2.data(), db2.data(), dx, M, K1, N1, N2, arena, planner);
+                            EXPECT(lastStatus() == JH_OK && launches >= 5 && r.grads.dX == dx, "%d x %d x %d x %d: %s", M,
+                                   K1, N1, N2, lastError());
+                        }
+                        const MLPParams p{W1.data(), b1.data(), W2.data(), b2.data(), M, K1, N1, N2};
+                        fusedMLPForward(out.data(), X.data(), p, arena, planner);
+                        EXPECT(lastStatus() == JH_OK, "%s", lastError());
+                        const MLPParams bad{W1.data(), b1.data(), W2.data(), b2.data(), M, 0, N1, N2};
+                        fusedMLPForward(out.data(), X.data(), bad, arena, planner);
+                        EXPECT(lastStatus() == JH_ERR_SHAPE, "%d", lastStatus());
+                    }
+        EXPECT(stub::allocations() == with_arena, "%zu device buffers are left", stub::allocations().size());
+    }
+    EXPECT(stub::allocations() == before, "%zu device buffers are left", stub::allocations().size());
+}
+
 static const struct {
     const char* name;
     void (*run)();
@@ -262,6 +302,7 @@ static const struct {
     {"stream_locks", stream_locks},
     {"grid_limits", grid_limits},
     {"overlapping_outputs", overlapping_outputs},
+    {"mlp_wrappers", mlp_wrappers},
 };
 
 int main(int argc, char** argv) {

@@ -24,7 +24,7 @@ def _binary():
 
 
 @pytest.mark.parametrize("check", ["f32_offsets", "graph_workspace", "stream_locks", "grid_limits",
-                                   "overlapping_outputs"])
+                                   "overlapping_outputs", "mlp_wrappers"])
 def test_host_launch(check, tmp_path):
     if subprocess.run(["g++", "--version"], capture_output=True).returncode != 0:
         pytest.skip("no g++")
