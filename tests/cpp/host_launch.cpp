@@ -10,6 +10,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <future>
+#include <iostream>
+#include <sstream>
 #include <string>
 #include <vector>
 
@@ -293,6 +295,49 @@ static void mlp_wrappers() {
     EXPECT(stub::allocations() == before, "%zu device buffers are left", stub::allocations().size());
 }
 
+// Names what each product read from stdin launches: "f32 M N K", "bf16 M N K",
+// "int8 M N K" or "sgemm ta tb M N K", one a line.  The fp32 tile as BM x BN x BK
+// and its variant, with "folded" where it adds ranges of K itself; "whole" for
+// the kernels of whole 256 x 256 tiles; "split" where a reduction follows.
+static void tiles() {
+    std::string line, said;
+    stub::on_launch = [&](const stub::Launch& l) {
+        F32Launch f;
+        int bm, bn;
+        const size_t cfg = l.kernel.find("TileCfg<");
+        char s[80];
+        if (f32_launch(l.kernel, &f))
+            std::snprintf(s, sizeof s, "%dx%dx%d v%d%s", 2 * f.mt * f.mf, 2 * f.nt * f.mf, f.bk, f.v,
+                          f.fold ? " folded" : "");
+        else if (cfg != std::string::npos && std::sscanf(l.kernel.c_str() + cfg, "TileCfg<jh::%*[A-Za-z0-9], %d, %d", &bm, &bn) == 2)
+            std::snprintf(s, sizeof s, "%dx%d", bm, bn);
+        else if (l.kernel.find("_dma_kernel") != std::string::npos)
+            std::snprintf(s, sizeof s, "whole");
+        else if (l.kernel.find("_reduce_kernel") != std::string::npos)
+            std::snprintf(s, sizeof s, " split");
+        else
+            std::snprintf(s, sizeof s, "%s", l.kernel.c_str());
+        said += s;
+    };
+    while (std::getline(std::cin, line)) {
+        std::istringstream in(line);
+        std::string kind;
+        int ta = 0, tb = 0, M = 0, N = 0, K = 0, st;
+        in >> kind;
+        if (kind == "sgemm") in >> ta >> tb;
+        in >> M >> N >> K;
+        said.clear();
+        if (kind == "sgemm")
+            st = jules_hip_sgemm(ta, tb, M, N, K, 1.0f, fake(0), ta ? M : K, fake(1), tb ? K : N, 1.0f, fake(2), N, nullptr);
+        else if (kind == "int8")
+            st = jules_hip_matmul_int8(fake<int8_t>(0), fake<int8_t>(1), fake(2), M, N, K, 1.0f, 1.0f, nullptr, nullptr);
+        else
+            st = jules_hip_gemm_bias_act(kind == "bf16" ? JH_BF16 : JH_F32, JH_ACT_NONE, fake(0), fake(1), nullptr,
+                                         fake(2), M, N, K, nullptr);
+        std::printf("%s: %s\n", line.c_str(), st == JH_OK ? said.c_str() : jules_hip_last_error());
+    }
+}
+
 static const struct {
     const char* name;
     void (*run)();
@@ -303,6 +348,7 @@ static const struct {
     {"grid_limits", grid_limits},
     {"overlapping_outputs", overlapping_outputs},
     {"mlp_wrappers", mlp_wrappers},
+    {"tiles", tiles},
 };
 
 int main(int argc, char** argv) {

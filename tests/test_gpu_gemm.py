@@ -140,29 +140,44 @@ def test_activation_kernel_bit_exact(dev):
     np.testing.assert_array_equal(to_np(ops.activation(dx, "gelu")), po.fused_gelu(x))
 
 
-def _special(seed, shape):
+def _special(seed, shape, last_is_k):
     """Values whose products and sums meet every corner of an fma: signed
-    zeros, ones, subnormals, numbers whose products are subnormal or overflow."""
+    zeros, ones, subnormals, numbers whose products are subnormal or overflow;
+    and, in about one row or column of 16 only (they end every sum they meet),
+    infinities and NaNs."""
     v = I.uniform(seed, 0, shape, -1, 1)
     pool = np.array([0.0, -0.0, 1.0, -1.0, 1e-40, -3e-39, 1e-25, -1e-22, 1e25, -3e19], np.float32)
     pick = (I.uniform(seed, 1, shape, 0, 16)).astype(np.int64)
-    return np.where(pick < len(pool), pool[np.minimum(pick, len(pool) - 1)], v).astype(np.float32)
+    v = np.where(pick < len(pool), pool[np.minimum(pick, len(pool) - 1)], v).astype(np.float32)
+    k_axis = 1 if last_is_k else 0
+    lines = np.flatnonzero(I.uniform(seed, 2, (shape[1 - k_axis],), 0, 16) < 1)
+    for n, line in enumerate(lines):
+        k = int(I.uniform(seed, 3 + n, (1,), 0, shape[k_axis])[0])
+        v[(line, k) if last_is_k else (k, line)] = (np.inf, -np.inf, np.nan)[n % 3]
+    return v
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (33, 48, 65), (32, 32, 64), (1, 16, 3),             # 32 x 32 tiles, K tails, 4-byte and 16-byte loads
-    (1025, 1040, 33), (1024, 1008, 36),                 # 64 x 64
-    (1000, 2064, 70), (1024, 2048, 20),                 # 64 x 128
-    (2049, 4112, 17), (2048, 4096, 48),                 # 128 x 128
-])
-def test_f32_tiles_bit_exact(dev, M, N, K):
+# the tile that each shape takes, and its loads of an operand whose k is the
+# outer dimension: 16 bytes (v4) or 4 (v1); held by tests/test_tile_coverage.py
+F32_TILES = [
+    (33, 48, 65, "32x32x64 v4"), (32, 32, 64, "32x32x64 v4"), (1, 16, 3, "32x32x64 v4"), (41, 45, 19, "32x32x64 v1"),
+    (70, 52, 700, "32x32x128 v4"), (31, 33, 257, "32x32x128 v1"),
+    (1024, 1008, 36, "64x64x32 v4"), (1000, 2064, 70, "64x64x32 v4"), (1001, 1021, 35, "64x64x32 v1"),
+    (1025, 1040, 33, "64x128x16 v4"), (1024, 2048, 20, "64x128x16 v4"), (2049, 4112, 17, "64x128x16 v4"),
+    (2048, 4096, 48, "64x128x16 v4"), (1001, 2041, 21, "64x128x16 v1"),
+    (2040, 4092, 72, "128x128x16 v4"), (2041, 4089, 69, "128x128x16 v1"),
+]
+
+
+@pytest.mark.parametrize("M,N,K,tile", F32_TILES)
+def test_f32_tiles_bit_exact(dev, M, N, K, tile):
     """Every tile at its edges is the oracle's fma chain bit for bit, on
     ordinary values and on those where a different chain or a k past the end
-    would show (a -0 sum, a subnormal, an overflow)."""
+    would show (a -0 sum, a subnormal, an overflow, an infinity, a NaN)."""
     case(f"gemm f32 tiles {M}x{N}x{K}")
     A, B, _ = I.gemm_inputs(M, N, K, "f32", seed=M + N + K)
     np.testing.assert_array_equal(_gemm_f32(dev, A, B, None, "none"), po.tiled_matmul_act(A, B, "none"))
-    A, B = _special(M, (M, K)), _special(N + 7, (K, N))
+    A, B = _special(M, (M, K), True), _special(N + 7, (K, N), False)
     y, r = _gemm_f32(dev, A, B, None, "none"), po.tiled_matmul_act(A, B, "none")
     same = (y.view(np.int32) == r.view(np.int32)) | (np.isnan(y) & np.isnan(r))
     assert same.all(), f"{(~same).sum()} of {same.size} differ"

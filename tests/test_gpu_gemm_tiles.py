@@ -31,17 +31,23 @@ def _check(y, A, B, bias, act):
     assert ((y.double() - ref).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (8, 8, 8), (8, 72, 16), (32, 64, 64), (40, 264, 136),   # 32 x 64 tiles
-    (24, 504, 4352),                                        # the same, K split in 8
-    (72, 1096, 4360),                                       # 64 x 64, split in 6, ragged last range
-    (1016, 384, 4544),                                      # 64 x 128, two k groups, split in 4
-    (600, 2056, 1032), (1272, 2304, 520),                   # 64 x 128 and 128 x 128
-    (1000, 5000, 328),                                      # 128 x 256
-    (1288, 6152, 776), (1376, 3120, 4888),                  # 256 x 256, whole and split in 3
-])
+# the tile that each shape takes ("whole": the kernel of whole 256x256 tiles),
+# and whether K is split; held by tests/test_tile_coverage.py
+BF16_TILES = [
+    (8, 8, 8, "32x64"), (8, 72, 16, "32x64"), (32, 64, 64, "32x64"), (40, 264, 136, "32x64"),
+    (24, 504, 4352, "32x64 split"),
+    (464, 1240, 80, "64x64"), (72, 1096, 4360, "64x64 split"),           # the last range is ragged
+    (600, 2056, 1032, "64x128"), (1016, 384, 4544, "64x128 split"),
+    (1272, 2304, 520, "128x128"), (536, 1968, 3736, "128x128 split"),
+    (1000, 5000, 328, "128x256"), (512, 4224, 6984, "128x256 split"),
+    (1288, 6152, 776, "256x256"), (1376, 3120, 4888, "256x256 split"),
+    (3840, 2304, 32, "whole"), (3840, 2304, 96, "whole"), (3072, 3072, 160, "whole"),  # 1, 3 and 5 slices
+]
+
+
+@pytest.mark.parametrize("M,N,K,tile", BF16_TILES)
 @pytest.mark.parametrize("act", ["none", "silu"])
-def test_bf16_tiles(dev, M, N, K, act):
+def test_bf16_tiles(dev, M, N, K, tile, act):
     case(f"gemm bf16 tiles {M}x{N}x{K} {act}")
     A, B, bias = _operands(dev, M, N, K, M + N + K)
     bias = bias if act == "silu" else None
@@ -156,16 +162,22 @@ def _int8_ref(A, B, rs, cs, bias):
     return z if bias is None else z + bias
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (17, 16, 16), (40, 272, 144),                       # 32 x 64 tiles
-    (39, 2960, 8128), (72, 1104, 4368),                 # 64 x 64, K split, ragged last range
-    (645, 688, 6768), (540, 4112, 1040),                # 64 x 128, split in 3 and whole
-    (222, 5264, 7328), (1000, 2064, 912),               # 128 x 128
-    (796, 5616, 6864),                                  # 128 x 256
-    (1304, 6160, 784), (768, 1280, 320),                # 256 x 256; whole tiles
-    (1, 1, 1), (3, 65, 17), (64, 64, 64 - 1), (65, 130, 129), (33, 1000, 255),  # rows of any length
-])
-def test_int8_tiles(dev, M, N, K):
+INT8_TILES = [
+    (23, 992, 2816, "32x64"), (22, 2832, 6720, "32x64 split"),
+    (17, 16, 16, "64x64"), (40, 272, 144, "64x64"), (768, 1280, 320, "64x64"), (645, 688, 6768, "64x64"),
+    (39, 2960, 8128, "64x64 split"), (72, 1104, 4368, "64x64 split"),    # the last range is ragged
+    (222, 5264, 7328, "64x128"), (39, 5952, 6768, "64x128 split"),
+    (540, 4112, 1040, "128x128"), (1000, 2064, 912, "128x128"),
+    (796, 5616, 6864, "128x256"),
+    (1304, 6160, 784, "256x256"),
+    (2816, 3072, 128, "whole"), (2304, 3840, 320, "whole"),
+]
+# rows of any length: a kernel of their own
+INT8_ROWS = [(1, 1, 1, ""), (3, 65, 17, ""), (64, 64, 64 - 1, ""), (65, 130, 129, ""), (33, 1000, 255, "")]
+
+
+@pytest.mark.parametrize("M,N,K,tile", INT8_TILES + INT8_ROWS)
+def test_int8_tiles(dev, M, N, K, tile):
     case(f"int8 tiles {M}x{N}x{K}")
     g = torch.Generator(device=dev).manual_seed(M + N + K)
     A = torch.randint(-128, 128, (M, K), generator=g, device=dev, dtype=torch.int8)

@@ -51,3 +51,32 @@ def test_more_tiles_than_a_launch_has(dev, ta, tb, M, N):
 ])
 def test_wide_leading_dimensions(dev, ta, tb, M, N, K, lda, ldb):
     _check_sgemm(dev, ta, tb, M, N, K, lda, ldb)
+
+
+# every tile of each orientation (a transposed B has none of 128x128), with
+# 16-byte and 4-byte loads where an operand's k is the outer dimension; held by
+# tests/test_tile_coverage.py
+SGEMM_TILES = [
+    (0, 0, 41, 45, 19, "32x32x64 v1"), (0, 0, 1001, 1021, 35, "64x64x32 v1"), (0, 0, 1024, 2048, 20, "64x128x16 v4"),
+    (0, 0, 2040, 4092, 72, "128x128x16 v4"), (0, 0, 2041, 4089, 69, "128x128x16 v1"),
+    (0, 0, 70, 50, 700, "32x32x128 v1 folded"), (0, 0, 130, 260, 2050, "64x128x16 v4 split"),
+    (1, 0, 33, 48, 65, "32x32x64 v1"), (1, 0, 1024, 1008, 36, "64x64x32 v4"), (1, 0, 1001, 1021, 35, "64x64x32 v1"),
+    (1, 0, 1024, 2048, 20, "64x128x16 v4"), (1, 0, 1001, 2041, 21, "64x128x16 v1"),
+    (1, 0, 2040, 4092, 72, "128x128x16 v4"), (1, 0, 2041, 4089, 69, "128x128x16 v1"),
+    (1, 0, 70, 50, 700, "32x32x128 v1 folded"), (1, 0, 300, 300, 300, "32x32x128 v4 folded"),
+    (1, 0, 130, 260, 2050, "64x128x16 v1 split"),
+    (0, 1, 33, 48, 65, "32x32x64 v4"), (0, 1, 1001, 1021, 35, "64x64x32 v4"), (0, 1, 1001, 2041, 21, "64x128x16 v4"),
+    (0, 1, 2041, 4089, 69, "64x128x16 v4"), (0, 1, 70, 50, 700, "32x32x128 v4 folded"),
+    (0, 1, 130, 260, 2050, "64x128x16 v4 split"),
+    (1, 1, 33, 48, 65, "32x32x64 v1"), (1, 1, 1024, 1008, 36, "64x64x32 v4"), (1, 1, 1001, 1021, 35, "64x64x32 v1"),
+    (1, 1, 1024, 2048, 20, "64x128x16 v4"), (1, 1, 1001, 2041, 21, "64x128x16 v1"),
+    (1, 1, 70, 50, 700, "32x32x128 v1 folded"), (1, 1, 300, 300, 300, "32x32x128 v4 folded"),
+    (1, 1, 130, 260, 2050, "64x128x16 v1 split"), (1, 1, 64, 64, 4096, "32x32x64 v4 split"),
+]
+
+
+@pytest.mark.parametrize("ta,tb,M,N,K,tile", SGEMM_TILES)
+def test_sgemm_tiles(dev, ta, tb, M, N, K, tile):
+    """Padded leading dimensions, alpha and beta."""
+    ar, br = (M if ta else K) + 3, (K if tb else N) + 5
+    _check_sgemm(dev, ta, tb, M, N, K, ar, br, N + 2, alpha=0.75, beta=-1.25)
