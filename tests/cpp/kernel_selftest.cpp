@@ -31,6 +31,7 @@ static double max_rel(const std::vector<float>& y, const std::vector<double>& r)
 }
 
 int main() {
+    std::setvbuf(stdout, nullptr, _IONBF, 0);
     const int M = 19, K1 = 23, N1 = 17, N2 = 5;
     unsigned s = 12345u;
     auto rnd = [&]() {
@@ -101,6 +102,7 @@ int main() {
     CHECK(max_rel(dW2, rdW2) < 1e-5);
     CHECK(max_rel(db2, rdb2) < 1e-5);
     CHECK(max_rel(dX, rdX) < 1e-5);
+    std::printf("training step ok\n");
 
     // without dX, and a shape error
     r = interleavedMLPForwardBackward(X.data(), W1.data(), b1.data(), W2.data(), b2.data(), t.data(),
@@ -111,6 +113,8 @@ int main() {
                                       out.data(), dW1.data(), db1.data(), dW2.data(), db2.data(),
                                       nullptr, M, K1, 0, N2, arena, planner);
     CHECK(lastStatus() == JH_ERR_SHAPE && std::isnan(r.loss));
+
+    std::printf("training step without dX and its shape error ok\n");
 
     // fusedMLPForward (FusedKernels.h:659): the same forward, no loss
     std::vector<float> fwd(M * N2, -7.0f);
