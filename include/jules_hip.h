@@ -95,7 +95,10 @@ const char* jules_hip_last_error(void);
  *   vector path covers the column (N and tile_n multiples of 16).
  * dtype JH_BF16: A, B, C bf16; fp32 accumulation on MFMA; bias fp32;
  *   epilogue in fp32, C rounded to bf16.  M, N, K must be multiples of 8
- *   (16-byte rows); other shapes return JH_ERR_UNSUPPORTED.
+ *   (16-byte rows); other shapes return JH_ERR_UNSUPPORTED.  Where the output
+ *   tiles would not fill the chip, K is summed in ranges whose fp32 sums are
+ *   added in order, but not under graph capture or on hipStreamPerThread: there
+ *   C may differ by that order of summation.  Either is deterministic.
  * bias may be NULL.  K = 0 gives act(bias) (act(0) without bias).
  */
 int jules_hip_gemm_bias_act(int dtype, int act, const void* A, const void* B,
@@ -103,8 +106,8 @@ int jules_hip_gemm_bias_act(int dtype, int act, const void* A, const void* B,
                             void* stream);
 
 /* ---- GEMM tile table -------------------------------------------------------
- * out[4] = {entry, tile_m, tile_n, tile_k} of the table that plans
- * jules_hip_gemm_bias_act for this dtype and shape (needs no GPU).
+ * out[4] = {entry, tile_m, tile_n, tile_k} of the table that classifies the
+ * shapes of jules_hip_gemm_bias_act for this dtype (needs no GPU).
  * Entries: 0/1 fp32 by rows, 1/2 rows per wave (4 or 8 rows x 64 columns, all
  * of K, K <= 2048), 2/3 fp32 32x32 / 64x64 tiles with 32-deep K slices, 4 bf16
  * 256x256 tiles with 32-deep LDS-DMA stages, 5 the other bf16 shapes.  An

@@ -55,8 +55,11 @@ constexpr int BOWN = BW * 32;    // keys (dK/dV pass) or queries (dQ pass) a wor
 // heads (head = 8*j + xcd) two at a time with their blocks interleaved,
 // longest first, so the heads' operands stay in that XCD's L2 and the CUs
 // that finish early take the next long blocks.  (The forward interleaves four
-// heads, which gives the XCD's four shader engines equal work there; with two
-// workgroups per CU here, four heads measured the same as two.)
+// heads, which gives the XCD's four shader engines equal work there.  With two
+// workgroups per CU here, four heads measured the same as two at 256 heads of
+// 32 blocks; at 64 heads of 16 blocks the long blocks of the last two heads
+// start late, and list scheduling of this order ends at 1.47 times the balanced
+// time, of four heads at 1.00.)
 __device__ __forceinline__ void bwd_block(int nblk, int* bh, int* rank) {
     const int b = blockIdx.x, BH = gridDim.x / nblk;
     if ((BH & 7) == 0) {

@@ -501,9 +501,12 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_bf16_dma_kernel(
 // fp32 partial sums to part[z][M][N], which the reduce kernel adds in range
 // order before bias and activation.
 //
-// What bounds it (328 x 4096 x 4096): the copies of the operand tiles from L2
-// to LDS, (1/BM + 1/BN) of K per output.  64 x 128 tiles move 302 MB in 22.7
-// us; 256 x 256 tiles move a third of that but only fill 32 CUs, which took the
+// What bounds it (328 x 4096 x 4096, 64 x 128 tiles on 192 CUs, 22.5 us): no
+// one unit.  By counters the MFMAs are busy 17 % of the time and LDS reads 13
+// %, without bank conflicts; a CU copies 28 and reads 57 bytes of LDS a clock.
+// A slice takes about 880 clocks, the rest of which is its chain of copy,
+// barrier, reads and MFMAs; which link of it binds has not been measured.  256
+// x 256 tiles copy a third of the bytes but fill 32 CUs only, which took the
 // register-staged kernel 181 us.  The tile is as large as still fills the chip.
 // ---------------------------------------------------------------------------
 template <class T>
@@ -573,9 +576,11 @@ __global__ __launch_bounds__(256) void gemm_bf16_reduce_kernel(const float* __re
 }
 
 // The tile kernel's tiles, with the waves, slice bytes and ring depth measured
-// best for each.  The model is a least-squares fit to 250 shapes (M 24-4096, N
-// and K 256-8192) timed at every tile and split: its choice is 2 % off the
-// best of them on average.  Larger tiles move fewer bytes per output (per_k /
+// best for each.  The model was fitted to times of shapes with M 24-4096, N and
+// K 256-8192.  Over 120 shapes of these ranges, each timed at every tile
+// and split on operands that change from launch to launch, its choice is 7 %
+// off the best on average, 1 % in the middle, 40 % at worst (small M x N with a
+// long K, which it splits too late).  Larger tiles move fewer bytes per output (per_k /
 // (bm bn) falls from 1.2 to 0.34 ps), smaller ones fill the chip sooner.
 constexpr TileModel kBf16Model = {
     {{32, 64, 64, 128, 5.0f, 0.0024f, 1.2f, 0.79f},
