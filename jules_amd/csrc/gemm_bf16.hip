@@ -610,6 +610,23 @@ hipError_t launch_gemm_bf16(int act, const uint16_t* A, const uint16_t* B, const
                                                      A, B, bias, C, M, N, K));
         return hipGetLastError();
     }
+    // Whole 256 x 256 tiles: 4 waves of 128 x 128 read less LDS per MFMA than 8 of
+    // 128 x 64 (4096^3 113 against 122 us), but hold every register, none left for
+    // the edges.
+    const bool whole = bf16_gemm_tile(M, N, K).variant == GV_BF16_DMA;
+    const auto launch_whole = [&] {
+        JH_DISPATCH_ACT(act, ACT, hipLaunchKernelGGL(gemm_bf16_dma_kernel<ACT>, dim3((M / BM) * (N / BN)),
+                                                     dim3(THREADS), 0, s, A, B, bias, C, M, N, K));
+        return hipGetLastError();
+    };
+    // Half the chip filled with them, they are the fastest whatever K: of 86 shapes
+    // of 128 such tiles and more, what the model picked was up to 2.4 times as slow
+    // and once 3 % faster (2304 x 3840 x 2560 59.7 us against 74.3 on 128 x 128
+    // tiles, 5888 x 11776 x 64 43 against 103 on 64 x 64).  From 64 tiles on a short K is still worth it: the
+    // next best takes 1.4 times as long at K below 128, 1.25 up to 512, 1.08 at 640,
+    // 0.8 at 2048.
+    const int64_t tiles = whole ? (int64_t)(M / BM) * (N / BN) : 0;
+    if (tiles >= 128 || (tiles >= 64 && K <= 768)) return launch_whole();
     WorkspaceLock lock;
     void* ws;
     const TileChoice c = tile_plan(kBf16Model, M, N, K, s, &ws, &lock);
@@ -621,15 +638,7 @@ hipError_t launch_gemm_bf16(int act, const uint16_t* A, const uint16_t* B, const
     case 3: launch_tile<TileCfg<Bf16Op, 128, 128, 2, 2, 2, 128, 4, 1>>(act, A, B, bias, C, part, M, N, K, c, s); break;
     case 4: launch_tile<TileCfg<Bf16Op, 128, 256, 2, 4, 1, 64, 6, 1>>(act, A, B, bias, C, part, M, N, K, c, s); break;
     default:
-        // Whole 256 x 256 tiles: 4 waves of 128 x 128 read less LDS per MFMA
-        // than 8 of 128 x 64 (4096^3 113 against 122 us; 2304 x 3840 x 2560
-        // 60 against 65), but hold every register, none left for the edges.
-        if (!part && bf16_gemm_tile(M, N, K).variant == GV_BF16_DMA) {
-            const int tiles = (M / BM) * (N / BN);
-            JH_DISPATCH_ACT(act, ACT, hipLaunchKernelGGL(gemm_bf16_dma_kernel<ACT>, dim3(tiles), dim3(THREADS),
-                                                         0, s, A, B, bias, C, M, N, K));
-            return hipGetLastError();
-        }
+        if (!part && whole) return launch_whole();
         launch_tile<TileCfg<Bf16Op, 256, 256, 2, 4, 1, 64, 4, 1>>(act, A, B, bias, C, part, M, N, K, c, s);
     }
     if (part) {

@@ -503,6 +503,18 @@ hipError_t launch_int8(const int8_t* A, const int8_t* B, float* C, int M, int N,
                            row_scale, col_scale, bias);
         return hipGetLastError();
     }
+    // Whole 256 x 256 tiles, 4 waves of 128 x 128, as in the bf16 GEMM and by the
+    // same rule (4096^3 66.9 against 73.6 us in the loop; 2048 x 11520 x 768 36
+    // against 56 on 128 x 256 tiles; at 64 tiles the next best takes 1.25 times as
+    // long for K <= 512, 1.0 to 1.26 for 1024, 0.8 to 1.0 for 2048).
+    const bool whole = M % QBM == 0 && N % QBN == 0 && K % QBK == 0;
+    const auto launch_whole = [&] {
+        hipLaunchKernelGGL(int8_dma_kernel, dim3((M / QBM) * (N / QBN)), dim3(256), 0, s, A, B, C, M, N, K,
+                           scale_a, scale_b, row_scale, col_scale, bias);
+        return hipGetLastError();
+    };
+    const int64_t tiles256 = whole ? (int64_t)(M / QBM) * (N / QBN) : 0;
+    if (tiles256 >= 128 || (tiles256 >= 64 && K <= 1024)) return launch_whole();
     WorkspaceLock lock;
     void* ws;
     const TileChoice c = tile_plan(kInt8Model, M, N, K, s, &ws, &lock);
@@ -520,13 +532,7 @@ hipError_t launch_int8(const int8_t* A, const int8_t* B, float* C, int M, int N,
     case 3: tile(TileCfg<Int8Op, 128, 128, 2, 2, 2, 128, 4, 1>{}); break;
     case 4: tile(TileCfg<Int8Op, 128, 256, 2, 4, 1, 64, 6, 1>{}); break;
     default:
-        // whole 256 x 256 tiles: 4 waves of 128 x 128, as in the bf16 GEMM
-        // (4096^3 66.9 against 73.6 us, 2048 x 8192 x 8192 120 against 125)
-        if (!part && M % QBM == 0 && N % QBN == 0 && K % QBK == 0) {
-            hipLaunchKernelGGL(int8_dma_kernel, dim3((M / QBM) * (N / QBN)), dim3(256), 0, s, A, B, C, M, N,
-                               K, scale_a, scale_b, row_scale, col_scale, bias);
-            return hipGetLastError();
-        }
+        if (!part && whole) return launch_whole();
         tile(TileCfg<Int8Op, 256, 256, 2, 4, 1, 64, 4, 1>{});
     }
     if (part) {

@@ -42,6 +42,9 @@ BF16_TILES = [
     (1000, 5000, 328, "128x256"), (512, 4224, 6984, "128x256 split"),
     (1288, 6152, 776, "256x256"), (1376, 3120, 4888, "256x256 split"),
     (3840, 2304, 32, "whole"), (3840, 2304, 96, "whole"), (3072, 3072, 160, "whole"),  # 1, 3 and 5 slices
+    # whole tiles for half the chip and more, or a quarter and a short K: smaller
+    # tiles took up to twice as long
+    (1024, 4096, 512, "whole"), (2560, 2560, 256, "whole"), (2048, 4096, 1024, "whole"), (2304, 3840, 2560, "whole"),
 ]
 
 
@@ -171,6 +174,7 @@ INT8_TILES = [
     (796, 5616, 6864, "128x256"),
     (1304, 6160, 784, "256x256"),
     (2816, 3072, 128, "whole"), (2304, 3840, 320, "whole"),
+    (768, 7168, 256, "whole"), (2048, 11520, 768, "whole"),
 ]
 # rows of any length: a kernel of their own
 INT8_ROWS = [(1, 1, 1, ""), (3, 65, 17, ""), (64, 64, 64 - 1, ""), (65, 130, 129, ""), (33, 1000, 255, "")]
