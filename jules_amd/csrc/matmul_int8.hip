@@ -515,16 +515,30 @@ hipError_t launch_int8(const int8_t* A, const int8_t* B, float* C, int M, int N,
     };
     const int64_t tiles256 = whole ? (int64_t)(M / QBM) * (N / QBN) : 0;
     if (tiles256 >= 128 || (tiles256 >= 64 && K <= 1024)) return launch_whole();
-    WorkspaceLock lock;
-    void* ws;
-    const TileChoice c = tile_plan(kInt8Model, M, N, K, s, &ws, &lock);
-    int* part = static_cast<int*>(ws);
+    TileChoice c{0, 1, K};
+    int* part = nullptr;
     auto tile = [&](auto cfg) {
         using T = decltype(cfg);
         const int64_t tiles = (((int64_t)M + T::BM - 1) / T::BM) * (((int64_t)N + T::BN - 1) / T::BN);
         hipLaunchKernelGGL(int8_tile_kernel<T>, dim3((unsigned)(tiles * c.splits)), dim3(T::THREADS), 0, s, A,
                            B, C, part, M, N, K, c.kc, scale_a, scale_b, row_scale, col_scale, bias);
     };
+    // Many tiles and a short K: storing the fp32 outputs takes as long as the
+    // products, so a ring of 3 stages, which leaves room for two workgroups on a
+    // CU, one of which stores while the other multiplies.  From 257 tiles on it is
+    // 1.2 to 1.7 times as fast as the deeper rings up to K = 1024 and 1.1 at 2048
+    // (2840 x 6400 x 384 50 -> 33 us, 133 x 72384 x 96 44 -> 19); with fewer tiles,
+    // one a CU, it is slower, and past 2048 as fast.
+    using Short = TileCfg<Int8Op, 128, 256, 2, 4, 1, 64, 3, 1>;
+    const int64_t tiles_s = (((int64_t)M + Short::BM - 1) / Short::BM) * (((int64_t)N + Short::BN - 1) / Short::BN);
+    if (tiles_s > 256 && K <= 2048 && tiles_s * Short::THREADS < int64_t(1) << 32) {
+        tile(Short{});
+        return hipGetLastError();
+    }
+    WorkspaceLock lock;
+    void* ws;
+    c = tile_plan(kInt8Model, M, N, K, s, &ws, &lock);
+    part = static_cast<int*>(ws);
     switch (c.plan) {
     case 0: tile(TileCfg<Int8Op, 32, 64, 1, 2, 1, 128, 6, 3>{}); break;
     case 1: tile(TileCfg<Int8Op, 64, 64, 2, 2, 1, 128, 4, 3>{}); break;

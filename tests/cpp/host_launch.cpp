@@ -298,19 +298,21 @@ static void mlp_wrappers() {
 // Names what each product read from stdin launches: "f32 M N K", "bf16 M N K",
 // "int8 M N K" or "sgemm ta tb M N K", one a line.  The fp32 tile as BM x BN x BK
 // and its variant, with "folded" where it adds ranges of K itself; "whole" for
-// the kernels of whole 256 x 256 tiles; "split" where a reduction follows.
+// the kernels of whole 256 x 256 tiles; "/3" for a ring of 3 stages; "split" where
+// a reduction follows.
 static void tiles() {
     std::string line, said;
     stub::on_launch = [&](const stub::Launch& l) {
         F32Launch f;
-        int bm, bn;
+        int bm, bn, stages;
         const size_t cfg = l.kernel.find("TileCfg<");
         char s[80];
         if (f32_launch(l.kernel, &f))
             std::snprintf(s, sizeof s, "%dx%dx%d v%d%s", 2 * f.mt * f.mf, 2 * f.nt * f.mf, f.bk, f.v,
                           f.fold ? " folded" : "");
-        else if (cfg != std::string::npos && std::sscanf(l.kernel.c_str() + cfg, "TileCfg<jh::%*[A-Za-z0-9], %d, %d", &bm, &bn) == 2)
-            std::snprintf(s, sizeof s, "%dx%d", bm, bn);
+        else if (cfg != std::string::npos && std::sscanf(l.kernel.c_str() + cfg, "TileCfg<jh::%*[A-Za-z0-9], %d, %d, %*d, %*d, %*d, %*d, %d", &bm, &bn,
+                                                         &stages) == 3)
+            std::snprintf(s, sizeof s, stages == 3 ? "%dx%d/3" : "%dx%d", bm, bn);
         else if (l.kernel.find("_dma_kernel") != std::string::npos)
             std::snprintf(s, sizeof s, "whole");
         else if (l.kernel.find("_reduce_kernel") != std::string::npos)

@@ -172,9 +172,12 @@ INT8_TILES = [
     (222, 5264, 7328, "64x128"), (39, 5952, 6768, "64x128 split"),
     (540, 4112, 1040, "128x128"), (1000, 2064, 912, "128x128"),
     (796, 5616, 6864, "128x256"),
-    (1304, 6160, 784, "256x256"),
+    (1304, 6160, 784, "128x256/3"), (1304, 6160, 2064, "256x256"),
     (2816, 3072, 128, "whole"), (2304, 3840, 320, "whole"),
     (768, 7168, 256, "whole"), (2048, 11520, 768, "whole"),
+    # many tiles and a short K, 1 to 32 slices
+    (33, 65552, 64, "128x256/3"), (2177, 4368, 80, "128x256/3"), (276, 24016, 144, "128x256/3"),
+    (2281, 5376, 256, "128x256/3"), (2840, 6400, 2032, "128x256/3"),
 ]
 # rows of any length: a kernel of their own
 INT8_ROWS = [(1, 1, 1, ""), (3, 65, 17, ""), (64, 64, 64 - 1, ""), (65, 130, 129, ""), (33, 1000, 255, "")]
