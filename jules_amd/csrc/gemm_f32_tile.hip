@@ -10,15 +10,18 @@ namespace {
 // C = epilogue(sum over z of part[z], in z order)
 __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(F32Gemm g, int S, const float* __restrict__ part) {
     const int64_t total = (int64_t)g.M * g.N, stride = (int64_t)gridDim.x * 256;
-    finish<true>(g, [&](auto&& f) {
+    const auto sums = [&](auto&& f) {
         for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += stride) {
             float v = part[e];
 #pragma unroll 4
             for (int z = 1; z < S; ++z) v += part[(int64_t)z * total + e];
-            const int m = (int)(e / g.N), n = (int)(e - (int64_t)m * g.N);
-            f(m, n, v, g.bias ? g.bias[n] : 0.0f);
+            const int m = (int)(e / g.N);
+            f(m, (int)(e - (int64_t)m * g.N), v);
         }
-    });
+    };
+    finish<true>(
+        g, [&](auto&& f) { sums([&](int m, int n, float v) { f(m, n, v, g.bias ? g.bias[n] : 0.0f); }); },
+        [&](auto&& load, auto&& f) { sums([&](int m, int n, float v) { f(m, n, v, load(m, n)); }); });
 }
 
 // The tiles, and what they cost: n = ceil(workgroups / 256) tiles on a CU take
