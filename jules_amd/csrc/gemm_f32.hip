@@ -41,7 +41,7 @@ __global__ void fused_gelu_kernel(float* out, const float* __restrict__ in, int6
 hipError_t launch_gemm_f32(int act, const float* A, const float* B, const float* bias, float* C,
                            int M, int N, int K, hipStream_t s) {
     const F32Gemm g = {false, false, A, K, B, N, C, N, M, N, K, F32_EPI_ACT, act, bias, nullptr, 0, 1.0f, 0.0f, nullptr};
-    return launch_f32_gemm(g, 1, 0, nullptr, s);
+    return launch_f32_gemm(g, 1, 0, nullptr, s, 0.0f);
 }
 
 hipError_t launch_activation(int act, float* out, const float* in, int64_t n, hipStream_t s) {

@@ -106,23 +106,32 @@ F32Gemm f32_half(F32Gemm g, bool second) {
 
 }  // namespace
 
-hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s) {
+// What 32 x 32 tiles that fold a long K's ranges take: its chain, one piece of k
+// after the other, fitted to 1500 products with K 256-8192 in each orientation
+// (within 0.5 to 1.5 us).  An operand whose k is outermost in memory and whose
+// rows are no whole 16-byte pieces is loaded float by float.
+static float f32_fold_us(const F32Gemm& g, bool vec) {
+    const int64_t wg = (((int64_t)g.M + 31) / 32) * (((int64_t)g.N + 31) / 32);
+    const float n = (float)((wg + 255) / 256);
+    const float per_k = !g.ta && g.tb ? 0.0110f : vec || g.tb ? 0.0088f : g.ta ? 0.0133f : 0.0100f;
+    return 4.0f + g.K * per_k * (n > 1.0f ? 0.7f * n : 1.0f);
+}
+
+hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s, float launch_us) {
     if (g.M == 0 || g.N == 0) return hipSuccess;
     int chunk = 0, plan;
-    float us, fold_us = 0.0f;
+    float us;
+    // whole 16-byte pieces of the operands whose k is the outer dimension
+    const bool vec = (!g.ta || (g.M - (g.colsum ? 1 : 0)) % 4 == 0) && (g.tb || g.N % 4 == 0);
     if (splits > 1) {
         // The same sums in the same order in one launch, 32 x 32 tiles that fold
         // a range at a time, unless spreading the ranges over workgroups pays
-        // for its reduction (64 x 256 x 784 in 10 ranges: 17.4 us in two
-        // launches before, 8.2 in two on these tiles; the training step of 64
-        // rows around it 36.9 us with two, 34.4 folded).
+        // for its reduction (825 x 74 x 2667, A transposed: 40 us folded, 23 in
+        // two launches) and for what the caller says one launch more costs it.
         plan = f32_plan(g.M, g.N, kc, splits, &us);
-        us += 4.5f + 0.1f * splits + 1.2e-6f * splits * g.M * g.N;
-        const int64_t wg = ((int64_t)g.M + 31) / 32 * (((int64_t)g.N + 31) / 32);
-        const float n = (float)((wg + 255) / 256);
-        fold_us = n > 1.0f ? n * (g.K * kF32Plans[0].per_k + kF32Plans[0].round)
-                           : g.K * kF32Plans[0].alone + kF32Plans[0].round;
-        if (!part || fold_us < us) {
+        us += 4.5f + 0.07f * splits + 2.4e-6f * splits * g.M * g.N + launch_us;
+        if (!part || f32_fold_us(g, vec) < us) {
+            const int64_t wg = ((int64_t)g.M + 31) / 32 * (((int64_t)g.N + 31) / 32);
             chunk = kc;
             splits = 1;
             plan = wg <= 256 && g.K >= 256 ? 4 : 0;
@@ -135,14 +144,12 @@ hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hi
     }
     // a tile whose offsets pass 32 bits gives way to 32 x 32, then to 64-bit ones
     if (!f32_fits(g, plan)) plan = 0;
-    // whole 16-byte pieces of the operands whose k is the outer dimension
-    const int v = !f32_fits(g, plan) ? 0
-                  : (!g.ta || (g.M - (g.colsum ? 1 : 0)) % 4 == 0) && (g.tb || g.N % 4 == 0) ? 4 : 1;
+    const int v = !f32_fits(g, plan) ? 0 : vec ? 4 : 1;
     // the runtime takes fewer than 2^32 threads a launch
     const F32Dims& t = kF32Dims[g.tb && plan == 3 ? 2 : plan];  // as launch_f32_tile
     if (splits <= 1 && (((int64_t)g.M + t.bm - 1) / t.bm) * (((int64_t)g.N + t.bn - 1) / t.bn) >= int64_t(1) << 24) {
-        const hipError_t e = launch_f32_gemm(f32_half(g, false), 1, 0, nullptr, s);
-        return e != hipSuccess ? e : launch_f32_gemm(f32_half(g, true), 1, 0, nullptr, s);
+        const hipError_t e = launch_f32_gemm(f32_half(g, false), 1, 0, nullptr, s, 0.0f);
+        return e != hipSuccess ? e : launch_f32_gemm(f32_half(g, true), 1, 0, nullptr, s, 0.0f);
     }
     if (g.ta || g.tb) launch_f32_tile_trans(plan, v, g, splits, kc, chunk, part, s);
     else launch_f32_tile<false, false>(plan, v, g, splits, kc, chunk, part, s);

@@ -41,7 +41,8 @@ struct F32Gemm {
     // op(B), added in row order
     float* colsum;
 };
-hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s);
+// launch_us: what one launch more costs the caller
+hipError_t launch_f32_gemm(const F32Gemm& g, int splits, int kc, float* part, hipStream_t s, float launch_us);
 // C = alpha op(A) op(B) + beta C, fp32 on MFMA (mlp.hip); op(X) = X^T when
 // the trans flag is set; row-major with leading dimensions lda, ldb, ldc
 hipError_t launch_sgemm(bool transA, bool transB, int M, int N, int K, float alpha, const float* A,

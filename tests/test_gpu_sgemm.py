@@ -59,18 +59,22 @@ def test_wide_leading_dimensions(dev, ta, tb, M, N, K, lda, ldb):
 SGEMM_TILES = [
     (0, 0, 41, 45, 19, "32x32x64 v1"), (0, 0, 1001, 1021, 35, "64x64x32 v1"), (0, 0, 1024, 2048, 20, "64x128x16 v4"),
     (0, 0, 2040, 4092, 72, "128x128x16 v4"), (0, 0, 2041, 4089, 69, "128x128x16 v1"),
-    (0, 0, 70, 50, 700, "32x32x128 v1 folded"), (0, 0, 130, 260, 2050, "64x128x16 v4 split"),
+    (0, 0, 70, 50, 700, "32x32x64 v1 split"),
+    (0, 0, 190, 230, 270, "32x32x128 v1 folded"), (0, 0, 130, 260, 2050, "64x128x16 v4 split"),
     (1, 0, 33, 48, 65, "32x32x64 v1"), (1, 0, 1024, 1008, 36, "64x64x32 v4"), (1, 0, 1001, 1021, 35, "64x64x32 v1"),
     (1, 0, 1024, 2048, 20, "64x128x16 v4"), (1, 0, 1001, 2041, 21, "64x128x16 v1"),
     (1, 0, 2040, 4092, 72, "128x128x16 v4"), (1, 0, 2041, 4089, 69, "128x128x16 v1"),
-    (1, 0, 70, 50, 700, "32x32x128 v1 folded"), (1, 0, 300, 300, 300, "32x32x128 v4 folded"),
+    (1, 0, 70, 50, 700, "32x32x64 v1 split"),
+    (1, 0, 190, 230, 270, "32x32x128 v1 folded"), (1, 0, 300, 300, 300, "32x32x128 v4 folded"),
     (1, 0, 130, 260, 2050, "64x128x16 v1 split"),
     (0, 1, 33, 48, 65, "32x32x64 v4"), (0, 1, 1001, 1021, 35, "64x64x32 v4"), (0, 1, 1001, 2041, 21, "64x128x16 v4"),
-    (0, 1, 2041, 4089, 69, "64x128x16 v4"), (0, 1, 70, 50, 700, "32x32x128 v4 folded"),
+    (0, 1, 2041, 4089, 69, "64x128x16 v4"), (0, 1, 70, 50, 700, "32x32x64 v4 split"),
+    (0, 1, 190, 230, 270, "32x32x128 v4 folded"),
     (0, 1, 130, 260, 2050, "64x128x16 v4 split"),
     (1, 1, 33, 48, 65, "32x32x64 v1"), (1, 1, 1024, 1008, 36, "64x64x32 v4"), (1, 1, 1001, 1021, 35, "64x64x32 v1"),
     (1, 1, 1024, 2048, 20, "64x128x16 v4"), (1, 1, 1001, 2041, 21, "64x128x16 v1"),
-    (1, 1, 70, 50, 700, "32x32x128 v1 folded"), (1, 1, 300, 300, 300, "32x32x128 v4 folded"),
+    (1, 1, 70, 50, 700, "32x32x64 v1 split"),
+    (1, 1, 190, 230, 270, "32x32x128 v1 folded"), (1, 1, 300, 300, 300, "32x32x128 v4 folded"),
     (1, 1, 130, 260, 2050, "64x128x16 v1 split"), (1, 1, 64, 64, 4096, "32x32x64 v4 split"),
 ]
 
