@@ -82,24 +82,51 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Gemm g, int kc
         each([&](int m, int n, float v, float) { p[(int64_t)m * g.N + n] = v; });
     } else {
         finish<ACTS>(g, each, [&](auto&& load, auto&& f) {
-            float x[CF::NT][CF::MT][T::Mf::NR];
-            // rows and columns past the end as the last: what they load is not used
-            const auto row = [&](int i, int e) { return mw + i * CF::MF + T::Mf::row(lane, e); };
+            // All 64 outputs of a 128 x 128 tile at once take 232 registers, which
+            // leaves two workgroups on a CU, not three (5936 x 1716 x 96, beta 0 too,
+            // 34 -> 45 us): there an accumulator at a time, or with A transposed,
+            // where that still costs the tile 10 %, one by one.
+            if constexpr (CF::MT * CF::NT * T::Mf::NR > 32 && TA) {
+                each([&](int m, int n, float v, float) { f(m, n, v, load(m, n)); });
+            } else if constexpr (CF::MT * CF::NT * T::Mf::NR > 32) {
 #pragma unroll
-            for (int j = 0; j < CF::NT; ++j)
+                for (int j = 0; j < CF::NT; ++j) {
+                    const int n = nw + j * CF::MF;
+                    if (n >= g.N) continue;
 #pragma unroll
-                for (int i = 0; i < CF::MT; ++i)
+                    for (int i = 0; i < CF::MT; ++i) {
+                        const int mi = mw + i * CF::MF;
+                        float x[T::Mf::NR];
 #pragma unroll
-                    for (int e = 0; e < T::Mf::NR; ++e)
-                        x[j][i][e] = load(min(row(i, e), g.M - 1), min(nw + j * CF::MF, g.N - 1));
+                        for (int e = 0; e < T::Mf::NR; ++e)
+                            x[e] = load(min(mi + T::Mf::row(lane, e), g.M - 1), n);  // past the end: not used
 #pragma unroll
-            for (int j = 0; j < CF::NT; ++j)
+                        for (int e = 0; e < T::Mf::NR; ++e) {
+                            const int m = mi + T::Mf::row(lane, e);
+                            if (m < g.M) f(m, n, acc[i][j][e], x[e]);
+                        }
+                    }
+                }
+            } else {
+                float x[CF::NT][CF::MT][T::Mf::NR];
+                // rows and columns past the end as the last: what they load is not used
+                const auto row = [&](int i, int e) { return mw + i * CF::MF + T::Mf::row(lane, e); };
 #pragma unroll
-                for (int i = 0; i < CF::MT; ++i)
+                for (int j = 0; j < CF::NT; ++j)
 #pragma unroll
-                    for (int e = 0; e < T::Mf::NR; ++e)
-                        if (row(i, e) < g.M && nw + j * CF::MF < g.N)
-                            f(row(i, e), nw + j * CF::MF, acc[i][j][e], x[j][i][e]);
+                    for (int i = 0; i < CF::MT; ++i)
+#pragma unroll
+                        for (int e = 0; e < T::Mf::NR; ++e)
+                            x[j][i][e] = load(min(row(i, e), g.M - 1), min(nw + j * CF::MF, g.N - 1));
+#pragma unroll
+                for (int j = 0; j < CF::NT; ++j)
+#pragma unroll
+                    for (int i = 0; i < CF::MT; ++i)
+#pragma unroll
+                        for (int e = 0; e < T::Mf::NR; ++e)
+                            if (row(i, e) < g.M && nw + j * CF::MF < g.N)
+                                f(row(i, e), nw + j * CF::MF, acc[i][j][e], x[j][i][e]);
+            }
         });
     }
 }
